@@ -17,33 +17,6 @@
 
 #define MT 256
 
-/* per-axis candidate source coarse cells of a mesh cell, in visit order
-   restricted to one axis: cells with different k are ordered by
-   (ilayer(k), k) with ilayer = (k - k0) mod 3 */
-struct Src {
-  int n;
-  int c[3];
-};
-__device__ static inline void order_z(Src &s, int k0) {
-  /* sort s.c[0..n) by ((c-k0) mod 3, c), n <= 3 */
-  for (int a = 1; a < s.n; ++a) {
-    const int x = s.c[a];
-    const int kx = ((x - k0) % 3 + 3) % 3;
-    int b = a - 1;
-    while (b >= 0) {
-      const int y = s.c[b];
-      const int ky = ((y - k0) % 3 + 3) % 3;
-      if (ky > kx || (ky == kx && y > x)) {
-        s.c[b + 1] = y;
-        --b;
-      } else {
-        break;
-      }
-    }
-    s.c[b + 1] = x;
-  }
-}
-
 /* the coarse CIC coordinate ((cell-1)+(x offset))-0.5 of W/pm.f90:213,335
    rounded to real(4); c = cell-1 (tile frame or global).  With 1-byte codes
    c + (u+0.5)/256 has at most 24 significant bits for c < 2^15, so the
@@ -55,63 +28,6 @@ template <int IX> __device__ __forceinline__ float coarse_tempx(int c, int32_t c
   else
     return (float)(((double)c + cube_xoff(IX, code)) - 0.5);
 }
-/* ---------------- coarse CIC deposit, W/pm.f90:205-267 ---------------- */
-template <int IX>
-__global__ __launch_bounds__(MT) void k_coarse_deposit(const typename IntOf<IX>::T *__restrict__ xp,
-                                                       const int32_t *__restrict__ rhoc,
-                                                       const int64_t *__restrict__ cstart, Geo g, float mass,
-                                                       float *__restrict__ r3, double *__restrict__ part) {
-  const int nc = g.nc;
-  const int64_t nc3 = (int64_t)nc * nc * nc;
-  double tsum = 0;
-  for (int64_t m = blockIdx.x * (int64_t)MT + threadIdx.x; m < nc3; m += (int64_t)gridDim.x * MT) {
-    const int gg[3] = {(int)(m % nc), (int)((m / nc) % nc), (int)(m / ((int64_t)nc * nc))};
-    int T[3], lm[3];
-    Src s[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      T[a] = gg[a] / g.nt;
-      lm[a] = gg[a] - T[a] * g.nt + 1;
-      s[a].n = 3; s[a].c[0] = lm[a] - 1; s[a].c[1] = lm[a]; s[a].c[2] = lm[a] + 1;
-    }
-    order_z(s[2], 0);
-    float acc = 0.f;
-    for (int qz = 0; qz < 3; ++qz)
-      for (int qy = 0; qy < 3; ++qy)
-        for (int qx = 0; qx < 3; ++qx) {
-          const int ci[3] = {s[0].c[qx], s[1].c[qy], s[2].c[qz]};
-          const int64_t cc = cid_global(g, T[0] * g.nt + ci[0] - 1, T[1] * g.nt + ci[1] - 1, T[2] * g.nt + ci[2] - 1);
-          const int np = rhoc[cc];
-          const int64_t p0 = cstart[cc];
-          for (int l = 0; l < np; ++l) {
-            float w[3];
-            bool hit = true;
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-              const int32_t code = (int32_t)xp[3 * (p0 + l) + a];
-              const float tempx = coarse_tempx<IX>(ci[a] - 1, code);
-              const int i1 = (int)floorf(tempx) + 1;
-              const float d1 = (float)i1 - tempx;
-              if (i1 == lm[a]) w[a] = d1;
-              else if (i1 + 1 == lm[a]) w[a] = 1.0f - d1;
-              else hit = false;
-            }
-            if (hit) acc = acc + w[0] * w[1] * w[2] * mass;
-          }
-        }
-    r3[m] = acc;
-    tsum += (double)acc;
-  }
-  __shared__ double red[MT];
-  red[threadIdx.x] = tsum;
-  __syncthreads();
-  for (int o = MT / 2; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
-}
-
 /* sum of nb partials in a fixed order (thread t takes b = t mod 64, then a
    tree over the threads), so the sum repeats bit for bit */
 __global__ __launch_bounds__(64) void k_sum_parts1(const double *part, int nb, double *out) {
@@ -415,211 +331,408 @@ __global__ __launch_bounds__(FD_T) void k_fine_deposit_cc(const typename IntOf<I
 }
 
 /*
- * Coarse deposit, one thread per 2x2x2 block of mesh cells (m0..m0+1 per
- * axis, within one tile since nt is even): the sources are the 4 cells
- * m0-1..m0+2 per axis, walked in the reference order (ilayer=k mod 3, k,
- * j, i, l), with the 8 sums in registers.  A particle that misses a cell
- * adds +0.0, which leaves a sum of non-negative terms unchanged.
+ * Coarse deposit, W/pm.f90:205-267: one wave per block of 4x4x4 mesh cells of
+ * a tile (clipped at the tile's high edge), one lane per mesh cell.  A mesh
+ * cell sums the hits of its 3^3 source cells in the reference's order
+ * (ilayer = k mod 3, j, i, l); the block's sources are the 6^3 cells around
+ * it.  Source planes 3 apart have the same ilayer and no mesh cell needs
+ * both, so the wave works in three phases of two planes each: every lane has
+ * exactly one of the two planes to read in each phase, and the phases in
+ * order of ilayer give every lane the reference's order.
  *
- * The 16 source rows (k, j) are gathered in that order.  A lane whose
- * block's sources pass `heavy_at` particles (a clustered region) stops at
- * a row boundary, and its whole wave finishes the block: 64 lanes form 64
- * particles' 8 terms at once (the same expression), and 8 lanes add them
- * to the partial sums in particle order -- the same additions in the same
- * order, so the same bits, without one lane walking thousands of particles
- * while the other 63 wait.  The owner adds the 8 sums to its total in the
- * same place of its sequence as a light block's.
+ * A phase stages its 12 rows of 6 cells in LDS, a row padded to batches of
+ * 64 particles, as the own-cell weights in fixed point (one word per
+ * particle) and three 64-bit ballots per batch: which particles sit in the
+ * upper half of their cell on each axis.  A particle in the upper half
+ * reaches its own and the next mesh cell, else its own and the one before, so
+ * a lane gets the hits of three cells of a row from a few logic operations
+ * and walks only those, in slot order = reference order.  A particle that
+ * misses a mesh cell would add +0.0, which leaves a sum of non-negative
+ * terms unchanged, so nothing is lost by not visiting it.
+ *
+ * A phase with more than `heavy_at` particles (a clustered region) or more
+ * batches than are staged at once goes through its particles 32 at a time
+ * instead: the wave forms the 27 terms of each (zero where it misses) in LDS
+ * and each lane adds its column, two instructions per particle, so a halo of
+ * thousands of particles costs its additions and not a walk each.
+ *
+ * What bounds it: VALU work (the hit loop above all) at 16 waves per CU (9.4
+ * KB of LDS per wave, 4 waves per SIMD by registers), on small meshes the one
+ * chain of dependent loads of a wave, and with halos the additions of the
+ * fullest block.  Alone on one MI355X, against one lane per 2^3 mesh cells
+ * with the sources read where they lie: 32^3 particles 0.046 ms (was 0.24),
+ * 128^3 0.08 (0.30), 256^3 with 2-byte codes at z = 3 0.92 (1.90), 512^3 2.2
+ * (3.35), 128^3 at z = 0.5 with cells of up to 2300 particles 0.48 (4.6).
  */
-template <int IX>
-__device__ __forceinline__ void cd_weights(const int ci[3], const int m0[3], const int32_t code[3], float w0[3],
-                                           float w1[3]) {
+template <int IX> struct CdWord;
+template <> struct CdWord<1> { /* bytes q: own weight (2q+257)/512, the neighbour's (255-2q)/512 */
+  typedef uint32_t T;
+  static constexpr float H = 256.f, scale = 0x1p-27f; /* half a cell; 1/(2H)^3 */
+  static constexpr int field = 8, NB = 16; /* NB: batches of 64 slots staged at once */
+};
+template <> struct CdWord<2> { /* 21-bit fields q: own weight (65536+q)/2^17, the neighbour's (65536-q)/2^17 */
+  typedef uint64_t T;
+  static constexpr float H = 65536.f, scale = 0x1p-51f;
+  static constexpr int field = 21, NB = 14; /* 12 rows, a few of them over 64 particles */
+};
+/* the staged fields of a particle's codes (in the low bytes of `raw`) and a
+   word with the top bit of axis a's field position set where corner 1 of the
+   cloud is the particle's own cell (the upper half).  The own weight is d1
+   there and 1-d1 in the lower half, both exact.  EX: tempx is exact in
+   real(4) in every cell of the tile, so the weights are those of the code
+   alone; else they come from tempx as the reference rounds it in cell c
+   (0-based, tile frame) */
+template <int IX, bool EX>
+__device__ __forceinline__ typename CdWord<IX>::T cd_fields(typename CdWord<IX>::T raw, const int c[3], bool up[3]) {
+  if constexpr (IX == 1) {
+    /* upper: 255-u, lower: u, all three bytes at once */
+    const uint32_t h = (raw >> 7) & 0x010101u;
 #pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    const float tempx = coarse_tempx<IX>(ci[a] - 1, code[a]);
-    const int i1 = (int)floorf(tempx) + 1;
-    const float d1 = (float)i1 - tempx, d2 = 1.0f - d1;
-    const int r = i1 - m0[a]; /* corner 1 relative to the block */
-    w0[a] = r == 0 ? d1 : (r == -1 ? d2 : 0.f);
-    w1[a] = r == 1 ? d1 : (r == 0 ? d2 : 0.f);
+    for (int a = 0; a < 3; ++a) up[a] = (raw & (0x80u << (8 * a))) != 0u;
+    return (raw & 0xffffffu) ^ (h * 255u);
+  } else {
+    uint64_t w = 0;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const uint32_t u = (uint32_t)(raw >> (16 * a)) & 0xffffu;
+      uint32_t q;
+      if constexpr (EX) {
+        up[a] = u >= 32768u;
+        q = (2u * u + 1u) ^ (up[a] ? 0x1ffffu : 0u); /* 131071 - 2u - ... : 131072-(2u+1), 17 bits */
+        q += up[a] ? 1u : 0u;
+      } else {
+        const float tempx = coarse_tempx<2>(c[a], (int32_t)u);
+        const int i1 = (int)floorf(tempx) + 1;
+        const float d1 = (float)i1 - tempx;
+        up[a] = i1 == c[a] + 1;
+        q = (uint32_t)((up[a] ? d1 : 1.0f - d1) * 131072.f) - 65536u;
+      }
+      w |= (uint64_t)q << (21 * a);
+    }
+    return w;
   }
 }
-
+/* weight of axis a in units of 1/(2H) times k: s = 1 the own cell's, -1 the
+   neighbour's; (k, s) come folded as (ks, kh), see CdWord */
+template <int IX> __device__ __forceinline__ float cd_q(typename CdWord<IX>::T w, int a) {
+  if constexpr (IX == 1) return (float)((w >> (8 * a)) & 0xff);
+  else return (float)(uint32_t)((w >> (21 * a)) & 0x1fffff);
+}
+/* H + s*t as q*cd_mul(s) + cd_add(s): t = 2q+1 (1-byte codes) or q */
+template <int IX> __device__ __forceinline__ float cd_mul(float s) { return IX == 1 ? 2.f * s : s; }
+template <int IX> __device__ __forceinline__ float cd_add(float s) { return IX == 1 ? CdWord<IX>::H + s : CdWord<IX>::H; }
+/* the codes of particle p as stored: one 4- or 8-byte read of its 3 or 6
+   bytes (the particle arrays end in padding) */
 template <int IX>
-__global__ __launch_bounds__(MT) void k_coarse_deposit_b2(const typename IntOf<IX>::T *__restrict__ xp,
-                                                          const int32_t *__restrict__ rhoc,
-                                                          const int64_t *__restrict__ cstart, Geo g, float mass,
-                                                          float *__restrict__ r3, double *__restrict__ part,
-                                                          int heavy_at) {
-  const int nc = g.nc, nb = nc / 2;
-  const int64_t nb3 = (int64_t)nb * nb * nb;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  __shared__ float cw[MT / 64][64 * 9]; /* a wave's 64 particles x 8 terms, rows of 9: no bank conflicts */
-  __shared__ float sfin[MT / 64][8];
+__device__ __forceinline__ typename CdWord<IX>::T cd_load(const char *__restrict__ q) {
+  typename CdWord<IX>::T v;
+  __builtin_memcpy(&v, q, sizeof(v));
+  return v;
+}
+
+template <int IX> struct CdLds { /* per wave */
+  union {
+    typename CdWord<IX>::T word[CdWord<IX>::NB * 64];
+    float term[27 * 65 + 8]; /* 27 columns of 64 terms, in 27 different banks; read up to 7 past a column's end */
+  };
+  uint64_t up[CdWord<IX>::NB][3];
+  int64_t start[36][3]; /* a row's first particle, and that of its cells iL and iE */
+  int pre[36][7]; /* first particle of each cell of a row, counted from the row's first */
+  int rb[12];     /* first batch of each row of the phase */
+  int cax[3][6];  /* a source cell's id is the sum of its three axes' parts */
+};
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+/* bits [0, p), p clipped to [0, 64] */
+__device__ __forceinline__ uint64_t bits_below(int p) {
+  p = max(p, 0);
+  return p >= 64 ? ~0ull : (1ull << p) - 1ull;
+}
+__device__ __forceinline__ int64_t rl_i64(int64_t v, int l) {
+  return (int64_t)(((uint64_t)(uint32_t)rl_i((int)(v >> 32), l) << 32) | (uint64_t)(uint32_t)rl_i((int)(v & 0xffffffff), l));
+}
+
+template <int IX, bool EX, int NW>
+__global__ __launch_bounds__(64 * NW, 4) void k_coarse_deposit(const typename IntOf<IX>::T *__restrict__ xp,
+                                                            const int32_t *__restrict__ rhoc,
+                                                            const int64_t *__restrict__ cstart, Geo g, float mass,
+                                                            float *__restrict__ r3, double *__restrict__ part,
+                                                            int nblk, int heavy_at) {
+  typedef typename CdWord<IX>::T W;
+  constexpr float H = CdWord<IX>::H, SC = CdWord<IX>::scale;
+  constexpr int PB = 3 * IX; /* bytes per particle */
+  __shared__ CdLds<IX> lds[NW];
+  __shared__ double wsum[NW];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  CdLds<IX> &S = lds[wv];
+  const char *xb8 = reinterpret_cast<const char *>(xp);
+  const int nt = g.nt, nbt = (nt + 3) / 4;
+  const int xi = lane & 3, yi = (lane >> 2) & 3, zi = lane >> 4;
   double tsum = 0;
-  /* the loop is uniform over a wave: lane l takes block b0 + l */
-  for (int64_t b0 = blockIdx.x * (int64_t)MT + wv * 64; b0 < nb3; b0 += (int64_t)gridDim.x * MT) {
-    const int64_t b = b0 + lane;
-    const bool live = b < nb3;
-    int gg[3] = {0, 0, 0}, T[3] = {0, 0, 0}, m0[3] = {1, 1, 1}, zs[4] = {0, 0, 0, 0};
-    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    int rrow = 16; /* first source row the lane has not gathered */
-    if (live) {
-      gg[0] = 2 * (int)(b % nb);
-      gg[1] = 2 * (int)((b / nb) % nb);
-      gg[2] = 2 * (int)(b / ((int64_t)nb * nb));
+  for (int b = blockIdx.x * NW + wv; b < nblk; b += gridDim.x * NW) {
+    /* the block: tile T, first mesh cell m0 (0-based, tile frame) */
+    const uint32_t ub = (uint32_t)b, un = (uint32_t)nbt, q1 = ub / un, q2 = q1 / un, t = q2 / un;
+    const uint32_t tn = (uint32_t)g.nnt, t1 = t / tn;
+    const int T[3] = {(int)(t - t1 * tn), (int)(t1 % tn), (int)(t1 / tn)};
+    const int m0[3] = {4 * (int)(ub - q1 * un), 4 * (int)(q1 - q2 * un), 4 * (int)(q2 - t * un)};
+    /* a row's particles are contiguous but for the cells of the neighbour
+       tiles: cell 0 at the tile's low edge, cell iE on at its high edge */
+    const int iL = m0[0] == 0 ? 1 : 0, iE = nt - (m0[0] - 1);
+    const bool oneseg = iL == 0 && iE >= 6; /* uniform */
+    /* starts of the 6^3 source cells m0-1..m0+4 (those past the tile's next
+       cell are not needed: empty), then prefix sums along each row of 6 */
+    if (lane < 18) {
+      const int a = lane / 6, sc = (a == 0 ? m0[0] : a == 1 ? m0[1] : m0[2]) - 1 + lane % 6;
+      int ta = a == 0 ? T[0] : a == 1 ? T[1] : T[2];
+      int l = sc;
+      if (sc < 0) { l = nt - 1; ta = ta > 0 ? ta - 1 : g.nnt - 1; }
+      if (sc == nt) { l = 0; ta = ta < g.nnt - 1 ? ta + 1 : 0; }
+      const int st = a == 0 ? 1 : a == 1 ? nt : nt * nt, ts = a == 0 ? 1 : a == 1 ? g.nnt : g.nnt * g.nnt;
+      S.cax[a][lane % 6] = sc > nt ? -1 : l * st + nt * nt * nt * ts * ta;
+    }
+    wave_lds_sync();
+    int cnt4[4];
 #pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        T[a] = gg[a] / g.nt;
-        m0[a] = gg[a] - T[a] * g.nt + 1;
-      }
-      zs[0] = m0[2] - 1;
-      zs[1] = m0[2];
-      zs[2] = m0[2] + 1;
-      zs[3] = m0[2] + 2;
-      /* order by (k mod 3, k): insertion sort of 4 */
-      for (int a = 1; a < 4; ++a) {
-        const int x = zs[a];
-        int bb = a - 1;
-        while (bb >= 0 && ((zs[bb] % 3) > (x % 3) || ((zs[bb] % 3) == (x % 3) && zs[bb] > x))) {
-          zs[bb + 1] = zs[bb];
-          --bb;
+    for (int u = 0; u < 4; ++u) {
+      const int q = lane + 64 * u;
+      cnt4[u] = 0;
+      if (q < 216) {
+        const int cx = S.cax[0][q % 6], cy = S.cax[1][(q / 6) % 6], cz = S.cax[2][q / 36];
+        if ((cx | cy | cz) >= 0) {
+          const int cc = cx + cy + cz;
+          cnt4[u] = rhoc[cc];
+          const int sx = q % 6;
+          const int64_t st = cstart[cc];
+          if (sx == 0) S.start[q / 6][0] = st;
+          if (sx == iL) S.start[q / 6][1] = st;
+          if (sx == iE) S.start[q / 6][2] = st;
         }
-        zs[bb + 1] = x;
       }
-      int cum = 0;
-      for (int row = 0; row < 16; ++row) {
-        const int qz = row >> 2, sy = m0[1] - 1 + (row & 3);
-        /* the row's 4 source cells: counts and starts loaded together */
-        int npr[4];
-        int64_t p0r[4];
+    }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int64_t cc = cid_global(g, T[0] * g.nt + m0[0] - 2 + u, T[1] * g.nt + sy - 1, T[2] * g.nt + zs[qz] - 1);
-          npr[u] = rhoc[cc];
-          p0r[u] = cstart[cc];
-        }
-        cum += (npr[0] + npr[1]) + (npr[2] + npr[3]);
-        if (cum > heavy_at) {
-          rrow = row;
-          break;
-        }
+    for (int u = 0; u < 4; ++u)
+      if (lane + 64 * u < 216) S.pre[(lane + 64 * u) / 6][(lane + 64 * u) % 6 + 1] = cnt4[u];
+    wave_lds_sync();
+    if (lane < 36) {
+      int acc = 0;
+      S.pre[lane][0] = 0;
+#pragma unroll
+      for (int q = 1; q < 7; ++q) {
+        acc += S.pre[lane][q];
+        S.pre[lane][q] = acc;
+      }
+    }
+    wave_lds_sync();
+    float acc = 0.f;
+    const int k0 = m0[2] % 3; /* 1-based local k of source plane s is m0z + s */
 #pragma unroll 1
-        for (int sx = m0[0] - 1; sx <= m0[0] + 2; ++sx) {
-          const int ci[3] = {sx, sy, zs[qz]};
-          const int ui = sx - (m0[0] - 1);
-          int np = npr[0];
-          int64_t p0 = p0r[0];
+    for (int il = 0; il < 3; ++il) {
+      const int s0 = (il - k0 + 3) % 3;      /* planes s0 and s0+3 */
+      const int sz = s0 >= zi ? s0 : s0 + 3; /* this lane's, offset sz-zi-1 from its cell */
+      /* lane t < 12 keeps row t of the phase (y = t/2, plane s0 + 3*(t&1)):
+         particles, and where they start in memory per segment */
+      const int rt = lane < 12 ? (s0 + 3 * (lane & 1)) * 6 + (lane >> 1) : 0;
+      const int nrow = lane < 12 ? S.pre[rt][6] : 0;
+      const int64_t dA = S.start[rt][0];
+      int64_t dB = 0, dC = 0;
+      int sB = 0, sC = 0;
+      if (!oneseg) {
+        sB = iL ? S.pre[rt][1] : 0;
+        sC = iE < 6 ? S.pre[rt][iE] : nrow;
+        dB = S.start[rt][1] - sB;
+        dC = iE < 6 ? S.start[rt][2] - sC : 0;
+      }
+      const int nbr = (nrow + 63) >> 6;
+      const int bsc = wave_incl_scan(nbr), psc = wave_incl_scan(nrow);
+      if (lane < 12) S.rb[lane] = bsc - nbr;
+      const int nbat = rl_i(bsc, 11), npart = rl_i(psc, 11);
+      /* row tr of the phase, wave-uniform (read from its lane before any
+         branch that turns lanes off), and its particle l's codes as stored */
+      struct Seg {
+        int64_t a, b, c;
+        int sb, sc, n;
+      };
+      auto seg = [&](int tr) -> Seg {
+        Seg e = {rl_i64(dA, tr), 0, 0, 0, 0, rl_i(nrow, tr)};
+        if (!oneseg) {
+          e.b = rl_i64(dB, tr);
+          e.c = rl_i64(dC, tr);
+          e.sb = rl_i(sB, tr);
+          e.sc = rl_i(sC, tr);
+        }
+        return e;
+      };
+      auto load = [&](const Seg &e, int l) -> W {
+        if (oneseg) return cd_load<IX>(xb8 + e.a * PB + (uint32_t)(l * PB));
+        const int64_t d = l < e.sb ? e.a : (l < e.sc ? e.b : e.c);
+        return cd_load<IX>(xb8 + (d + l) * PB);
+      };
+      /* its staged word and halves (the row's cell only where rounding asks for it) */
+      auto fields = [&](W raw, int tr, int l, bool up[3]) -> W {
+        int c[3] = {0, 0, 0};
+        if constexpr (!EX) {
+          const int r = (s0 + 3 * (tr & 1)) * 6 + (tr >> 1);
+          c[0] = m0[0] - 1;
 #pragma unroll
-          for (int u = 1; u < 4; ++u) { /* register select, no dynamic indexing */
-            np = ui == u ? npr[u] : np;
-            p0 = ui == u ? p0r[u] : p0;
-          }
-          /* four particles' codes in flight at once (the last one repeated) */
-          for (int l0 = 0; l0 < np; l0 += 4) {
-            int32_t code4[4][3];
+          for (int q = 1; q < 6; ++q) c[0] += S.pre[r][q] <= l ? 1 : 0;
+          c[1] = m0[1] - 1 + (tr >> 1);
+          c[2] = m0[2] - 1 + s0 + 3 * (tr & 1);
+        }
+        return cd_fields<IX, EX>(raw, c, up);
+      };
+      wave_lds_sync();
+      if (nbat <= CdWord<IX>::NB && npart <= heavy_at) {
+        auto stage = [&](W raw, int tr, int o) {
+          const int q = rl_i(bsc - nbr, tr) + (o >> 6);
+          bool up[3];
+          const W w = fields(raw, tr, o + lane, up);
+          const uint64_t u0 = __ballot(up[0]), u1 = __ballot(up[1]), u2 = __ballot(up[2]);
+          S.word[q * 64 + lane] = w;
+          if (lane < 3) S.up[q][lane] = lane == 0 ? u0 : (lane == 1 ? u1 : u2);
+        };
+        /* the first batch of every row is on its way before one is used */
+        W raw[12];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const int64_t q = p0 + min(l0 + u, np - 1);
+        for (int tr = 0; tr < 12; ++tr) {
+          raw[tr] = 0;
+          const Seg e = seg(tr);
+          if (lane < e.n) raw[tr] = load(e, lane);
+        }
 #pragma unroll
-              for (int a = 0; a < 3; ++a) code4[u][a] = (int32_t)xp[3 * q + a];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              if (l0 + u >= np) break;
-              float w0[3], w1[3];
-              cd_weights<IX>(ci, m0, code4[u], w0, w1);
-#pragma unroll
-              for (int q = 0; q < 8; ++q) {
-                const float wx = (q & 1) ? w1[0] : w0[0], wy = (q & 2) ? w1[1] : w0[1], wz = (q & 4) ? w1[2] : w0[2];
-                s[q] = s[q] + wx * wy * wz * mass;
-              }
+        for (int tr = 0; tr < 12; ++tr)
+          if (rl_i(nrow, tr) > 0) stage(raw[tr], tr, 0);
+        if (__ballot(nrow > 64)) {
+#pragma unroll 1
+          for (int tr = 0; tr < 12; ++tr) {
+            const Seg e = seg(tr);
+            for (int o = 64; o < e.n; o += 64) {
+              W w = 0;
+              if (o + lane < e.n) w = load(e, o + lane);
+              stage(w, tr, o);
             }
           }
         }
-      }
-    }
-    /* the wave finishes each heavy lane's block from its row rrow on */
-    uint64_t hm = __ballot(live && rrow < 16);
-    while (hm) {
-      const int L = __builtin_ctzll(hm);
-      hm &= hm - 1;
-      const int Lgg[3] = {rl_i(gg[0], L), rl_i(gg[1], L), rl_i(gg[2], L)};
-      const int LT[3] = {rl_i(T[0], L), rl_i(T[1], L), rl_i(T[2], L)};
-      const int Lm0[3] = {rl_i(m0[0], L), rl_i(m0[1], L), rl_i(m0[2], L)};
-      const int Lzs[4] = {rl_i(zs[0], L), rl_i(zs[1], L), rl_i(zs[2], L), rl_i(zs[3], L)};
-      const int Lrow = rl_i(rrow, L);
-      float acc = 0.f; /* lane q < 8: sum q, from the owner's partial sum */
+        wave_lds_sync();
+        const int oz = sz - zi - 1;
+        const float zs = oz == 0 ? 1.f : -1.f, mz = cd_mul<IX>(zs) * SC, az = cd_add<IX>(zs) * SC;
+#pragma unroll 1
+        for (int j = 0; j < 3; ++j) { /* rows y-1, y, y+1 */
+          const int sy = yi + j, r = sz * 6 + sy, tr = 2 * sy + (sz >= 3 ? 1 : 0);
+          const int pA = S.pre[r][xi], pB = S.pre[r][xi + 1], pC = S.pre[r][xi + 2], pD = S.pre[r][xi + 3];
+          const int rb = S.rb[tr];
+          const float ys = j == 1 ? 1.f : -1.f, my = cd_mul<IX>(ys), ay = cd_add<IX>(ys);
+          for (int bb = pA >> 6; bb * 64 < pD; ++bb) {
+            const int q = rb + bb, o = 64 * bb;
+            const uint64_t ux = S.up[q][0], uy = S.up[q][1], uz = S.up[q][2];
+            const uint64_t fA = bits_below(pA - o), fB = bits_below(pB - o), fC = bits_below(pC - o), fD = bits_below(pD - o);
+            uint64_t m = ((fB & ~fA) & ux) | (fC & ~fB) | ((fD & ~fC) & ~ux);
+            m &= j == 0 ? uy : (j == 1 ? ~0ull : ~uy);
+            m &= oz < 0 ? uz : (oz == 0 ? ~0ull : ~uz);
+            const uint32_t xb = (uint32_t)(pB - o), xn = (uint32_t)(pC - pB);
+            const W *wd = S.word + q * 64;
+            /* two hits per turn, so that two words are on their way at once;
+               without a second one its term is +0 */
+            while (m) {
+              const int i0 = __builtin_ctzll(m);
+              m &= m - 1ull;
+              const bool two = m != 0ull;
+              const int i1 = two ? __builtin_ctzll(m) : i0;
+              m &= m - 1ull; /* 0 stays 0 */
+              const W w0 = wd[i0], w1 = wd[i1];
+              const float s0x = (uint32_t)i0 - xb < xn ? 1.f : -1.f, s1x = (uint32_t)i1 - xb < xn ? 1.f : -1.f;
+              const float x0 = fmaf(cd_q<IX>(w0, 0), cd_mul<IX>(s0x), cd_add<IX>(s0x));
+              const float x1 = fmaf(cd_q<IX>(w1, 0), cd_mul<IX>(s1x), cd_add<IX>(s1x));
+              const float y0 = fmaf(cd_q<IX>(w0, 1), my, ay), y1 = fmaf(cd_q<IX>(w1, 1), my, ay);
+              const float z0 = fmaf(cd_q<IX>(w0, 2), mz, az), z1 = fmaf(cd_q<IX>(w1, 2), mz, az);
+              /* the reference's ((wx*wy)*wz)*mass: the units are powers of two */
+              const float e0 = x0 * y0 * z0 * mass, e1 = x1 * y1 * z1 * mass;
+              acc = acc + e0;
+              acc = acc + (two ? e1 : 0.f);
+            }
+          }
+        }
+      } else {
+#pragma unroll 1
+        for (int tr = 0; tr < 12; ++tr) {
+          const int sy = tr >> 1, sp = s0 + 3 * (tr & 1), r = sp * 6 + sy;
+          const Seg e = seg(tr);
+          const int n = e.n;
+          const bool mine = sp == sz && sy >= yi && sy <= yi + 2;
+          const int col = ((sp - zi) * 3 + (sy - yi)) * 3; /* +0, 1, 2 for the cells x-1, x, x+1 */
+          int pr[7];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const float v = rl_f(s[q], L);
-        acc = lane == q ? v : acc;
-      }
-      for (int row = Lrow; row < 16; ++row) {
-        const int qz = row >> 2, sy = Lm0[1] - 1 + (row & 3);
-        for (int u = 0; u < 4; ++u) {
-          const int sx = Lm0[0] - 1 + u;
-          const int64_t cc = cid_global(g, LT[0] * g.nt + sx - 1, LT[1] * g.nt + sy - 1, LT[2] * g.nt + Lzs[qz] - 1);
-          const int np = rhoc[cc];
-          const int64_t p0 = cstart[cc];
-          const int ci[3] = {sx, sy, Lzs[qz]};
-          for (int base = 0; base < np; base += 64) {
-            const int l = base + lane;
-            if (l < np) {
-              int32_t code[3];
+          for (int q = 0; q < 7; ++q) pr[q] = __builtin_amdgcn_readfirstlane(S.pre[r][q]);
+          W next = 0;
+          if (lane < n) next = load(e, lane);
+          for (int o = 0; o < n; o += 64) {
+            const int m = min(64, n - o);
+            const W raw = next; /* the next batch is on its way while this one is added */
+            if (o + 64 + lane < n) next = load(e, o + 64 + lane);
+            if (lane < m) {
+              bool up[3];
+              const W f = fields(raw, tr, o + lane, up);
+              float w[3][3]; /* weights for a mesh cell one above, at and one below the particle's */
 #pragma unroll
-              for (int a = 0; a < 3; ++a) code[a] = (int32_t)xp[3 * (p0 + l) + a];
-              float w0[3], w1[3];
-              cd_weights<IX>(ci, Lm0, code, w0, w1);
+              for (int a = 0; a < 3; ++a) {
+                const float q = cd_q<IX>(f, a), k = a == 2 ? SC : 1.f;
+                const float nb = fmaf(q, cd_mul<IX>(-1.f), cd_add<IX>(-1.f)) * k;
+                w[a][0] = up[a] ? nb : 0.f;
+                w[a][1] = fmaf(q, cd_mul<IX>(1.f), cd_add<IX>(1.f)) * k;
+                w[a][2] = up[a] ? 0.f : nb;
+              }
 #pragma unroll
-              for (int q = 0; q < 8; ++q) {
-                const float wx = (q & 1) ? w1[0] : w0[0], wy = (q & 2) ? w1[1] : w0[1], wz = (q & 4) ? w1[2] : w0[2];
-                cw[wv][lane * 9 + q] = wx * wy * wz * mass;
+              for (int y = 0; y < 3; ++y)
+#pragma unroll
+                for (int x = 0; x < 3; ++x) {
+                  const float wxy = w[0][x] * w[1][y];
+#pragma unroll
+                  for (int z = 0; z < 3; ++z) S.term[((z * 3 + y) * 3 + x) * 65 + lane] = wxy * w[2][z] * mass;
+                }
+            }
+            wave_lds_sync();
+            /* cell by cell of the row, so that the slots are the same for
+               every lane and a crowded cell is gone through once */
+#pragma unroll
+            for (int cx = 0; cx < 6; ++cx) {
+              const int lo = max(pr[cx] - o, 0), hi = min(pr[cx + 1] - o, m);
+              if (lo < hi && mine && (unsigned)(cx - xi) <= 2u) {
+                const float *c = S.term + (col + cx - xi) * 65;
+                for (int i = lo; i < hi; i += 8) {
+                  float v[8];
+#pragma unroll
+                  for (int k = 0; k < 8; ++k) v[k] = c[i + k];
+#pragma unroll
+                  for (int k = 0; k < 8; ++k) acc = acc + (i + k < hi ? v[k] : 0.f);
+                }
               }
             }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            if (lane < 8) {
-              const int m = min(64, np - base);
-              for (int i = 0; i < m; ++i) acc = acc + cw[wv][i * 9 + lane];
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            wave_lds_sync();
           }
         }
       }
-      if (lane < 8) {
-        const int x = Lgg[0] + (lane & 1), y = Lgg[1] + ((lane >> 1) & 1), z = Lgg[2] + ((lane >> 2) & 1);
-        r3[((int64_t)z * nc + y) * nc + x] = acc;
-        sfin[wv][lane] = acc;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      if (lane == L)
-        for (int q = 0; q < 8; ++q) tsum += (double)sfin[wv][q];
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      wave_lds_sync(); /* rb, word and up are read until here */
     }
-    if (live && rrow == 16) {
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int x = gg[0] + (q & 1), y = gg[1] + ((q >> 1) & 1), z = gg[2] + ((q >> 2) & 1);
-        r3[((int64_t)z * nc + y) * nc + x] = s[q];
-        tsum += (double)s[q];
-      }
+    if (m0[0] + xi < nt && m0[1] + yi < nt && m0[2] + zi < nt) {
+      const int64_t X = T[0] * nt + m0[0] + xi, Y = T[1] * nt + m0[1] + yi, Z = T[2] * nt + m0[2] + zi;
+      r3[(Z * g.nc + Y) * g.nc + X] = acc;
+      tsum += (double)acc;
     }
   }
-  __shared__ double red[MT];
-  red[threadIdx.x] = tsum;
-  __syncthreads();
-  for (int o = MT / 2; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) tsum += __shfl_xor(tsum, o, 64);
+  if constexpr (NW == 1) {
+    if (lane == 0) part[blockIdx.x] = tsum;
+  } else {
+    if (lane == 0) wsum[wv] = tsum;
     __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int w = 1; w < NW; ++w) tsum += wsum[w];
+      part[blockIdx.x] = tsum;
+    }
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
 
 #define DEP_BLOCKS 2048
@@ -644,24 +757,30 @@ template <int IX> static int fine_dep(cube_ctx *c, float mass, double *t) {
 int cube_fine_deposit(cube_ctx *c, float mass_p, double *testrhof) {
   return c->p.izipx == 1 ? fine_dep<1>(c, mass_p, testrhof) : fine_dep<2>(c, mass_p, testrhof);
 }
-template <int IX> static int coarse_dep(cube_ctx *c, float mass, double *t) {
+template <int IX, bool EX> static int coarse_dep(cube_ctx *c, float mass, double *t) {
   /* partial sums in the upper half of dred, apart from the fine deposit's,
      so that the two deposits may run at the same time */
   double *part = c->dred + 4096;
-  /* source particles a lane gathers alone before its wave takes the rest
-     of its block (CUBE_CD_HEAVY) */
-  int heavy_at = 1024;
+  /* particles of a phase's 72 source cells above which it adds 64 particles'
+     terms at a time (CUBE_CD_HEAVY); the staged batches hold no more */
+  int heavy_at = 64 * CdWord<IX>::NB;
   if (const char *e = getenv("CUBE_CD_HEAVY"); e && *e) heavy_at = std::max(0, atoi(e));
-  if (c->nt % 2 == 0)
-    hipLaunchKernelGGL(k_coarse_deposit_b2<IX>, dim3(DEP_BLOCKS), dim3(MT), 0, c->stream,
-                       (const typename IntOf<IX>::T *)c->xp, c->rhoc, c->cstart, geo_of(c), mass, c->rho_c, part,
-                       heavy_at);
+  const int64_t nbt = (c->nt + 3) / 4, nblk = nbt * nbt * nbt * c->ntiles;
+  /* small meshes: one wave per workgroup, so that few blocks spread over many
+     CUs (with more than DEP_BLOCKS every CU has its waves either way, and
+     there are no more partial sums than that); else four */
+  const bool small = nblk <= DEP_BLOCKS;
+  const int64_t want = small ? nblk : (nblk + 3) / 4;
+  const unsigned grid = (unsigned)std::min<int64_t>(want, DEP_BLOCKS);
+  const typename IntOf<IX>::T *xp = (const typename IntOf<IX>::T *)c->xp;
+  if (small)
+    hipLaunchKernelGGL((k_coarse_deposit<IX, EX, 1>), dim3(grid), dim3(64), 0, c->stream, xp, c->rhoc, c->cstart,
+                       geo_of(c), mass, c->rho_c, part, (int)nblk, heavy_at);
   else
-    hipLaunchKernelGGL(k_coarse_deposit<IX>, dim3(DEP_BLOCKS), dim3(MT), 0, c->stream,
-                       (const typename IntOf<IX>::T *)c->xp, c->rhoc, c->cstart, geo_of(c), mass, c->rho_c, part);
+    hipLaunchKernelGGL((k_coarse_deposit<IX, EX, 4>), dim3(grid), dim3(256), 0, c->stream, xp, c->rhoc, c->cstart,
+                       geo_of(c), mass, c->rho_c, part, (int)nblk, heavy_at);
   CUBE_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_sum_parts1, dim3(1), dim3(64), 0, c->stream, part, DEP_BLOCKS,
-                     c->dred + CUBE_DRED_COARSE_SUM);
+  hipLaunchKernelGGL(k_sum_parts1, dim3(1), dim3(64), 0, c->stream, part, (int)grid, c->dred + CUBE_DRED_COARSE_SUM);
   CUBE_LAUNCH_CHECK();
   if (t) {
     CUBE_CHECK(hipMemcpyAsync(t, c->dred + CUBE_DRED_COARSE_SUM, sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -670,7 +789,10 @@ template <int IX> static int coarse_dep(cube_ctx *c, float mass, double *t) {
   return CUBE_OK;
 }
 int cube_coarse_deposit(cube_ctx *c, float mass_p, double *testrhoc) {
-  return c->p.izipx == 1 ? coarse_dep<1>(c, mass_p, testrhoc) : coarse_dep<2>(c, mass_p, testrhoc);
+  if (c->p.izipx == 1) return coarse_dep<1, true>(c, mass_p, testrhoc);
+  /* 2-byte codes: c + (u+0.5)/65536 - 0.5 needs 17 fraction bits, exact in
+     real(4) below 128, and a source cell's c reaches nt */
+  return c->nt < 128 ? coarse_dep<2, true>(c, mass_p, testrhoc) : coarse_dep<2, false>(c, mass_p, testrhoc);
 }
 
 /* ---------------- kicks ---------------- */

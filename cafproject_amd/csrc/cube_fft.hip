@@ -587,15 +587,15 @@ __global__ __launch_bounds__(FFT_T) void k_r2c_x(const float *__restrict__ in, f
 
 /* in-place strided line FFTs: element (col, n) at base + n*stride + col,
    col in [0, ncol); grid.x = column blocks, grid.y = outer index with
-   outer stride `ostride` */
+   outer stride `ostride`, grid.z = component with stride `cstride` */
 template <int N, int DIR>
 __global__ __launch_bounds__(FFT_T) void k_c2c_s(float2 *__restrict__ a, const float2 *__restrict__ tw,
-                                               int ncol, int64_t stride, int64_t ostride) {
+                                               int ncol, int64_t stride, int64_t ostride, int64_t cstride) {
   constexpr int B = Cfg<N>::BS, TL = FFT_T / B, NP = lspan(N);
   __shared__ float2 sm[B * NP];
   const int tid = threadIdx.x, line = tid / TL, tl = tid % TL;
   const int col0 = blockIdx.x * B;
-  float2 *base = a + (int64_t)blockIdx.y * ostride + col0;
+  float2 *base = a + (int64_t)blockIdx.z * cstride + (int64_t)blockIdx.y * ostride + col0;
   /* every load in flight before the first LDS store */
   constexpr int IT = (B * N + FFT_T - 1) / FFT_T;
   float2 ld[IT];
@@ -681,6 +681,216 @@ __global__ __launch_bounds__(FFT_T) void k_green_z(const float2 *spec, float2 *o
       const int l = idx % B, n = idx / B;
       if (col0 + l < NH) dst[n * stride + l] = sm[l * NP + lpad(n)];
     }
+  }
+}
+
+/* ---------------- the differentiable model's z passes ----------------
+ * The Poisson operator i K_d with K_d = k_d/k^2 formed where it is used (three
+ * quotients per mode against 12 bytes of table read), and its transpose.
+ * KA: K_d times amp[kz][ky][kx] (the initial conditions' filter).
+ *
+ * k_pois_r / k_pois_z: forward FFT along z, times i K_d, inverse FFT for
+ * components blockIdx.z*nd .. +nd of the three, one 16-column block of one
+ * (x, y) line set per workgroup.
+ * k_pois_tr / k_pois_tz: the transpose: forward FFT along z of the three
+ * components, the sum of (-i K_d) times each, one inverse FFT. */
+__device__ __forceinline__ float2 mul_ik(float2 v, float K) { return make_float2((-v.y) * K, v.x * K); }
+
+template <int N, bool KA>
+__global__ __launch_bounds__(RC<N>::NT) void k_pois_r(const float2 *__restrict__ spec, float2 *__restrict__ outd,
+                                                    const float *__restrict__ amp, const float2 *__restrict__ tw,
+                                                    int nd) {
+  using G = RC<N>;
+  constexpr int NH = N / 2 + 1, R1 = G::R1, R2 = G::R2, SP = cube_spec_pitch(N);
+  constexpr int64_t stride = (int64_t)N * SP, plane = (int64_t)SP * N * N;
+  __shared__ float S[G::CB * G::SC];
+  __shared__ float2 twls[G::TWL ? N : 1];
+  const int tid = threadIdx.x, c = tid % G::CB, t = tid / G::CB;
+  if constexpr (G::TWL)
+    for (int e = tid; e < N; e += G::NT) twls[e] = tw[e];
+  const float2 *twl = G::TWL ? twls : tw;
+  const int y = blockIdx.y, d0 = blockIdx.z * nd;
+  const int kx0 = blockIdx.x * G::CB + c;
+  const bool ok = kx0 < NH;
+  const int kx = ok ? kx0 : NH - 1;
+  const uint32_t lo = (uint32_t)(((int64_t)t * stride + kx) * 8);
+  const float2 *src = spec + (int64_t)y * SP;
+  float2 v[R2];
+  const int s0 = opaque_zero();
+#pragma unroll
+  for (int m = 0; m < R2; ++m) v[m] = *boff(uni(src + (int64_t)(R1 * m) * stride, s0), lo);
+  __syncthreads();
+  blk_fft<N, -1>(v, c, t, S, twl);
+#pragma unroll 1
+  for (int d = d0; d < d0 + nd; ++d) {
+    float2 w[R2];
+#pragma unroll
+    for (int m = 0; m < R2; ++m) {
+      const int n = t + R1 * m;
+      float K = cube_kfac(d, kx, y, n, N);
+      if constexpr (KA) K = K * amp[((int64_t)n * N + y) * NH + kx];
+      w[m] = mul_ik(v[m], K);
+    }
+    blk_fft<N, +1>(w, c, t, S, twl);
+    if (ok) {
+      float2 *dst = outd + d * plane + (int64_t)y * SP;
+      const int s1 = opaque_zero();
+#pragma unroll
+      for (int m = 0; m < R2; ++m) *boff(uni(dst + (int64_t)(R1 * m) * stride, s1), lo) = w[m];
+    }
+  }
+}
+template <int N, bool KA>
+__global__ __launch_bounds__(FFT_T) void k_pois_z(const float2 *__restrict__ spec, float2 *__restrict__ outd,
+                                                const float *__restrict__ amp, const float2 *__restrict__ tw, int nd) {
+  constexpr int B = Cfg<N>::BS, TL = FFT_T / B, NP = lspan(N), NH = N / 2 + 1, SP = cube_spec_pitch(N);
+  constexpr int EPT = (B * N + FFT_T - 1) / FFT_T;
+  __shared__ float2 sm[B * NP];
+  const int tid = threadIdx.x, line = tid / TL, tl = tid % TL;
+  const int col0 = blockIdx.x * B, y = blockIdx.y, d0 = blockIdx.z * nd;
+  const int64_t stride = (int64_t)N * SP, plane = (int64_t)SP * N * N;
+  const float2 *src = spec + (int64_t)y * SP + col0;
+  float2 keep[EPT];
+#pragma unroll
+  for (int s = 0; s < EPT; ++s) {
+    const int idx = tid + s * FFT_T, l = idx % B, n = idx / B;
+    keep[s] = idx < B * N && col0 + l < NH ? src[n * stride + l] : make_float2(0.f, 0.f);
+  }
+#pragma unroll
+  for (int s = 0; s < EPT; ++s) {
+    const int idx = tid + s * FFT_T;
+    if (idx < B * N) sm[(idx % B) * NP + lpad(idx / B)] = keep[s];
+  }
+  __syncthreads();
+  line_fft<N, -1, TL>(sm + line * NP, tl, tw, N);
+#pragma unroll
+  for (int s = 0; s < EPT; ++s) {
+    const int idx = tid + s * FFT_T;
+    if (idx < B * N) keep[s] = sm[(idx % B) * NP + lpad(idx / B)];
+  }
+#pragma unroll 1
+  for (int d = d0; d < d0 + nd; ++d) {
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < EPT; ++s) {
+      const int idx = tid + s * FFT_T;
+      if (idx < B * N) {
+        const int l = idx % B, n = idx / B, kx = min(col0 + l, NH - 1);
+        float K = cube_kfac(d, kx, y, n, N);
+        if constexpr (KA) K = K * amp[((int64_t)n * N + y) * NH + kx];
+        sm[l * NP + lpad(n)] = mul_ik(keep[s], K);
+      }
+    }
+    __syncthreads();
+    line_fft<N, +1, TL>(sm + line * NP, tl, tw, N);
+    float2 *dst = outd + d * plane + (int64_t)y * SP + col0;
+    for (int idx = tid; idx < B * N; idx += FFT_T) {
+      const int l = idx % B, n = idx / B;
+      if (col0 + l < NH) dst[n * stride + l] = sm[l * NP + lpad(n)];
+    }
+  }
+}
+
+template <int N, bool KA>
+__global__ __launch_bounds__(RC<N>::NT) void k_pois_tr(const float2 *__restrict__ spec3, float2 *__restrict__ out,
+                                                     const float *__restrict__ amp, const float2 *__restrict__ tw) {
+  using G = RC<N>;
+  constexpr int NH = N / 2 + 1, R1 = G::R1, R2 = G::R2, SP = cube_spec_pitch(N);
+  constexpr int64_t stride = (int64_t)N * SP, plane = (int64_t)SP * N * N;
+  __shared__ float S[G::CB * G::SC];
+  __shared__ float2 twls[G::TWL ? N : 1];
+  const int tid = threadIdx.x, c = tid % G::CB, t = tid / G::CB;
+  if constexpr (G::TWL)
+    for (int e = tid; e < N; e += G::NT) twls[e] = tw[e];
+  const float2 *twl = G::TWL ? twls : tw;
+  const int y = blockIdx.y;
+  const int kx0 = blockIdx.x * G::CB + c;
+  const bool ok = kx0 < NH;
+  const int kx = ok ? kx0 : NH - 1;
+  const uint32_t lo = (uint32_t)(((int64_t)t * stride + kx) * 8);
+  float2 acc[R2];
+#pragma unroll
+  for (int m = 0; m < R2; ++m) acc[m] = make_float2(0.f, 0.f);
+  __syncthreads();
+#pragma unroll 1
+  for (int d = 0; d < 3; ++d) {
+    const float2 *src = spec3 + d * plane + (int64_t)y * SP;
+    float2 v[R2];
+    const int s0 = opaque_zero();
+#pragma unroll
+    for (int m = 0; m < R2; ++m) v[m] = *boff(uni(src + (int64_t)(R1 * m) * stride, s0), lo);
+    blk_fft<N, -1>(v, c, t, S, twl);
+#pragma unroll
+    for (int m = 0; m < R2; ++m) {
+      const int n = t + R1 * m;
+      float f = cube_kfac(d, kx, y, n, N);
+      if constexpr (KA) f = f * amp[((int64_t)n * N + y) * NH + kx];
+      acc[m].x += f * v[m].y;
+      acc[m].y -= f * v[m].x;
+    }
+  }
+  blk_fft<N, +1>(acc, c, t, S, twl);
+  if (ok) {
+    float2 *dst = out + (int64_t)y * SP;
+    const int s1 = opaque_zero();
+#pragma unroll
+    for (int m = 0; m < R2; ++m) *boff(uni(dst + (int64_t)(R1 * m) * stride, s1), lo) = acc[m];
+  }
+}
+template <int N, bool KA>
+__global__ __launch_bounds__(FFT_T) void k_pois_tz(const float2 *__restrict__ spec3, float2 *__restrict__ out,
+                                                 const float *__restrict__ amp, const float2 *__restrict__ tw) {
+  constexpr int B = Cfg<N>::BS, TL = FFT_T / B, NP = lspan(N), NH = N / 2 + 1, SP = cube_spec_pitch(N);
+  constexpr int EPT = (B * N + FFT_T - 1) / FFT_T;
+  __shared__ float2 sm[B * NP];
+  const int tid = threadIdx.x, line = tid / TL, tl = tid % TL;
+  const int col0 = blockIdx.x * B, y = blockIdx.y;
+  const int64_t stride = (int64_t)N * SP, plane = (int64_t)SP * N * N;
+  float2 acc[EPT];
+#pragma unroll
+  for (int s = 0; s < EPT; ++s) acc[s] = make_float2(0.f, 0.f);
+#pragma unroll 1
+  for (int d = 0; d < 3; ++d) {
+    const float2 *src = spec3 + d * plane + (int64_t)y * SP + col0;
+    float2 ld[EPT];
+#pragma unroll
+    for (int s = 0; s < EPT; ++s) {
+      const int idx = tid + s * FFT_T, l = idx % B, n = idx / B;
+      ld[s] = idx < B * N && col0 + l < NH ? src[n * stride + l] : make_float2(0.f, 0.f);
+    }
+    __syncthreads(); /* the last component's reads of sm are done */
+#pragma unroll
+    for (int s = 0; s < EPT; ++s) {
+      const int idx = tid + s * FFT_T;
+      if (idx < B * N) sm[(idx % B) * NP + lpad(idx / B)] = ld[s];
+    }
+    __syncthreads();
+    line_fft<N, -1, TL>(sm + line * NP, tl, tw, N);
+#pragma unroll
+    for (int s = 0; s < EPT; ++s) {
+      const int idx = tid + s * FFT_T;
+      if (idx < B * N) {
+        const int l = idx % B, n = idx / B, kx = min(col0 + l, NH - 1);
+        const float2 v = sm[l * NP + lpad(n)];
+        float f = cube_kfac(d, kx, y, n, N);
+        if constexpr (KA) f = f * amp[((int64_t)n * N + y) * NH + kx];
+        acc[s].x += f * v.y;
+        acc[s].y -= f * v.x;
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < EPT; ++s) {
+    const int idx = tid + s * FFT_T;
+    if (idx < B * N) sm[(idx % B) * NP + lpad(idx / B)] = acc[s];
+  }
+  __syncthreads();
+  line_fft<N, +1, TL>(sm + line * NP, tl, tw, N);
+  float2 *dst = out + (int64_t)y * SP + col0;
+  for (int idx = tid; idx < B * N; idx += FFT_T) {
+    const int l = idx % B, n = idx / B;
+    if (col0 + l < NH) dst[n * stride + l] = sm[l * NP + lpad(n)];
   }
 }
 
@@ -809,6 +1019,7 @@ __global__ __launch_bounds__(FFT_T) void k_c2r_x3(const float2 *__restrict__ spe
       m = fmaxf(m, f2);
     }
   }
+  if (!f2slots) return; /* uniform: the caller wants no maximum */
   red[tid] = m;
   __syncthreads();
   for (int s = FFT_T / 2; s > 0; s >>= 1) {
@@ -1013,8 +1224,9 @@ void cube_fft_destroy(FFTPlan *p) {
 }
 
 template <int N> struct Launch {
-  static int r2c(cube_ctx *c, FFTPlan *p, const float *in, float2 *out) {
-    const int64_t rows = (int64_t)N * N;
+  /* ncomp meshes behind one another, likewise their spectra: the rows of all */
+  static int r2c(cube_ctx *c, FFTPlan *p, const float *in, float2 *out, int ncomp = 1) {
+    const int64_t rows = (int64_t)N * N * ncomp;
     const int64_t nb = (rows + Cfg<N>::BC - 1) / Cfg<N>::BC;
     hipLaunchKernelGGL(k_r2c_x<N>, dim3((unsigned)nb), dim3(FFT_T), 0, c->stream, in, out, p->tw, rows);
     CUBE_LAUNCH_CHECK();
@@ -1031,12 +1243,9 @@ template <int N> struct Launch {
                          cstride);
       CUBE_LAUNCH_CHECK();
     } else {
-      dim3 g((NH + Cfg<N>::BS - 1) / Cfg<N>::BS, N);
-      for (int d = 0; d < ncomp; ++d) {
-        hipLaunchKernelGGL((k_c2c_s<N, DIR>), g, dim3(FFT_T), 0, c->stream, a + d * cstride, p->tw, NH, stride,
-                           ostride);
-        CUBE_LAUNCH_CHECK();
-      }
+      dim3 g((NH + Cfg<N>::BS - 1) / Cfg<N>::BS, N, ncomp);
+      hipLaunchKernelGGL((k_c2c_s<N, DIR>), g, dim3(FFT_T), 0, c->stream, a, p->tw, NH, stride, ostride, cstride);
+      CUBE_LAUNCH_CHECK();
     }
     return CUBE_OK;
   }
@@ -1106,8 +1315,35 @@ template <int N> struct Launch {
     }
     return CUBE_OK;
   }
-  static int c2r1(cube_ctx *c, FFTPlan *p, const float2 *spec, float *out) {
-    const int64_t rows = (int64_t)N * N;
+  /* The model's z passes.  Below 256^3 a line set does one component per
+     workgroup, forward transform redone, because a workgroup per line set
+     alone would leave CUs without work (64^3: 192 line sets). */
+  template <bool KA> static int pois(cube_ctx *c, FFTPlan *p, const float2 *spec, const float *amp, float2 *work3) {
+    constexpr int NH = N / 2 + 1, nd = N < 192 ? 1 : 3;
+    if constexpr (RC<N>::ok && N < 2048) {
+      dim3 g((NH + RC<N>::CB - 1) / RC<N>::CB, N, 3 / nd);
+      hipLaunchKernelGGL((k_pois_r<N, KA>), g, dim3(RC<N>::NT), 0, c->stream, spec, work3, amp, p->tw, nd);
+    } else {
+      dim3 g((NH + Cfg<N>::BS - 1) / Cfg<N>::BS, N, 3 / nd);
+      hipLaunchKernelGGL((k_pois_z<N, KA>), g, dim3(FFT_T), 0, c->stream, spec, work3, amp, p->tw, nd);
+    }
+    CUBE_LAUNCH_CHECK();
+    return CUBE_OK;
+  }
+  template <bool KA> static int pois_t(cube_ctx *c, FFTPlan *p, const float2 *work3, const float *amp, float2 *spec) {
+    constexpr int NH = N / 2 + 1;
+    if constexpr (RC<N>::ok && N < 2048) {
+      dim3 g((NH + RC<N>::CB - 1) / RC<N>::CB, N);
+      hipLaunchKernelGGL((k_pois_tr<N, KA>), g, dim3(RC<N>::NT), 0, c->stream, work3, spec, amp, p->tw);
+    } else {
+      dim3 g((NH + Cfg<N>::BS - 1) / Cfg<N>::BS, N);
+      hipLaunchKernelGGL((k_pois_tz<N, KA>), g, dim3(FFT_T), 0, c->stream, work3, spec, amp, p->tw);
+    }
+    CUBE_LAUNCH_CHECK();
+    return CUBE_OK;
+  }
+  static int c2r1(cube_ctx *c, FFTPlan *p, const float2 *spec, float *out, int ncomp = 1) {
+    const int64_t rows = (int64_t)N * N * ncomp;
     hipLaunchKernelGGL(k_c2r_x1<N>, dim3((unsigned)((rows + Cfg<N>::BC - 1) / Cfg<N>::BC)), dim3(FFT_T), 0,
                        c->stream, spec, out, p->tw, rows);
     CUBE_LAUNCH_CHECK();
@@ -1160,6 +1396,58 @@ int cube_fft_inverse_full(cube_ctx *c, FFTPlan *p, float2 *spec, float *out) {
     if ((st = Launch<N>::c2c_y<+1>(c, p, spec))) return st;            \
     return Launch<N>::c2r1(c, p, spec, out);                           \
   }
+    FFT_SIZES(CASE)
+#undef CASE
+  }
+  return CUBE_ERR_INVALID;
+}
+
+/* The Poisson force of rho: F_d = (1/div^3) C2R[i K_d R2C(rho)], three
+   components per mesh point.  spec, work3: scratch. */
+int cube_fft_poisson(cube_ctx *c, FFTPlan *p, const float *rho, float2 *spec, float2 *work3, float *force, float div) {
+  int st = cube_fft_r2c_3d(c, p, rho, spec);
+  if (st) return st;
+  switch (p->n) {
+#define CASE(N)                                                                    \
+  case N:                                                                          \
+    if ((st = Launch<N>::template pois<false>(c, p, spec, nullptr, work3))) return st; \
+    if ((st = Launch<N>::template c2c_y<+1>(c, p, work3, 3))) return st;           \
+    return Launch<N>::c2r3(c, p, work3, force, div, nullptr, 0.f, 0.f, 0);
+    FFT_SIZES(CASE)
+#undef CASE
+  }
+  return CUBE_ERR_INVALID;
+}
+/* out_d = C2R[i K_d amp R2C(in)], d = 0..2 behind one another (unnormalised) */
+int cube_fft_filter3(cube_ctx *c, FFTPlan *p, const float *in, const float *amp, float2 *spec, float2 *work3,
+                     float *out3) {
+  int st = cube_fft_r2c_3d(c, p, in, spec);
+  if (st) return st;
+  switch (p->n) {
+#define CASE(N)                                                                \
+  case N:                                                                      \
+    if ((st = Launch<N>::template pois<true>(c, p, spec, amp, work3))) return st; \
+    if ((st = Launch<N>::template c2c_y<+1>(c, p, work3, 3))) return st;       \
+    return Launch<N>::c2r1(c, p, work3, out3, 3);
+    FFT_SIZES(CASE)
+#undef CASE
+  }
+  return CUBE_ERR_INVALID;
+}
+/* The transpose: out = C2R[sum_d (-i K_d amp) R2C(in_d)] (amp null: 1) */
+int cube_fft_filter3_t(cube_ctx *c, FFTPlan *p, const float *in3, const float *amp, float2 *spec, float2 *work3,
+                       float *out) {
+  int st;
+  switch (p->n) {
+#define CASE(N)                                                                            \
+  case N:                                                                                  \
+    if ((st = Launch<N>::r2c(c, p, in3, work3, 3))) return st;                             \
+    if ((st = Launch<N>::template c2c_y<-1>(c, p, work3, 3))) return st;                   \
+    st = amp ? Launch<N>::template pois_t<true>(c, p, work3, amp, spec)                    \
+             : Launch<N>::template pois_t<false>(c, p, work3, amp, spec);                  \
+    if (st) return st;                                                                     \
+    if ((st = Launch<N>::template c2c_y<+1>(c, p, spec))) return st;                       \
+    return Launch<N>::c2r1(c, p, spec, out);
     FFT_SIZES(CASE)
 #undef CASE
   }

@@ -277,6 +277,18 @@ int cube_slots_zero(cube_ctx *c, unsigned long long *region, int nreg);
 int cube_slots_fold(cube_ctx *c, const unsigned long long *region, int nreg, int add, unsigned long long *d64,
                     unsigned *d32);
 
+/* K_d = k_d/k^2 for the mode (mx, my, mz), mx in [0, n/2], of an n^3 mesh,
+   k = 2 pi m/n; zero at k = 0 and on the Nyquist plane of axis d, so every
+   product spectrum stays Hermitian */
+__device__ static inline float cube_kfac(int d, int mx, int my, int mz, int n) {
+  const int m[3] = {mx, my <= n / 2 ? my : my - n, mz <= n / 2 ? mz : mz - n};
+  if (2 * (m[d] < 0 ? -m[d] : m[d]) == n) return 0.f;
+  const float s = 6.28318530717958648f / (float)n;
+  const float k[3] = {s * m[0], s * m[1], s * m[2]};
+  const float k2 = (k[0] * k[0] + k[1] * k[1]) + k[2] * k[2];
+  return k2 > 0.f ? k[d] / k2 : 0.f;
+}
+
 /* launchers (one file each) */
 int cube_drift(cube_ctx *c, float dt_old, float dt, float vz_max, float sigma_vi, cube_vstats *out);
 int cube_vdec_table(cube_ctx *c, double *dst, float sigma);
@@ -302,6 +314,12 @@ float2 *cube_fft_plan_twiddles(FFTPlan *p);
 /* the same with the size-n twiddles already on the device at tw (no plan) */
 int cube_fft_forward_full_tw(cube_ctx *c, int n, float2 *tw, const float *in, float2 *out);
 int cube_fft_inverse_full(cube_ctx *c, FFTPlan *p, float2 *spec, float *out);
+/* the differentiable model's operators (cube_fft.hip) */
+int cube_fft_poisson(cube_ctx *c, FFTPlan *p, const float *rho, float2 *spec, float2 *work3, float *force, float div);
+int cube_fft_filter3(cube_ctx *c, FFTPlan *p, const float *in, const float *amp, float2 *spec, float2 *work3,
+                     float *out3);
+int cube_fft_filter3_t(cube_ctx *c, FFTPlan *p, const float *in3, const float *amp, float2 *spec, float2 *work3,
+                       float *out);
 
 int cube_fine_deposit(cube_ctx *c, float mass_p, double *testrhof);
 /* device slots (in dred) of the deposits' mesh sums */

@@ -11,8 +11,7 @@
  * box, each on its own stream, joined at the end) and replays it with a
  * single launch; mode 0 runs the same kernels box after box on one stream
  * (the per-box loop).  cube_batch_tune times candidate launch shapes of the
- * model's particle and mesh loops for every distinct box size and keeps the
- * fastest.  The I/O pointers are device pointers fixed by set_io; a captured
+ * model's particle loops for every distinct box size and keeps the fastest.  The I/O pointers are device pointers fixed by set_io; a captured
  * graph keeps using them (call set_io before the first mode-1 run, or again
  * to force a new capture).
  */

@@ -20,9 +20,13 @@
  * scatter (the transpose of the gather), the Poisson operator with the
  * conjugate factor -i k/k^2, the CIC weight-gradient gather (the position
  * derivative of deposit and gather), the transposed drift and kicks, and
- * the transposed IC filter.  The forward either keeps the positions of
- * every step (checkpoint=1: 12 bytes per particle per step) or only the
- * ICs and recomputes (checkpoint=0: O(nsteps^2) force evaluations).
+ * the transposed IC filter.  With checkpoint=1 the forward keeps the
+ * positions of every step (12 bytes per particle per step) and, while those
+ * of all steps take at most an eighth of the device's free memory when the
+ * box is created, the force meshes (12 bytes per mesh point per step), which
+ * the adjoint else forms again.  With checkpoint=0 it keeps within 24 bytes
+ * per mesh point: the positions of every step if they fit, else position and
+ * momentum of every k-th step, from which the others are recomputed.
  *
  * Array arguments of forward/adjoint are DEVICE pointers on the context's
  * device (e.g. torch tensors' data_ptr()); the amplitude and schedule are
@@ -41,7 +45,7 @@ typedef struct {
   int32_t ng;         /* particles per dimension (lattice), power of two or 2^a 3^b */
   int32_t nf;         /* density / force mesh per dimension, a multiple of ng */
   int32_t nsteps;     /* KDK steps */
-  int32_t checkpoint; /* 1: keep every step's positions; 0: recompute */
+  int32_t checkpoint; /* 1: keep every step; 0: keep what fits 24 bytes per mesh point, recompute the rest */
   int32_t device;
   int32_t reserved;
 } cube_dpm_params;

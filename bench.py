@@ -110,7 +110,7 @@ def stage_bytes(np_, nf3, nc3, bx, bv):
 
 MAIN_KERNEL = {
     "drift": "k_drift_dest+k_place_ranked+k_sort_small+k_drift_final2",
-    "pp": "k_pp_blk", "fine_deposit": "k_fine_deposit_cc", "fine_kick": "k_kick<fine>",
+    "pp": "k_pp_blk", "fine_deposit": "k_fine_deposit", "fine_kick": "k_kick<fine>",
     "coarse_deposit": "k_coarse_deposit", "coarse_kick": "k_kick<coarse>",
     "fine_fft": "k_r2c_x+k_c2c_r", "fine_inverse": "k_green_r+k_c2c_r+k_c2r_x3",
     "coarse_force": "coarse fft kernels",
@@ -122,7 +122,7 @@ CONCURRENT = {"pp": "fine_deposit+fine_fft+fine_inverse+coarse_deposit+coarse_fo
               "fine_deposit": "pp+coarse_deposit+coarse_force", "coarse_deposit": "pp+fine_deposit+fine_fft",
               "coarse_force": "pp+fine_fft"}
 # kernel-name prefixes in the rocprofv3 PMC traffic table, per single-kernel stage
-PMC_NAMES = {"pp": ["k_pp_blk<"], "fine_deposit": ["k_fine_deposit_cc<"], "fine_kick": ["k_kick<"],
+PMC_NAMES = {"pp": ["k_pp_blk<"], "fine_deposit": ["k_fine_deposit<"], "fine_kick": ["k_kick<"],
              "coarse_deposit": ["k_coarse_deposit<"], "coarse_kick": ["k_kick<"]}
 PMC_TABLE = os.path.join(ROOT, "profiles", "pmpp512_step_pmc_traffic.md")
 

@@ -63,7 +63,7 @@ static void free_all(cube_ctx *c) {
                   c->cstart, c->cstart2, c->dest, c->key, c->sortbuf, c->fill, c->xdest, c->xkey, c->rank, c->xrank, c->fbflag,
                   c->tanf_tab, c->venc_tab, c->vdec0, c->vdec1, c->rho_f, c->spec_f, c->specd_f, c->force_f,
                   c->kern_f, c->rho_c, c->spec_c, c->specd_c, c->force_c, c->kern_c, c->dred,
-                  c->ured, c->ired, c->scanbuf, c->vpart, c->slots, c->ppdefer, c->ppitems};
+                  c->ured, c->fdsum, c->fdlist, c->fdmask, c->ired, c->scanbuf, c->vpart, c->slots, c->ppdefer, c->ppitems};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   cube_fft_destroy(c->plan_f);
@@ -226,6 +226,13 @@ extern "C" int cube_ctx_create(const cube_params *p, cube_ctx **out) {
   st |= dalloc(&c->kern_c, 3 * (c->nc / 2 + 1) * c->nc * c->nc); /* unpadded [d][kz][ky][kx] */
   st |= dalloc(&c->dred, 8192);
   st |= dalloc(&c->ured, 64);
+  {
+    const int64_t nbt = (nt + 3) / 4, nb4 = nbt * nbt * nbt * c->ntiles;
+    st |= dalloc(&c->fdsum, nb4);
+    st |= dalloc(&c->fdlist, nb4);
+    st |= dalloc(&c->fdmask, nb4);
+  }
+  if (!st && hipMemset(c->ured, 0, 64 * sizeof(uint64_t)) != hipSuccess) st = CUBE_ERR_HIP;
   st |= dalloc(&c->slots, CUBE_NSLOTREG * CUBE_SLOTS);
   st |= dalloc(&c->ired, 4096);
   st |= dalloc(&c->scanbuf, c->ncells / 1024 + 4);

@@ -90,6 +90,9 @@ struct cube_ctx {
   double *dred;             /* 8192 doubles: [0,4096) reductions of work on `stream`,
                                [4096,8192) of work on `side` */
   uint64_t *ured;           /* 64 words */
+  double *fdsum;            /* fine deposit: one sum per block of 4^3 coarse cells */
+  int32_t *fdlist;          /* and its list of blocks with crowded cells (length in ured) */
+  uint64_t *fdmask;         /* those cells, by block */
   int64_t *ired;            /* 4096 */
   int64_t *scanbuf;         /* ncells/1024 + 2 block sums of the scan */
   double *vpart;            /* 3 per finalize block of the drift (velocity sums) */
@@ -323,6 +326,7 @@ int cube_fft_filter3_t(cube_ctx *c, FFTPlan *p, const float *in3, const float *a
 
 int cube_fine_deposit(cube_ctx *c, float mass_p, double *testrhof);
 /* device slots (in dred) of the deposits' mesh sums */
+#define CUBE_URED_FDHEAVY 32 /* word of ured: the fine deposit's crowded blocks */
 #define CUBE_DRED_FINE_SUM 4000
 #define CUBE_DRED_COARSE_SUM (4096 + 4000)
 int cube_fine_kick(cube_ctx *c, float a_mid, float dt, float sigma_vi, float sigma_vi_new, int sync);

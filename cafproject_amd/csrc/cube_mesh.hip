@@ -44,292 +44,7 @@ __global__ __launch_bounds__(64) void k_sum_parts1(const double *part, int nb, d
   if (t == 0) *out = r[0];
 }
 
-/*
- * Fine deposit, one thread per coarse cell C owning its 4x4x4 fine cells.
- * Every particle that can reach them lives in the 2x2x2 source cells
- * {C-1,C} per axis.  The thread walks those cells in the reference's visit
- * order -- z by (ilayer,k), then y, then x, then l -- and adds each hit into
- * a per-thread LDS accumulator of its 64 fine cells.  Restricted to one fine
- * cell this is exactly that cell's reference order, so the sums are
- * bit-identical; each particle is read by the 8 threads whose blocks its
- * cloud can touch instead of by all 64+ fine cells around it.
- */
-/* global coordinates of cell cg of the nc^3 x-fastest mesh (32-bit
-   divisions while the index fits, which is every mesh up to 1290^3) */
-__device__ __forceinline__ void gcoords(int64_t cg, int nc, int gg[3]) {
-  if (cg <= 0x7fffffff) {
-    const uint32_t c = (uint32_t)cg, n = (uint32_t)nc, q = c / n, z = q / n;
-    gg[0] = (int)(c - q * n);
-    gg[1] = (int)(q - z * n);
-    gg[2] = (int)z;
-  } else {
-    gg[0] = (int)(cg % nc);
-    gg[1] = (int)((cg / nc) % nc);
-    gg[2] = (int)(cg / ((int64_t)nc * nc));
-  }
-}
-#define FD_T 128
 __device__ __forceinline__ int rl_i(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
-__device__ __forceinline__ float rl_f(float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); }
-template <int IX>
-__global__ __launch_bounds__(FD_T) void k_fine_deposit_cc(const typename IntOf<IX>::T *__restrict__ xp,
-                                                          const int32_t *__restrict__ rhoc,
-                                                          const int64_t *__restrict__ cstart, Geo g, float mass,
-                                                          float *__restrict__ rho, double *__restrict__ part,
-                                                          int heavy_at) {
-  __shared__ float acc[64 * FD_T]; /* element q of thread t at q*FD_T + t: conflict free */
-  const int nc = g.nc, nf = 4 * nc;
-  const int64_t nc3 = (int64_t)nc * nc * nc;
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  double tsum = 0;
-  for (int64_t cg = blockIdx.x * (int64_t)FD_T + t; cg - t < nc3; cg += (int64_t)gridDim.x * FD_T) {
-    const bool live = cg < nc3;
-    for (int q = 0; q < 64; ++q) acc[q * FD_T + t] = 0.f;
-    int gg[3] = {0, 0, 0}, C[3] = {1, 1, 1}, za = 0, zb = 0;
-    int npc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    int64_t p0c[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    bool heavy = false;
-    if (live) {
-      gcoords(cg, nc, gg);
-      int T[3];
-#pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        T[a] = gg[a] / g.nt;
-        C[a] = gg[a] - T[a] * g.nt + 1; /* 1-based local coarse cell */
-      }
-      /* cell ids are linear in the local coordinates and the tile index, so
-         a source below C on an axis is C's id plus that axis's step down:
-         -stride inside the tile, the wrapped neighbour tile's last cell at
-         the tile's low edge */
-      const int64_t nt = g.nt, nt3 = nt * nt * nt;
-      const int64_t cidC = g.cid(C[0] - 1, C[1] - 1, C[2] - 1, T[0] + g.nnt * (T[1] + g.nnt * T[2]));
-      int64_t dm[3];
-      {
-        const int64_t stride[3] = {1, nt, nt * nt}, tstride[3] = {nt3, nt3 * g.nnt, nt3 * g.nnt * g.nnt};
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-          dm[a] = C[a] > 1 ? -stride[a] : stride[a] * (nt - 1) + tstride[a] * (T[a] > 0 ? -1 : g.nnt - 1);
-      }
-      /* the two source z cells in (ilayer, k) order, ilayer = (k-k0) mod 3 */
-      za = C[2] - 1;
-      zb = C[2];
-      {
-        const int k0 = 2 - g.ncb;
-        const int ka = ((za - k0) % 3 + 3) % 3, kb = ((zb - k0) % 3 + 3) % 3;
-        if (ka > kb) {
-          za = C[2];
-          zb = C[2] - 1;
-        }
-      }
-      /* counts and starts of the 8 source cells, all loads issued up front */
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int64_t cc = cidC + ((q & 1) ? 0 : dm[0]) + (((q >> 1) & 1) ? 0 : dm[1]) +
-                           ((((q >> 2) ? zb : za) == C[2]) ? 0 : dm[2]);
-        npc[q] = rhoc[cc];
-        p0c[q] = cstart[cc];
-      }
-      heavy = ((npc[0] + npc[1]) + (npc[2] + npc[3])) + ((npc[4] + npc[5]) + (npc[6] + npc[7])) > heavy_at;
-      if (!heavy)
-#pragma unroll 1
-      for (int qz = 0; qz < 2; ++qz)
-#pragma unroll 1
-        for (int qy = 0; qy < 2; ++qy)
-#pragma unroll 1
-          for (int qx = 0; qx < 2; ++qx) {
-            const int ci[3] = {C[0] - 1 + qx, C[1] - 1 + qy, qz ? zb : za};
-            const int qi = (qz * 2 + qy) * 2 + qx;
-            int np = npc[0];
-            int64_t p0 = p0c[0];
-#pragma unroll
-            for (int q = 1; q < 8; ++q) { /* register select, no dynamic indexing */
-              np = qi == q ? npc[q] : np;
-              p0 = qi == q ? p0c[q] : p0;
-            }
-            /* a source cell below C on an axis reaches C's 4^3 fine cells
-               only through particles in its last fine sub-cell on that axis
-               (code >> sh == 3), so those visits first mark the candidates
-               of each 64-particle chunk in a mask and then visit only them,
-               in increasing l.  Where the real(4) tempx is inexact (2-byte
-               codes, nt > 128) the top code of a lower sub-cell can round up
-               onto the boundary itself, and its weight past the boundary is
-               then exactly 0: skipping it drops only +0 terms. */
-            const int sh = IX == 1 ? 6 : 14;
-            const bool ex = qx == 0, ey = qy == 0, ez = ci[2] == C[2] - 1;
-            for (int lb = 0; lb < np; lb += 64) {
-              const int nb = min(64, np - lb);
-              uint64_t mask = nb == 64 ? ~0ull : ((1ull << nb) - 1ull);
-              if (ex || ey || ez) {
-                uint64_t m = 0;
-                for (int l0 = 0; l0 < nb; l0 += 4) {
-                  int32_t c4[4][3];
-#pragma unroll
-                  for (int u = 0; u < 4; ++u) {
-                    const int64_t q = p0 + lb + min(l0 + u, nb - 1);
-#pragma unroll
-                    for (int a = 0; a < 3; ++a) c4[u][a] = (int32_t)xp[3 * q + a];
-                  }
-#pragma unroll
-                  for (int u = 0; u < 4; ++u) {
-                    const bool pass = (!ex || (cube_ucode(IX, c4[u][0]) >> sh) == 3) &&
-                                      (!ey || (cube_ucode(IX, c4[u][1]) >> sh) == 3) &&
-                                      (!ez || (cube_ucode(IX, c4[u][2]) >> sh) == 3);
-                    m |= (uint64_t)(pass ? 1 : 0) << (l0 + u);
-                  }
-                }
-                mask &= m;
-              }
-              /* two candidates per round so that both code loads are in flight */
-              while (mask) {
-                int lq[2];
-                lq[0] = lb + __builtin_ctzll(mask);
-                mask &= mask - 1ull;
-                const bool two = mask != 0ull;
-                lq[1] = two ? lb + __builtin_ctzll(mask) : lq[0];
-                if (two) mask &= mask - 1ull;
-                int32_t cq[2][3];
-#pragma unroll
-                for (int u = 0; u < 2; ++u)
-#pragma unroll
-                  for (int a = 0; a < 3; ++a) cq[u][a] = (int32_t)xp[3 * (p0 + lq[u]) + a];
-#pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                  if (u == 1 && !two) break;
-                  int r[3];
-                  float d1[3];
-#pragma unroll
-                  for (int a = 0; a < 3; ++a) {
-                    /* ncell*(i-1)+ncell*(x offset) rounded to real(4) (W/pm.f90:63):
-                       both terms are exact floats, so one float add rounds it */
-                    /* (u+0.5)*4*2^-8izipx: exact in real(4) as in real(8) */
-                    const float off4 = ((float)cube_ucode(IX, cq[u][a]) + 0.5f) * (IX == 1 ? 0x1p-6f : 0x1p-14f);
-                    const float tempx = (float)(4 * (ci[a] - 1)) + off4;
-                    const int i1 = (int)floorf(tempx) + 1;
-                    d1[a] = (float)i1 - tempx;
-                    r[a] = i1 - 4 * (C[a] - 1) - 1; /* 0-based in C's block */
-                  }
-#pragma unroll
-                  for (int cz = 0; cz < 2; ++cz) {
-                    const int z = r[2] + cz;
-                    if (z < 0 || z > 3) continue;
-                    const float wz = cz ? 1.0f - d1[2] : d1[2];
-#pragma unroll
-                    for (int cy = 0; cy < 2; ++cy) {
-                      const int y = r[1] + cy;
-                      if (y < 0 || y > 3) continue;
-                      const float wy = cy ? 1.0f - d1[1] : d1[1];
-#pragma unroll
-                      for (int cx = 0; cx < 2; ++cx) {
-                        const int x = r[0] + cx;
-                        if (x < 0 || x > 3) continue;
-                        const float wx = cx ? 1.0f - d1[0] : d1[0];
-                        float &sacc = acc[((z * 4 + y) * 4 + x) * FD_T + t];
-                        sacc = sacc + wx * wy * wz * mass;
-                      }
-                    }
-                  }
-                }
-              }
-            }
-          }
-    }
-    /* a heavy lane's cell is formed by its whole wave: lane f owns fine
-       cell f = (z*4+y)*4+x of it and adds, in the same order and with the
-       same expression as the lane would, the terms of the candidates that
-       64 lanes decode at a time */
-    uint64_t hm = __ballot(live && heavy);
-    while (hm) {
-      const int L = __builtin_ctzll(hm);
-      hm &= hm - 1;
-      const int LC[3] = {rl_i(C[0], L), rl_i(C[1], L), rl_i(C[2], L)};
-      const int Lza = rl_i(za, L), Lzb = rl_i(zb, L);
-      const int fx = lane & 3, fy = (lane >> 2) & 3, fz = lane >> 4;
-      float sacc = 0.f;
-      for (int qi = 0; qi < 8; ++qi) {
-        const int qx = qi & 1, qy = (qi >> 1) & 1, qz = qi >> 2;
-        const int ci[3] = {LC[0] - 1 + qx, LC[1] - 1 + qy, qz ? Lzb : Lza};
-        int np = 0;
-        int64_t p0 = 0;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) { /* the owner's counts and starts */
-          const int nq = rl_i(npc[q], L);
-          const int64_t pq = (int64_t)(((uint64_t)(uint32_t)rl_i((int)(p0c[q] >> 32), L) << 32) |
-                                       (uint64_t)(uint32_t)rl_i((int)(p0c[q] & 0xffffffff), L));
-          np = qi == q ? nq : np;
-          p0 = qi == q ? pq : p0;
-        }
-        const int sh = IX == 1 ? 6 : 14;
-        const bool ex = qx == 0, ey = qy == 0, ez = ci[2] == LC[2] - 1;
-        for (int lb = 0; lb < np; lb += 64) {
-          const int l = lb + lane;
-          bool pass = false;
-          float d1v[3] = {0.f, 0.f, 0.f}, d2v[3] = {0.f, 0.f, 0.f};
-          int rp = 0;
-          if (l < np) {
-            int32_t cq[3];
-#pragma unroll
-            for (int a = 0; a < 3; ++a) cq[a] = (int32_t)xp[3 * (p0 + l) + a];
-            pass = (!ex || (cube_ucode(IX, cq[0]) >> sh) == 3) && (!ey || (cube_ucode(IX, cq[1]) >> sh) == 3) &&
-                   (!ez || (cube_ucode(IX, cq[2]) >> sh) == 3);
-            if (pass) {
-              int r[3];
-#pragma unroll
-              for (int a = 0; a < 3; ++a) {
-                const float off4 = ((float)cube_ucode(IX, cq[a]) + 0.5f) * (IX == 1 ? 0x1p-6f : 0x1p-14f);
-                const float tempx = (float)(4 * (ci[a] - 1)) + off4;
-                const int i1 = (int)floorf(tempx) + 1;
-                d1v[a] = (float)i1 - tempx;
-                d2v[a] = 1.0f - d1v[a];
-                r[a] = i1 - 4 * (LC[a] - 1) - 1;
-              }
-              rp = ((r[0] + 1) & 7) | (((r[1] + 1) & 7) << 3) | (((r[2] + 1) & 7) << 6);
-            }
-          }
-          uint64_t m = __ballot(pass);
-          while (m) { /* candidates in increasing l, read from their lanes */
-            const int i = __builtin_ctzll(m);
-            m &= m - 1;
-            const int ri = rl_i(rp, i);
-            const int cx = fx - ((ri & 7) - 1), cy = fy - (((ri >> 3) & 7) - 1), cz = fz - (((ri >> 6) & 7) - 1);
-            const float ax0 = rl_f(d1v[0], i), ax1 = rl_f(d2v[0], i), ay0 = rl_f(d1v[1], i), ay1 = rl_f(d2v[1], i);
-            const float az0 = rl_f(d1v[2], i), az1 = rl_f(d2v[2], i);
-            if ((unsigned)cx <= 1u && (unsigned)cy <= 1u && (unsigned)cz <= 1u) {
-              const float wx = cx ? ax1 : ax0, wy = cy ? ay1 : ay0, wz = cz ? az1 : az0;
-              sacc = sacc + wx * wy * wz * mass;
-            }
-          }
-        }
-      }
-      acc[lane * FD_T + wv * 64 + L] = sacc;
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-    if (live) {
-      const int64_t f0x = 4 * (int64_t)gg[0], f0y = 4 * (int64_t)gg[1], f0z = 4 * (int64_t)gg[2];
-      for (int z = 0; z < 4; ++z)
-        for (int y = 0; y < 4; ++y) {
-          float4 v;
-          v.x = acc[((z * 4 + y) * 4 + 0) * FD_T + t];
-          v.y = acc[((z * 4 + y) * 4 + 1) * FD_T + t];
-          v.z = acc[((z * 4 + y) * 4 + 2) * FD_T + t];
-          v.w = acc[((z * 4 + y) * 4 + 3) * FD_T + t];
-          *reinterpret_cast<float4 *>(rho + ((f0z + z) * nf + (f0y + y)) * nf + f0x) = v;
-          tsum += ((double)v.x + (double)v.y) + ((double)v.z + (double)v.w);
-        }
-    }
-  }
-  __syncthreads();
-  double *red = reinterpret_cast<double *>(acc);
-  red[t] = tsum;
-  __syncthreads();
-  for (int o = FD_T / 2; o > 0; o >>= 1) {
-    if (t < o) red[t] += red[t + o];
-    __syncthreads();
-  }
-  if (t == 0) part[blockIdx.x] = red[0];
-}
-
 /*
  * Coarse deposit, W/pm.f90:205-267: one wave per block of 4x4x4 mesh cells of
  * a tile (clipped at the tile's high edge), one lane per mesh cell.  A mesh
@@ -735,18 +450,485 @@ __global__ __launch_bounds__(64 * NW, 4) void k_coarse_deposit(const typename In
   }
 }
 
+/*
+ * Fine deposit, W/pm.f90:49-108: one wave per block of 4x4x4 coarse cells of
+ * a tile, a lane per coarse cell owning its 4x4x4 fine cells.  Every particle
+ * that reaches them lives in the 2x2x2 source cells {C-1,C} per axis; the lane
+ * adds their terms in the reference's order -- z by (ilayer, k), then y, x,
+ * l -- into LDS accumulators, so each fine cell holds the reference's bits.
+ *
+ * The block's 5^3 source cells go through LDS in three phases by ilayer (the
+ * planes of one ilayer are 3 apart, so a lane needs at most one of them), as
+ * raw codes in batches of 64 slots with three ballots each: which particles
+ * sit in the last fine sub-cell (code >> sh == 3) on each axis.  Only those
+ * reach the next coarse cell, so a lane's hits of two cells of a row are a few
+ * logic operations.  Where the real(4) coordinate is inexact (EX false:
+ * 2-byte codes, nt > 128) the top code of a lower sub-cell can round up onto
+ * the boundary itself, and its weight past it is then exactly 0: leaving it
+ * out drops only +0 terms.
+ *
+ * A hit's two planes per axis that lie in the cell are b, b+1 with b = 0..2
+ * and weights that are 0 where a plane lies outside, so its 8 sums sit at
+ * constant distances from one address and need no bounds checks; a +0 term
+ * leaves a sum as it is.
+ *
+ * A cell whose 8 sources hold more than `heavy_at` particles would hold its
+ * wave up: its lane sits out, and the block goes to a list for
+ * k_fine_deposit_heavy with the mask of such cells.
+ *
+ * Bound by VALU issue (some 4,000 instructions a block, half of them the hits)
+ * with the 16 KiB of sums leaving 7 waves a CU to hide the rest.  Both kernels
+ * and the sum, against a thread per coarse cell walking its 8 cells in global
+ * memory with crowded cells handed round its wave: 5.12 -> 3.05 ms on the
+ * 256^3 mesh of 512^3 particles, 1.79 -> 1.16 ms on
+ * 128^3 at z = 3, 0.117 -> 0.086 ms on 64^3, 0.057 -> 0.045 ms on 16^3, 1.48
+ * -> 0.83 ms on the clustered 128^3 at z = 0 with 1-byte codes.
+ */
+template <int IX> struct FdLds { /* per wave */
+  static constexpr int NB = 10; /* batches staged at once: a phase's 10 rows of up to 64 */
+  float acc[64 * 64];                         /* fine cell q of lane t at q*64 + t: conflict free */
+  typename CdWord<IX>::T word[NB * 64];
+  uint64_t top[NB][3];
+  int64_t start[25][2]; /* a row's first particle, and that of its second cell */
+  int pre[25][6];
+  int rb[2][10]; /* a row's first batch, by phase parity */
+  int cax[3][5];
+};
+/* the two planes b, b+1 of an axis and their weights: a particle of code u in
+   the lane's own cell, or (below) in the last sub-cell of the one below.  EX
+   as in cd_fields; else ci is the particle's cell and C the lane's (1-based,
+   tile frame) */
+template <int IX, bool EX>
+__device__ __forceinline__ void fd_axis(uint32_t u, bool below, int ci, int C, int &b, float &wa, float &wb) {
+  if constexpr (EX) {
+    constexpr int sh = IX == 1 ? 6 : 14;
+    constexpr float s = 1.0f / (float)(1 << sh);
+    const float k = (float)(u & ((1u << sh) - 1u));
+    const float d1 = fmaf(k, -s, 1.0f - 0.5f * s), d2 = fmaf(k, s, 0.5f * s); /* exact */
+    const int sub = (int)(u >> sh);
+    const bool last = sub == 3;
+    b = below ? 0 : min(sub, 2);
+    wa = below ? d2 : (last ? 0.f : d1);
+    wb = below ? 0.f : (last ? d1 : d2);
+  } else {
+    /* ncell*(i-1)+ncell*(x offset) rounded to real(4) (W/pm.f90:63): both terms
+       are exact floats, so one float add rounds it */
+    const float off4 = ((float)u + 0.5f) * (IX == 1 ? 0x1p-6f : 0x1p-14f);
+    const float tempx = (float)(4 * (ci - 1)) + off4;
+    const int i1 = (int)floorf(tempx) + 1, r = i1 - 4 * (C - 1) - 1;
+    const float d1 = (float)i1 - tempx, d2 = 1.0f - d1;
+    b = min(max(r, 0), 2);
+    wa = r == b ? d1 : (r + 1 == b ? d2 : 0.f);
+    wb = r == b + 1 ? d1 : (r == b ? d2 : 0.f);
+  }
+}
+template <int IX> __device__ __forceinline__ uint32_t fd_code(typename CdWord<IX>::T w, int a) {
+  return (uint32_t)(w >> (8 * IX * a)) & (IX == 1 ? 0xffu : 0xffffu);
+}
+/* lane's fine cells from LDS to the mesh, and their sum over the wave in a
+   fixed order */
+__device__ __forceinline__ double fd_store(const float *acc, int lane, bool live, int64_t X, int64_t Y, int64_t Z, int64_t nf,
+                                           float *__restrict__ rho) {
+  double t = 0;
+  if (live) {
+    for (int z = 0; z < 4; ++z)
+      for (int y = 0; y < 4; ++y) {
+        float4 v;
+        v.x = acc[((z * 4 + y) * 4 + 0) * 64 + lane];
+        v.y = acc[((z * 4 + y) * 4 + 1) * 64 + lane];
+        v.z = acc[((z * 4 + y) * 4 + 2) * 64 + lane];
+        v.w = acc[((z * 4 + y) * 4 + 3) * 64 + lane];
+        *reinterpret_cast<float4 *>(rho + ((4 * Z + z) * nf + (4 * Y + y)) * nf + 4 * X) = v;
+        t += ((double)v.x + (double)v.y) + ((double)v.z + (double)v.w);
+      }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+  return t;
+}
+/* block b of the 4^3-cell blocks: tile T, first coarse cell m0 (0-based, tile frame) */
+__device__ __forceinline__ void blk4(int b, const Geo &g, int nbt, int T[3], int m0[3]) {
+  const uint32_t ub = (uint32_t)b, un = (uint32_t)nbt, q1 = ub / un, q2 = q1 / un, t = q2 / un;
+  const uint32_t tn = (uint32_t)g.nnt, t1 = t / tn;
+  T[0] = (int)(t - t1 * tn);
+  T[1] = (int)(t1 % tn);
+  T[2] = (int)(t1 / tn);
+  m0[0] = 4 * (int)(ub - q1 * un);
+  m0[1] = 4 * (int)(q1 - q2 * un);
+  m0[2] = 4 * (int)(q2 - t * un);
+}
+
+template <int IX, bool EX>
+__global__ __launch_bounds__(64) void k_fine_deposit(const typename IntOf<IX>::T *__restrict__ xp,
+                                                     const int32_t *__restrict__ rhoc,
+                                                     const int64_t *__restrict__ cstart, Geo g, float mass,
+                                                     float *__restrict__ rho, double *__restrict__ bsum, int nblk,
+                                                     int heavy_at, int32_t *__restrict__ hlist,
+                                                     uint64_t *__restrict__ hmask,
+                                                     unsigned long long *__restrict__ hcount) {
+  typedef typename CdWord<IX>::T W;
+  constexpr int PB = 3 * IX, sh = IX == 1 ? 6 : 14, NB = FdLds<IX>::NB;
+  __shared__ FdLds<IX> S;
+  const int lane = threadIdx.x;
+  const char *xb8 = reinterpret_cast<const char *>(xp);
+  const int nt = g.nt, nbt = (nt + 3) / 4;
+  const int xi = lane & 3, yi = (lane >> 2) & 3, zi = lane >> 4;
+  for (int b = blockIdx.x; b < nblk; b += gridDim.x) {
+    int T[3], m0[3];
+    blk4(b, g, nbt, T, m0);
+    wave_lds_sync();
+    /* the 5^3 source cells m0-1..m0+3, those past the tile empty */
+    if (lane < 15) {
+      const int a = lane / 5, sc = (a == 0 ? m0[0] : a == 1 ? m0[1] : m0[2]) - 1 + lane % 5;
+      int ta = a == 0 ? T[0] : a == 1 ? T[1] : T[2], l = sc;
+      if (sc < 0) {
+        l = nt - 1;
+        ta = ta > 0 ? ta - 1 : g.nnt - 1;
+      }
+      const int st = a == 0 ? 1 : a == 1 ? nt : nt * nt, ts = a == 0 ? 1 : a == 1 ? g.nnt : g.nnt * g.nnt;
+      S.cax[a][lane % 5] = sc >= nt ? -1 : l * st + nt * nt * nt * ts * ta;
+    }
+    wave_lds_sync();
+    const int i2 = m0[0] == 0 ? 1 : 0; /* at the tile's low edge cell 0 lies in the neighbour tile */
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int q = lane + 64 * u;
+      if (q < 125) {
+        int cnt = 0;
+        const int cx = S.cax[0][q % 5], cy = S.cax[1][(q / 5) % 5], cz = S.cax[2][q / 25];
+        if ((cx | cy | cz) >= 0) {
+          const int cc = cx + cy + cz;
+          cnt = rhoc[cc];
+          if (q % 5 < 2) S.start[q / 5][q % 5] = cstart[cc];
+        }
+        S.pre[q / 5][q % 5 + 1] = cnt;
+      }
+    }
+    wave_lds_sync();
+    if (lane < 25) {
+      int acc = 0;
+      S.pre[lane][0] = 0;
+#pragma unroll
+      for (int q = 1; q < 6; ++q) {
+        acc += S.pre[lane][q];
+        S.pre[lane][q] = acc;
+      }
+    }
+    wave_lds_sync();
+    const int kz = (m0[2] - 2 + g.ncb + 3) % 3; /* ilayer of plane 0 (k = m0z, 1-based) */
+    bool live = m0[0] + xi < nt && m0[1] + yi < nt && m0[2] + zi < nt;
+    {
+      int tot = 0; /* particles in the lane's 8 source cells */
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int r = (zi + (j >> 1)) * 5 + yi + (j & 1);
+        tot += S.pre[r][xi + 2] - S.pre[r][xi];
+      }
+      const uint64_t hv = __ballot(live && tot > heavy_at);
+      if (hv) { /* uniform */
+        if (lane == 0) {
+          hmask[b] = hv;
+          hlist[atomicAdd(hcount, 1ull)] = b;
+        }
+        live = live && tot <= heavy_at;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 16; ++q) reinterpret_cast<float4 *>(S.acc)[q * 64 + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+    float *acc = S.acc + lane;
+    /* lane t < 10: row t of the phase of ilayer il, y = t/2, plane p0 + 3*(t&1) */
+    struct Phase {
+      int nrow, sB, bsc, rb, nb;
+      int64_t dA, dB;
+    };
+    auto phase = [&](int il) -> Phase {
+      const int p0 = (il - kz + 3) % 3; /* planes p0 and p0+3 (if below 5) have this ilayer */
+      const bool on = lane < 10 && p0 + 3 * (lane & 1) < 5;
+      const int rt = on ? (p0 + 3 * (lane & 1)) * 5 + (lane >> 1) : 0;
+      Phase h;
+      h.nrow = on ? S.pre[rt][5] : 0;
+      h.sB = i2 ? S.pre[rt][1] : 0;
+      h.dA = S.start[rt][0];
+      h.dB = S.start[rt][1] - S.pre[rt][1];
+      const int nbr = (h.nrow + 63) >> 6;
+      h.bsc = wave_incl_scan(nbr);
+      h.rb = h.bsc - nbr;
+      h.nb = rl_i(h.bsc, 63); /* batches of 64 */
+      if (lane < 10) S.rb[il & 1][lane] = h.rb;
+      return h;
+    };
+    W raw[NB];
+    /* batches q0.. of the phase's rows, in flight */
+    auto fetch = [&](const Phase &h, int q0) {
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        raw[q] = 0;
+        if (q0 + q < h.nb) {
+          const int tr = __popcll(__ballot(lane < 10 && h.bsc <= q0 + q)); /* its row */
+          const int l = 64 * (q0 + q - rl_i(h.rb, tr)) + lane, n = rl_i(h.nrow, tr);
+          int64_t p = rl_i64(h.dA, tr);
+          if (i2) {
+            const int64_t pb = rl_i64(h.dB, tr);
+            if (l >= rl_i(h.sB, tr)) p = pb;
+          }
+          if (l < n) raw[q] = cd_load<IX>(xb8 + (p + l) * PB);
+        }
+      }
+    };
+    int il = 0, q0 = 0;
+    Phase h = phase(0);
+    fetch(h, 0);
+#pragma unroll 1
+    while (il < 3) {
+      wave_lds_sync(); /* the reads of word and top are done */
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        if (q0 + q < h.nb) {
+          const uint64_t t0 = __ballot((fd_code<IX>(raw[q], 0) >> sh) == 3u), t1 = __ballot((fd_code<IX>(raw[q], 1) >> sh) == 3u),
+                         t2 = __ballot((fd_code<IX>(raw[q], 2) >> sh) == 3u);
+          S.word[q * 64 + lane] = raw[q];
+          if (lane < 3) S.top[q][lane] = lane == 0 ? t0 : (lane == 1 ? t1 : t2);
+        }
+      }
+      wave_lds_sync();
+      /* the next batches, or the next phase's first, fly during the sums */
+      const int ci = il, c0 = q0;
+      q0 += NB;
+      if (q0 >= h.nb) {
+        q0 = 0;
+        if (++il < 3) h = phase(il);
+      }
+      if (il < 3) fetch(h, q0);
+      const int p0 = (ci - kz + 3) % 3;
+      /* this lane's plane: the one of zi (the cells below it), zi+1 (its own) that is p0 mod 3, or none */
+      const int pl = zi % 3 == p0 ? zi : ((zi + 1) % 3 == p0 ? zi + 1 : -1);
+      const bool zbelow = pl == zi;
+      if (pl >= 0 && live) {
+#pragma unroll 1
+        for (int j = 0; j < 2; ++j) { /* rows y-1, y */
+          const int r = pl * 5 + yi + j, rb = S.rb[ci & 1][2 * (yi + j) + (pl >= 3 ? 1 : 0)] - c0;
+          const int pA = S.pre[r][xi], pB = S.pre[r][xi + 1], pC = S.pre[r][xi + 2];
+          for (int bb = max(pA >> 6, -rb); bb * 64 < pC && rb + bb < NB; ++bb) {
+            const int q = rb + bb, o = 64 * bb;
+            const uint64_t fB = bits_below(pB - o);
+            uint64_t m = bits_below(pC - o) & ~bits_below(pA - o) & (S.top[q][0] | ~fB);
+            if (j == 0) m &= S.top[q][1];
+            if (zbelow) m &= S.top[q][2];
+            const W *wd = S.word + q * 64;
+            if (!m) continue;
+            int i = __builtin_ctzll(m);
+            W wn = wd[i];
+            while (m) {
+              const W w = wn;
+              const bool xbelow = o + i < pB;
+              m &= m - 1ull;
+              i = m ? __builtin_ctzll(m) : 0;
+              wn = wd[i]; /* the next hit's codes are on their way */
+              int bx, by, bz;
+              float wx[2], wy[2], wz[2];
+              fd_axis<IX, EX>(fd_code<IX>(w, 0), xbelow, m0[0] + xi + (xbelow ? 0 : 1), m0[0] + xi + 1, bx, wx[0], wx[1]);
+              fd_axis<IX, EX>(fd_code<IX>(w, 1), j == 0, m0[1] + yi + j, m0[1] + yi + 1, by, wy[0], wy[1]);
+              fd_axis<IX, EX>(fd_code<IX>(w, 2), zbelow, m0[2] + pl, m0[2] + zi + 1, bz, wz[0], wz[1]);
+              float *a0 = acc + 64 * ((bz * 4 + by) * 4 + bx);
+              float v[8];
+#pragma unroll
+              for (int k = 0; k < 8; ++k) v[k] = a0[64 * ((k >> 2) * 16 + ((k >> 1) & 1) * 4 + (k & 1))];
+#pragma unroll
+              for (int k = 0; k < 8; ++k) v[k] = v[k] + wx[k & 1] * wy[(k >> 1) & 1] * wz[k >> 2] * mass;
+#pragma unroll
+              for (int k = 0; k < 8; ++k) a0[64 * ((k >> 2) * 16 + ((k >> 1) & 1) * 4 + (k & 1))] = v[k];
+            }
+          }
+        }
+      }
+    }
+    const double t = fd_store(S.acc, lane, live, T[0] * nt + m0[0] + xi, T[1] * nt + m0[1] + yi, T[2] * nt + m0[2] + zi,
+                              4 * g.nc, rho);
+    if (lane == 0) bsum[b] = t;
+  }
+}
+
+/*
+ * The crowded cells of the listed blocks, sixteen waves a block: a wave takes
+ * one of its cells at a time, lane f owning fine cell f = (z*4+y)*4+x, and
+ * goes through the cell's 4 source rows (two cells of a row follow one another
+ * in order) 64 particles at a time.  Ballots over the particles' sub-cells on
+ * each axis give every lane the mask of the particles that reach its fine
+ * cell, and it adds those alone, in order, four weight reads in flight.
+ */
+#define FDH_W 16 /* waves per block */
+template <int IX, bool EX>
+__global__ __launch_bounds__(64 * FDH_W) void k_fine_deposit_heavy(const typename IntOf<IX>::T *__restrict__ xp,
+                                                                   const int32_t *__restrict__ rhoc,
+                                                                   const int64_t *__restrict__ cstart, Geo g, float mass,
+                                                                   float *__restrict__ rho, double *__restrict__ bsum,
+                                                                   const int32_t *__restrict__ hlist,
+                                                                   const uint64_t *__restrict__ hmask,
+                                                                   const unsigned long long *__restrict__ hcount) {
+  typedef typename CdWord<IX>::T W;
+  constexpr int PB = 3 * IX, sh = IX == 1 ? 6 : 14;
+  __shared__ double hsum[64];
+  __shared__ float wts[FDH_W][3][64]; /* per wave: d1 of the 64 particles at hand, per axis */
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const char *xb8 = reinterpret_cast<const char *>(xp);
+  const int nt = g.nt, nbt = (nt + 3) / 4;
+  const int64_t nf = 4 * (int64_t)g.nc;
+  const int fx = lane & 3, fy = (lane >> 2) & 3, fz = lane >> 4;
+  const int nh = (int)*hcount;
+  for (int h = blockIdx.x; h < nh; h += gridDim.x) {
+    const int b = hlist[h];
+    const uint64_t cells = hmask[b];
+    int T[3], m0[3];
+    blk4(b, g, nbt, T, m0);
+    int nth = 0;
+    for (uint64_t rest = cells; rest; rest &= rest - 1ull, ++nth) {
+      if (nth % FDH_W != wv) continue;
+      const int L = __builtin_ctzll(rest);
+      const int C[3] = {m0[0] + (L & 3), m0[1] + ((L >> 2) & 3), m0[2] + (L >> 4)}; /* 0-based */
+      float sacc = 0.f;
+      /* the source rows in order: the two z planes by ilayer, y-1 then y */
+      const int ka = (C[2] - 2 + g.ncb + 3) % 3; /* ilayer of plane C-1 (k = C, 1-based) */
+      /* lane 2r+i < 8: source cell i (x-1, x) of row r */
+      int n8 = 0;
+      int64_t s8 = 0;
+      if (lane < 8) {
+        const int i = lane & 1, y = (lane >> 1) & 1, zz = lane >> 2;
+        const int oz = ka == 2 ? 1 - zz : zz; /* (2, 0): the upper plane first */
+        const int64_t cc = cid_global(g, T[0] * nt + C[0] - 1 + i, T[1] * nt + C[1] - 1 + y, T[2] * nt + C[2] - 1 + oz);
+        n8 = rhoc[cc];
+        s8 = cstart[cc];
+      }
+#pragma unroll 1
+      for (int r = 0; r < 4; ++r) {
+        const int y = r & 1, oz = ka == 2 ? 1 - (r >> 1) : r >> 1;
+        const int n0 = rl_i(n8, 2 * r), nn = n0 + rl_i(n8, 2 * r + 1);
+        const int64_t s0 = rl_i64(s8, 2 * r), s1 = rl_i64(s8, 2 * r + 1) - n0;
+        W next = 0;
+        if (lane < nn) next = cd_load<IX>(xb8 + ((lane < n0 ? s0 : s1) + lane) * PB);
+        for (int o = 0; o < nn; o += 64) {
+          const W w = next;
+          const int l = o + lane;
+          if (l + 64 < nn) next = cd_load<IX>(xb8 + ((l + 64 < n0 ? s0 : s1) + l + 64) * PB);
+          const bool xbelow = l < n0;
+          const uint32_t u[3] = {fd_code<IX>(w, 0), fd_code<IX>(w, 1), fd_code<IX>(w, 2)};
+          const bool below[3] = {xbelow, y == 0, oz == 0};
+          bool pass = l < nn;
+          int rr[3]; /* plane of corner 1 in the cell's frame, -1..4 */
+          float d1[3];
+#pragma unroll
+          for (int a = 0; a < 3; ++a) {
+            pass = pass && (!below[a] || (u[a] >> sh) == 3u);
+            if constexpr (EX) {
+              constexpr float s = 1.0f / (float)(1 << sh);
+              d1[a] = fmaf((float)(u[a] & ((1u << sh) - 1u)), -s, 1.0f - 0.5f * s);
+              rr[a] = below[a] ? -1 : (int)(u[a] >> sh);
+            } else {
+              const int ci = C[a] + (below[a] ? 0 : 1);
+              const float tempx = (float)(4 * (ci - 1)) + ((float)u[a] + 0.5f) * (IX == 1 ? 0x1p-6f : 0x1p-14f);
+              const int i1 = (int)floorf(tempx) + 1;
+              d1[a] = (float)i1 - tempx;
+              rr[a] = i1 - 4 * C[a] - 1;
+            }
+          }
+          wave_lds_sync(); /* the last batch's weights are read */
+#pragma unroll
+          for (int a = 0; a < 3; ++a) wts[wv][a][lane] = d1[a];
+          wave_lds_sync();
+          /* particles whose corner 1 is this lane's plane (at), or the one below it (lo) */
+          uint64_t at[3], lo[3];
+#pragma unroll
+          for (int a = 0; a < 3; ++a) {
+            const int f = a == 0 ? fx : (a == 1 ? fy : fz);
+            uint64_t k[5];
+#pragma unroll
+            for (int q = 0; q < 5; ++q) k[q] = __ballot(rr[a] == q - 1);
+            at[a] = f == 0 ? k[1] : (f == 1 ? k[2] : (f == 2 ? k[3] : k[4]));
+            lo[a] = f == 0 ? k[0] : (f == 1 ? k[1] : (f == 2 ? k[2] : k[3]));
+          }
+          uint64_t m = __ballot(pass) & (at[0] | lo[0]) & (at[1] | lo[1]) & (at[2] | lo[2]);
+          while (m) {
+            float e[4][3];
+            uint64_t bit[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const int i = m ? __builtin_ctzll(m) : 0;
+              bit[k] = m & (0ull - m); /* 0: no particle left */
+              m &= ~bit[k];
+#pragma unroll
+              for (int a = 0; a < 3; ++a) e[k][a] = wts[wv][a][i];
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const float wx = at[0] & bit[k] ? e[k][0] : 1.0f - e[k][0], wy = at[1] & bit[k] ? e[k][1] : 1.0f - e[k][1],
+                          wz = at[2] & bit[k] ? e[k][2] : 1.0f - e[k][2];
+              const float s = sacc + wx * wy * wz * mass;
+              sacc = bit[k] ? s : sacc;
+            }
+          }
+        }
+      }
+      rho[((4 * (int64_t)(T[2] * nt + C[2]) + fz) * nf + 4 * (T[1] * nt + C[1]) + fy) * nf + 4 * (T[0] * nt + C[0]) + fx] = sacc;
+      double t = (double)sacc;
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+      if (lane == 0) hsum[L] = t;
+    }
+    __syncthreads();
+    if (wv == 0) {
+      double t = (cells >> lane) & 1ull ? hsum[lane] : 0.0;
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+      if (lane == 0) bsum[b] += t;
+    }
+    __syncthreads();
+  }
+}
+/* sum of the blocks' sums in a fixed order, whichever kernel formed them; the
+   list goes back to empty */
+__global__ __launch_bounds__(1024) void k_sum_blocks(const double *__restrict__ bsum, int nb, double *out,
+                                                     unsigned long long *hcount) {
+  __shared__ double r[1024];
+  const int t = threadIdx.x;
+  double s = 0;
+#pragma unroll 8
+  for (int b = t; b < nb; b += 1024) s += bsum[b];
+  r[t] = s;
+  __syncthreads();
+  for (int o = 512; o > 0; o >>= 1) {
+    if (t < o) r[t] += r[t + o];
+    __syncthreads();
+  }
+  if (t == 0) {
+    *out = r[0];
+    *hcount = 0ull;
+  }
+}
+
 #define DEP_BLOCKS 2048
-template <int IX> static int fine_dep(cube_ctx *c, float mass, double *t) {
-  /* a coarse cell whose 8 source cells hold more particles than this is
-     formed by its lane's whole wave (CUBE_FD_HEAVY) */
-  int heavy_at = 512;
+#define FD_GRID 16384
+template <int IX, bool EX> static int fine_dep(cube_ctx *c, float mass, double *t) {
+  /* a coarse cell whose 8 source cells hold more particles than this is formed
+     by a wave of its own (CUBE_FD_HEAVY): a lane's hit costs its wave some 60
+     instructions, a wave's pass over 64 candidates about 150 and the cell's 4
+     rows as many each.  96 / 160 / 256 measured 2.02 / 1.36 / 1.16 ms on 128^3
+     at z = 3, 0.120 / 0.105 / 0.099 ms on 48^3, 0.76 / 0.81 / 0.83 ms on the
+     clustered 128^3 with 1-byte codes */
+  int heavy_at = 256;
   if (const char *e = getenv("CUBE_FD_HEAVY"); e && *e) heavy_at = std::max(0, atoi(e));
-  hipLaunchKernelGGL(k_fine_deposit_cc<IX>, dim3(DEP_BLOCKS), dim3(FD_T), 0, c->stream,
-                     (const typename IntOf<IX>::T *)c->xp, c->rhoc, c->cstart, geo_of(c), mass, c->rho_f, c->dred,
-                     heavy_at);
+  const int64_t nbt = (c->nt + 3) / 4, nblk = nbt * nbt * nbt * c->ntiles;
+  const typename IntOf<IX>::T *xp = (const typename IntOf<IX>::T *)c->xp;
+  unsigned long long *hcount = (unsigned long long *)c->ured + CUBE_URED_FDHEAVY;
+  hipLaunchKernelGGL((k_fine_deposit<IX, EX>), dim3((unsigned)std::min<int64_t>(nblk, FD_GRID)), dim3(64), 0, c->stream,
+                     xp, c->rhoc, c->cstart, geo_of(c), mass, c->rho_f, c->fdsum, (int)nblk, heavy_at, c->fdlist,
+                     c->fdmask, hcount);
   CUBE_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_sum_parts1, dim3(1), dim3(64), 0, c->stream, c->dred, DEP_BLOCKS,
-                     c->dred + CUBE_DRED_FINE_SUM);
+  /* a fixed grid: the count stays on the device */
+  hipLaunchKernelGGL((k_fine_deposit_heavy<IX, EX>), dim3((unsigned)std::min<int64_t>(nblk, 512)), dim3(64 * FDH_W), 0, c->stream,
+                     xp, c->rhoc, c->cstart, geo_of(c), mass, c->rho_f, c->fdsum, c->fdlist, c->fdmask,
+                     hcount);
+  CUBE_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_sum_blocks, dim3(1), dim3(1024), 0, c->stream, c->fdsum, (int)nblk, c->dred + CUBE_DRED_FINE_SUM,
+                     hcount);
   CUBE_LAUNCH_CHECK();
   if (t) {
     CUBE_CHECK(hipMemcpyAsync(t, c->dred + CUBE_DRED_FINE_SUM, sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -755,7 +937,10 @@ template <int IX> static int fine_dep(cube_ctx *c, float mass, double *t) {
   return CUBE_OK;
 }
 int cube_fine_deposit(cube_ctx *c, float mass_p, double *testrhof) {
-  return c->p.izipx == 1 ? fine_dep<1>(c, mass_p, testrhof) : fine_dep<2>(c, mass_p, testrhof);
+  if (c->p.izipx == 1) return fine_dep<1, true>(c, mass_p, testrhof);
+  /* 2-byte codes: 4*(i-1) + (u+0.5)*2^-14 needs 15 fraction bits, exact in
+     real(4) below 512, and the coordinate reaches 4 nt */
+  return c->nt <= 128 ? fine_dep<2, true>(c, mass_p, testrhof) : fine_dep<2, false>(c, mass_p, testrhof);
 }
 template <int IX, bool EX> static int coarse_dep(cube_ctx *c, float mass, double *t) {
   /* partial sums in the upper half of dred, apart from the fine deposit's,

@@ -63,7 +63,7 @@ static void free_all(cube_ctx *c) {
                   c->cstart, c->cstart2, c->dest, c->key, c->sortbuf, c->fill, c->xdest, c->xkey, c->rank, c->xrank, c->fbflag,
                   c->tanf_tab, c->venc_tab, c->vdec0, c->vdec1, c->rho_f, c->spec_f, c->specd_f, c->force_f,
                   c->kern_f, c->rho_c, c->spec_c, c->specd_c, c->force_c, c->kern_c, c->dred,
-                  c->ured, c->fdsum, c->fdlist, c->fdmask, c->ired, c->scanbuf, c->vpart, c->slots, c->ppdefer, c->ppitems};
+                  c->ured, c->fdsum, c->fdheavy, c->fdlist, c->fdmask, c->ired, c->scanbuf, c->vpart, c->slots, c->ppdefer, c->ppitems};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   cube_fft_destroy(c->plan_f);
@@ -228,7 +228,8 @@ extern "C" int cube_ctx_create(const cube_params *p, cube_ctx **out) {
   st |= dalloc(&c->ured, 64);
   {
     const int64_t nbt = (nt + 3) / 4, nb4 = nbt * nbt * nbt * c->ntiles;
-    st |= dalloc(&c->fdsum, nb4);
+    st |= dalloc(&c->fdsum, nb4 + FDS_W);
+    st |= dalloc(&c->fdheavy, nb4 * FDH_W);
     st |= dalloc(&c->fdlist, nb4);
     st |= dalloc(&c->fdmask, nb4);
   }

@@ -90,7 +90,8 @@ struct cube_ctx {
   double *dred;             /* 8192 doubles: [0,4096) reductions of work on `stream`,
                                [4096,8192) of work on `side` */
   uint64_t *ured;           /* 64 words */
-  double *fdsum;            /* fine deposit: one sum per block of 4^3 coarse cells */
+  double *fdsum;            /* fine deposit: one sum per block of 4^3 coarse cells, then partial ones */
+  double *fdheavy;          /* and FDH_W sums of its crowded cells */
   int32_t *fdlist;          /* and its list of blocks with crowded cells (length in ured) */
   uint64_t *fdmask;         /* those cells, by block */
   int64_t *ired;            /* 4096 */
@@ -326,7 +327,9 @@ int cube_fft_filter3_t(cube_ctx *c, FFTPlan *p, const float *in3, const float *a
 
 int cube_fine_deposit(cube_ctx *c, float mass_p, double *testrhof);
 /* device slots (in dred) of the deposits' mesh sums */
-#define CUBE_URED_FDHEAVY 32 /* word of ured: the fine deposit's crowded blocks */
+#define CUBE_URED_FDHEAVY 32 /* words of ured: the fine deposit's listed blocks, and its sum's finished workgroups */
+#define FDH_W 16             /* waves that share a listed block */
+#define FDS_W 64             /* most workgroups of its sum */
 #define CUBE_DRED_FINE_SUM 4000
 #define CUBE_DRED_COARSE_SUM (4096 + 4000)
 int cube_fine_kick(cube_ctx *c, float a_mid, float dt, float sigma_vi, float sigma_vi_new, int sync);

@@ -482,7 +482,7 @@ __global__ __launch_bounds__(64 * NW, 4) void k_coarse_deposit(const typename In
  * memory with crowded cells handed round its wave: 5.12 -> 3.05 ms on the
  * 256^3 mesh of 512^3 particles, 1.79 -> 1.16 ms on
  * 128^3 at z = 3, 0.117 -> 0.086 ms on 64^3, 0.057 -> 0.045 ms on 16^3, 1.48
- * -> 0.83 ms on the clustered 128^3 at z = 0 with 1-byte codes.
+ * -> 0.68 ms on the clustered 128^3 at z = 0 with 1-byte codes.
  */
 template <int IX> struct FdLds { /* per wave */
   static constexpr int NB = 10; /* batches staged at once: a phase's 10 rows of up to 64 */
@@ -625,13 +625,11 @@ __global__ __launch_bounds__(64) void k_fine_deposit(const typename IntOf<IX>::T
         tot += S.pre[r][xi + 2] - S.pre[r][xi];
       }
       const uint64_t hv = __ballot(live && tot > heavy_at);
-      if (hv) { /* uniform */
-        if (lane == 0) {
-          hmask[b] = hv;
-          hlist[atomicAdd(hcount, 1ull)] = b;
-        }
-        live = live && tot <= heavy_at;
+      if (lane == 0) {
+        hmask[b] = hv;
+        if (hv) hlist[atomicAdd(hcount, 1ull)] = b;
       }
+      live = live && tot <= heavy_at;
     }
 #pragma unroll
     for (int q = 0; q < 16; ++q) reinterpret_cast<float4 *>(S.acc)[q * 64 + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -749,34 +747,34 @@ __global__ __launch_bounds__(64) void k_fine_deposit(const typename IntOf<IX>::T
 }
 
 /*
- * The crowded cells of the listed blocks, sixteen waves a block: a wave takes
- * one of its cells at a time, lane f owning fine cell f = (z*4+y)*4+x, and
+ * The crowded cells of the listed blocks, FDH_W waves a block, each a workgroup
+ * of its own that fits in beside whatever else runs: a wave takes one of its
+ * cells at a time, lane f owning fine cell f = (z*4+y)*4+x, and
  * goes through the cell's 4 source rows (two cells of a row follow one another
  * in order) 64 particles at a time.  Ballots over the particles' sub-cells on
  * each axis give every lane the mask of the particles that reach its fine
  * cell, and it adds those alone, in order, four weight reads in flight.
  */
-#define FDH_W 16 /* waves per block */
 template <int IX, bool EX>
-__global__ __launch_bounds__(64 * FDH_W) void k_fine_deposit_heavy(const typename IntOf<IX>::T *__restrict__ xp,
+__global__ __launch_bounds__(64) void k_fine_deposit_heavy(const typename IntOf<IX>::T *__restrict__ xp,
                                                                    const int32_t *__restrict__ rhoc,
                                                                    const int64_t *__restrict__ cstart, Geo g, float mass,
-                                                                   float *__restrict__ rho, double *__restrict__ bsum,
+                                                                   float *__restrict__ rho, double *__restrict__ hsum,
                                                                    const int32_t *__restrict__ hlist,
                                                                    const uint64_t *__restrict__ hmask,
                                                                    const unsigned long long *__restrict__ hcount) {
   typedef typename CdWord<IX>::T W;
   constexpr int PB = 3 * IX, sh = IX == 1 ? 6 : 14;
-  __shared__ double hsum[64];
-  __shared__ float wts[FDH_W][3][64]; /* per wave: d1 of the 64 particles at hand, per axis */
-  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  __shared__ float wts[3][64]; /* d1 of the 64 particles at hand, per axis */
+  const int lane = threadIdx.x;
   const char *xb8 = reinterpret_cast<const char *>(xp);
   const int nt = g.nt, nbt = (nt + 3) / 4;
   const int64_t nf = 4 * (int64_t)g.nc;
   const int fx = lane & 3, fy = (lane >> 2) & 3, fz = lane >> 4;
-  const int nh = (int)*hcount;
-  for (int h = blockIdx.x; h < nh; h += gridDim.x) {
-    const int b = hlist[h];
+  const int64_t items = (int64_t)*hcount * FDH_W;
+  for (int64_t h = blockIdx.x; h < items; h += gridDim.x) {
+    const int b = hlist[h / FDH_W], wv = (int)(h % FDH_W);
+    double hs = 0;
     const uint64_t cells = hmask[b];
     int T[3], m0[3];
     blk4(b, g, nbt, T, m0);
@@ -832,7 +830,7 @@ __global__ __launch_bounds__(64 * FDH_W) void k_fine_deposit_heavy(const typenam
           }
           wave_lds_sync(); /* the last batch's weights are read */
 #pragma unroll
-          for (int a = 0; a < 3; ++a) wts[wv][a][lane] = d1[a];
+          for (int a = 0; a < 3; ++a) wts[a][lane] = d1[a];
           wave_lds_sync();
           /* particles whose corner 1 is this lane's plane (at), or the one below it (lo) */
           uint64_t at[3], lo[3];
@@ -855,7 +853,7 @@ __global__ __launch_bounds__(64 * FDH_W) void k_fine_deposit_heavy(const typenam
               bit[k] = m & (0ull - m); /* 0: no particle left */
               m &= ~bit[k];
 #pragma unroll
-              for (int a = 0; a < 3; ++a) e[k][a] = wts[wv][a][i];
+              for (int a = 0; a < 3; ++a) e[k][a] = wts[a][i];
             }
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
@@ -871,36 +869,49 @@ __global__ __launch_bounds__(64 * FDH_W) void k_fine_deposit_heavy(const typenam
       double t = (double)sacc;
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
-      if (lane == 0) hsum[L] = t;
+      hs += t;
     }
-    __syncthreads();
-    if (wv == 0) {
-      double t = (cells >> lane) & 1ull ? hsum[lane] : 0.0;
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
-      if (lane == 0) bsum[b] += t;
-    }
-    __syncthreads();
+    if (lane == 0) hsum[(int64_t)b * FDH_W + wv] = hs; /* read if it had a cell */
   }
 }
-/* sum of the blocks' sums in a fixed order, whichever kernel formed them; the
-   list goes back to empty */
-__global__ __launch_bounds__(1024) void k_sum_blocks(const double *__restrict__ bsum, int nb, double *out,
-                                                     unsigned long long *hcount) {
-  __shared__ double r[1024];
+/* sum of the blocks' sums, those of their crowded cells among them, in a fixed
+   order: a workgroup sums its stretch of blocks, the last to finish the
+   workgroups' sums.  The list goes back to empty */
+#define FDS_B 1024 /* blocks a workgroup takes before there is a second */
+__global__ __launch_bounds__(256) void k_sum_blocks(const double *__restrict__ bsum, const uint64_t *__restrict__ hmask,
+                                                    const double *__restrict__ hsum, int nb, int per,
+                                                    double *__restrict__ part, double *__restrict__ out,
+                                                    unsigned long long *__restrict__ hcount) {
+  __shared__ double r[256];
+  __shared__ bool last;
   const int t = threadIdx.x;
+  const int64_t b0 = (int64_t)blockIdx.x * per, b1 = min(b0 + per, (int64_t)nb);
   double s = 0;
-#pragma unroll 8
-  for (int b = t; b < nb; b += 1024) s += bsum[b];
+#pragma unroll 4
+  for (int64_t b = b0 + t; b < b1; b += 256) {
+    s += bsum[b];
+    const int n = min(__popcll(hmask[b]), FDH_W);
+    for (int k = 0; k < n; ++k) s += hsum[b * FDH_W + k];
+  }
   r[t] = s;
   __syncthreads();
-  for (int o = 512; o > 0; o >>= 1) {
+  for (int o = 128; o > 0; o >>= 1) {
     if (t < o) r[t] += r[t + o];
     __syncthreads();
   }
   if (t == 0) {
-    *out = r[0];
-    *hcount = 0ull;
+    __hip_atomic_store(part + blockIdx.x, r[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    last = __hip_atomic_fetch_add(hcount + 1, 1ull, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last || t >= 64) return;
+  s = t < (int)gridDim.x ? __hip_atomic_load(part + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if (t == 0) {
+    *out = s;
+    hcount[0] = 0ull;
+    hcount[1] = 0ull;
   }
 }
 
@@ -922,13 +933,13 @@ template <int IX, bool EX> static int fine_dep(cube_ctx *c, float mass, double *
                      xp, c->rhoc, c->cstart, geo_of(c), mass, c->rho_f, c->fdsum, (int)nblk, heavy_at, c->fdlist,
                      c->fdmask, hcount);
   CUBE_LAUNCH_CHECK();
-  /* a fixed grid: the count stays on the device */
-  hipLaunchKernelGGL((k_fine_deposit_heavy<IX, EX>), dim3((unsigned)std::min<int64_t>(nblk, 512)), dim3(64 * FDH_W), 0, c->stream,
-                     xp, c->rhoc, c->cstart, geo_of(c), mass, c->rho_f, c->fdsum, c->fdlist, c->fdmask,
-                     hcount);
+  /* a fixed grid, four waves a SIMD: the count stays on the device */
+  hipLaunchKernelGGL((k_fine_deposit_heavy<IX, EX>), dim3((unsigned)std::min<int64_t>(nblk * FDH_W, 4096)), dim3(64), 0,
+                     c->stream, xp, c->rhoc, c->cstart, geo_of(c), mass, c->rho_f, c->fdheavy, c->fdlist, c->fdmask, hcount);
   CUBE_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_sum_blocks, dim3(1), dim3(1024), 0, c->stream, c->fdsum, (int)nblk, c->dred + CUBE_DRED_FINE_SUM,
-                     hcount);
+  const int nw = (int)std::min<int64_t>(FDS_W, (nblk + FDS_B - 1) / FDS_B), per = (int)((nblk + nw - 1) / nw);
+  hipLaunchKernelGGL(k_sum_blocks, dim3(nw), dim3(256), 0, c->stream, c->fdsum, c->fdmask, c->fdheavy, (int)nblk, per,
+                     c->fdsum + nblk, c->dred + CUBE_DRED_FINE_SUM, hcount);
   CUBE_LAUNCH_CHECK();
   if (t) {
     CUBE_CHECK(hipMemcpyAsync(t, c->dred + CUBE_DRED_FINE_SUM, sizeof(double), hipMemcpyDeviceToHost, c->stream));

@@ -109,7 +109,7 @@ def stage_bytes(np_, nf3, nc3, bx, bv):
 
 
 MAIN_KERNEL = {
-    "drift": "k_drift_dest+k_place_ranked+k_sort_small+k_drift_final2",
+    "drift": "k_drift_dest+k_place_ranked+k_sort_med+k_drift_final2",
     "pp": "k_pp_blk", "fine_deposit": "k_fine_deposit", "fine_kick": "k_kick<fine>",
     "coarse_deposit": "k_coarse_deposit", "coarse_kick": "k_kick<coarse>",
     "fine_fft": "k_r2c_x+k_c2c_r", "fine_inverse": "k_green_r+k_c2c_r+k_c2r_x3",

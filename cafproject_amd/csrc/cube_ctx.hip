@@ -60,7 +60,7 @@ static void free_all(cube_ctx *c) {
   if (c->scratch_in_force) /* carved out of force_f, not allocations of their own */
     c->dest = c->rank = c->xdest = c->xrank = nullptr, c->key = c->sortbuf = c->xkey = nullptr;
   void *ptrs[] = {c->xp, c->vp, c->xp2, c->vp2, c->pid, c->pid2, c->rhoc, c->rhoc2, c->vfield, c->vfield2,
-                  c->cstart, c->cstart2, c->dest, c->key, c->sortbuf, c->fill, c->xdest, c->xkey, c->rank, c->xrank, c->fbflag,
+                  c->cstart, c->cstart2, c->dest, c->key, c->sortbuf, c->fill, c->xdest, c->xkey, c->rank, c->xrank,
                   c->tanf_tab, c->venc_tab, c->vdec0, c->vdec1, c->rho_f, c->spec_f, c->specd_f, c->force_f,
                   c->kern_f, c->rho_c, c->spec_c, c->specd_c, c->force_c, c->kern_c, c->dred,
                   c->ured, c->fdsum, c->fdheavy, c->fdlist, c->fdmask, c->ired, c->scanbuf, c->vpart, c->slots, c->ppdefer, c->ppitems};
@@ -185,7 +185,6 @@ extern "C" int cube_ctx_create(const cube_params *p, cube_ctx **out) {
   st |= dalloc(&c->fill, c->ncells);
   st |= dalloc(&c->ppdefer, c->ncells / 64 + 1);
   st |= dalloc(&c->ppitems, c->ncells / 64 + 2);
-  st |= dalloc(&c->fbflag, c->ncells / 64 + 2); /* one per 64-cell finalize workgroup of the drift */
   st |= dalloc(&c->tanf_tab, c->nvbin);
   st |= dalloc(&c->venc_tab, c->nvbin / 2);
   st |= dalloc(&c->vdec0, c->nvbin);
@@ -235,7 +234,7 @@ extern "C" int cube_ctx_create(const cube_params *p, cube_ctx **out) {
   }
   if (!st && hipMemset(c->ured, 0, 64 * sizeof(uint64_t)) != hipSuccess) st = CUBE_ERR_HIP;
   st |= dalloc(&c->slots, CUBE_NSLOTREG * CUBE_SLOTS);
-  st |= dalloc(&c->ired, 4096);
+  st |= dalloc(&c->ired, c->ntiles * BOX_WG);
   st |= dalloc(&c->scanbuf, c->ncells / 1024 + 4);
   st |= dalloc(&c->vpart, 3 * (c->ncells / 64 + 2));
   if (st) {
@@ -411,7 +410,7 @@ extern "C" int cube_buffer_grid(cube_ctx *c) {
   CUBE_CHECK(hipSetDevice(c->device));
   int64_t *sums = (int64_t *)malloc(c->ntiles * sizeof(int64_t));
   tbeg(c);
-  int st = cube_tile_boxsum(c, c->rhoc, (int)c->ncb, sums);
+  int st = cube_tile_boxsum(c, (int)c->ncb, sums);
   tend(c, CUBE_T_CHECKS);
   int64_t tot = 0;
   for (int64_t t = 0; t < c->ntiles; ++t) tot += sums[t];
@@ -484,7 +483,7 @@ extern "C" int cube_pp_force(cube_ctx *c, float a_mid, float dt, float sigma_vi,
   /* W/ext_pp_force.f90:41-45: particles of coarse cells 0..nt+1 of a tile */
   int64_t *sums = (int64_t *)malloc(c->ntiles * sizeof(int64_t));
   tbeg(c);
-  int st = cube_tile_boxsum(c, c->rhoc, 1, sums);
+  int st = cube_tile_boxsum(c, 1, sums);
   tend(c, CUBE_T_CHECKS);
   int64_t mx = 0;
   for (int64_t t = 0; t < c->ntiles; ++t) mx = sums[t] > mx ? sums[t] : mx;

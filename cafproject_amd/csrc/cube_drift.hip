@@ -29,6 +29,7 @@
 #include <stdlib.h>
 #include <string.h>
 #include <algorithm>
+#include <vector>
 
 #define DT 256
 static const double WEIGHT_V = (double)0.1f; /* real(8),parameter :: weight_v=0.1 */
@@ -140,20 +141,25 @@ int cube_scan_counts(cube_ctx *c, const int32_t *cnt, int64_t *start, int64_t n,
 }
 
 /* ---------------- per-tile sums over the extended box ---------------- */
-/* out[t] = sum of rhoc over local cells [1-w, nt+w]^3 of tile t (periodic) */
-__global__ void k_tile_boxsum(const int32_t *rhoc, Geo g, int w, unsigned long long *out) {
-  const int t = blockIdx.y;
+/* particles of local cells [1-w, nt+w]^3 of tile t (periodic): a row of the
+   box is a run of cells in each tile it crosses, so its sum is a difference of
+   their starts.  BOX_WG workgroups share a tile's rows, the host adds their
+   sums.  Latency bound: some 10 us with the copy back for any tile, where
+   reading the cells' counts took 28 us on 8 tiles of 16^3 cells (784 rows of
+   28 cells each, w = 6) and 83 us on 8 of 128^3 */
+__global__ __launch_bounds__(256) void k_tile_boxsum(const int64_t *__restrict__ cstart, Geo g, int w,
+                                                     int64_t *__restrict__ out) {
+  const int t = blockIdx.y, nt = g.nt, e = nt + 2 * w;
   const int tz = t / (g.nnt * g.nnt), ty = (t / g.nnt) % g.nnt, tx = t % g.nnt;
-  /* (nt+2w)^3 < 2^31 cells per box: 32-bit index arithmetic; the tile's
-     own cells by their id, the buffer shell through cid_global */
-  const int e = g.nt + 2 * w, nt = g.nt;
-  const uint32_t vol = (uint32_t)e * e * e, ue = (uint32_t)e;
+  const int dn = (w + nt - 1) / nt; /* tiles the box reaches into on a side */
   int64_t s = 0;
-  for (uint32_t q = blockIdx.x * blockDim.x + threadIdx.x; q < vol; q += gridDim.x * blockDim.x) {
-    const uint32_t qe = q / ue;
-    const int i = (int)(q - qe * ue) - w, j = (int)(qe % ue) - w, k = (int)(qe / ue) - w;
-    const bool in = i >= 0 && i < nt && j >= 0 && j < nt && k >= 0 && k < nt;
-    s += rhoc[in ? g.cid(i, j, k, t) : cid_global(g, tx * nt + i, ty * nt + j, tz * nt + k)];
+  for (int q = blockIdx.x * 256 + threadIdx.x; q < e * e; q += BOX_WG * 256) {
+    const int j = q % e - w, k = q / e - w;
+    for (int d = -dn; d <= dn; ++d) { /* its part in tile tx + d: cells [i0, i1) of that tile */
+      const int i0 = max(-w - d * nt, 0), i1 = min(nt + w - d * nt, nt);
+      const int64_t row = cid_global(g, (tx + d) * nt, ty * nt + j, tz * nt + k);
+      s += cstart[row + i1] - cstart[row + i0];
+    }
   }
   __shared__ int64_t r[256];
   r[threadIdx.x] = s;
@@ -162,16 +168,19 @@ __global__ void k_tile_boxsum(const int32_t *rhoc, Geo g, int w, unsigned long l
     if (threadIdx.x < o) r[threadIdx.x] += r[threadIdx.x + o];
     __syncthreads();
   }
-  if (threadIdx.x == 0) atomicAdd(out + t, (unsigned long long)r[0]);
+  if (threadIdx.x == 0) out[t * BOX_WG + blockIdx.x] = r[0];
 }
-int cube_tile_boxsum(cube_ctx *c, const int32_t *rhoc, int w, int64_t *host_out) {
-  int st = fill_i64(c, c->ired, c->ntiles, 0);
-  if (st) return st;
-  hipLaunchKernelGGL(k_tile_boxsum, dim3(256, (unsigned)c->ntiles), dim3(256), 0, c->stream, rhoc, geo_of(c), w,
-                     (unsigned long long *)c->ired);
+int cube_tile_boxsum(cube_ctx *c, int w, int64_t *host_out) {
+  hipLaunchKernelGGL(k_tile_boxsum, dim3(BOX_WG, (unsigned)c->ntiles), dim3(256), 0, c->stream, c->cstart, geo_of(c), w,
+                     c->ired);
   CUBE_LAUNCH_CHECK();
-  CUBE_CHECK(hipMemcpyAsync(host_out, c->ired, c->ntiles * sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
+  std::vector<int64_t> part(c->ntiles * BOX_WG);
+  CUBE_CHECK(hipMemcpyAsync(part.data(), c->ired, part.size() * sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
   CUBE_CHECK(hipStreamSynchronize(c->stream));
+  for (int64_t t = 0; t < c->ntiles; ++t) {
+    host_out[t] = 0;
+    for (int b = 0; b < BOX_WG; ++b) host_out[t] += part[t * BOX_WG + b];
+  }
   return CUBE_OK;
 }
 
@@ -339,85 +348,112 @@ __global__ __launch_bounds__(DT) void k_drift_dest(const typename IntOf<IX>::T *
   }
 }
 
-/* ---------------- placement ---------------- */
-__global__ void k_place(const int32_t *__restrict__ dest, const uint64_t *__restrict__ key, int64_t n,
-                        const int64_t *__restrict__ start, int32_t *__restrict__ fill, uint64_t *__restrict__ out) {
-  for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < n; p += (int64_t)gridDim.x * blockDim.x) {
-    const int32_t d = dest[p];
-    if (d < 0) continue;
-    const int32_t s = atomicAdd(fill + d, 1);
-    out[start[d] + s] = key[p];
-  }
+/* ---------------- per-cell sort ---------------- */
+#define MED_SORT 1024
+#define BIG_SORT 16384
+#define FB_CELLS 64      /* cells per finalize workgroup (the context sizes vpart for it) */
+/* slots staged in LDS at once: 640 (10 per cell against the 8 of an average
+   cell) keeps the finalize workgroup at ~22 KB of LDS, 7 per CU; a workgroup
+   with more goes through its cells in runs of at most that many */
+#define FB_CH 640
+#define FB_LDS_SORT 64   /* largest cell whose keys are ranked there */
+/* cells above FB_LDS_SORT, for the sorts of their own: big ones (above
+   MED_SORT) from the front of the list, counted in counters[3], the others
+   from its back, counted in counters[4] */
+__device__ __forceinline__ void list_cell(int64_t c, int n, int64_t ncells, int32_t *__restrict__ list,
+                                          unsigned long long *__restrict__ counters) {
+  if (n > MED_SORT)
+    list[atomicAdd(counters + 3, 1ull)] = (int32_t)c;
+  else if (n > FB_LDS_SORT)
+    list[ncells - 1 - (int64_t)atomicAdd(counters + 4, 1ull)] = (int32_t)c;
 }
-
-/* scatter to the slot taken at counting time: no second round of atomics */
-__global__ void k_place_ranked(const int32_t *__restrict__ dest, const int32_t *__restrict__ rank,
-                               const uint64_t *__restrict__ key, int64_t n, const int64_t *__restrict__ start,
-                               uint64_t *__restrict__ out) {
-  for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < n; p += (int64_t)gridDim.x * blockDim.x) {
+/* scatter to the slot taken at counting time: no second round of atomics; and
+   (cnt given) the list of the cells that the finalize pass does not sort */
+__global__ __launch_bounds__(256) void k_place_ranked(const int32_t *__restrict__ dest, const int32_t *__restrict__ rank,
+                                                      const uint64_t *__restrict__ key, int64_t n,
+                                                      const int64_t *__restrict__ start, uint64_t *__restrict__ out,
+                                                      const int32_t *__restrict__ cnt, int64_t ncells,
+                                                      int32_t *__restrict__ list,
+                                                      unsigned long long *__restrict__ counters) {
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, nthr = (int64_t)gridDim.x * blockDim.x;
+  if (cnt)
+    for (int64_t c = t; c < ncells; c += nthr) list_cell(c, cnt[c], ncells, list, counters);
+  for (int64_t p = t; p < n; p += nthr) {
     const int32_t d = dest[p];
     if (d < 0) continue;
     out[start[d] + rank[p]] = key[p];
   }
 }
-
-/* ---------------- per-cell sort ---------------- */
-#define SMALL_SORT 48
-#define MED_SORT 1024
-#define BIG_SORT 16384
-#define FB_CELLS 64      /* cells per finalize workgroup (the context sizes fbflag/vpart for it) */
-/* slots staged in LDS per finalize pass: 640 (10 per cell against the 8 of
-   an average cell) keeps the workgroup at ~22 KB of LDS, 7 per CU; a block
-   with more slots takes the chunked path with the global key sort */
-#define FB_CH 640
-#define FB_LDS_SORT 64   /* largest cell sorted inside the finalize workgroup */
-/* flag[b] = 1 when finalize block b (cells b*FB_CELLS...) holds at most FB_CH
-   particles and no cell above FB_LDS_SORT: it sorts its cells in LDS */
-__global__ void k_fb_flags(const int32_t *__restrict__ cnt, const int64_t *__restrict__ start, int64_t ncells,
-                           uint8_t *__restrict__ flag) {
-  const int64_t b = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  const int64_t c0 = b * FB_CELLS;
-  if (c0 >= ncells) return;
-  const int64_t c1 = min(c0 + FB_CELLS, ncells);
-  int mx = 0;
-  for (int64_t c = c0; c < c1; ++c) mx = max(mx, (int)cnt[c]);
-  flag[b] = (start[c1] - start[c0] <= FB_CH && mx <= FB_LDS_SORT) ? 1 : 0;
+/* cells c_lo.. of a workgroup's ncl whose slots fit in FB_CH, at least one
+   (the same in every wave); returns the cell past them */
+__device__ __forceinline__ int seg_end(const int64_t *cst, int ncl, int c_lo) {
+  const int c = c_lo + 1 + (int)(threadIdx.x & 63);
+  return c_lo + max(1, (int)__popcll(__ballot(c <= ncl && cst[min(c, ncl)] - cst[c_lo] <= FB_CH)));
 }
-__global__ void k_sort_small(const int32_t *__restrict__ cnt, const int64_t *__restrict__ start, int64_t ncells,
-                             uint64_t *__restrict__ a, int32_t *__restrict__ biglist,
-                             unsigned long long *__restrict__ counters, const uint8_t *__restrict__ skip) {
-  const int64_t cidx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (cidx >= ncells) return;
-  if (skip && skip[cidx / FB_CELLS]) return; /* sorted by its finalize workgroup */
-  const int n = cnt[cidx];
-  if (n <= 1) return;
-  if (n > MED_SORT) { /* big cells from the front of the list */
-    const unsigned long long q = atomicAdd(counters + 3, 1ull);
-    biglist[q] = (int32_t)cidx;
-    return;
+/* The keys of cells [c_lo, c_hi), which fit, into pix in order, with their
+   cells in lcell.  A key's place in its cell is the number of smaller keys
+   there (unique: they carry the particle index): every lane ranks its own
+   slots at once instead of one lane per cell sorting serially.  Cells above
+   FB_LDS_SORT come sorted (or, in k_sort_cells, are left to be). */
+__device__ __forceinline__ void seg_sort(const uint64_t *__restrict__ keys, const int64_t *cst, int c_lo, int c_hi,
+                                         uint64_t *pix, uint8_t *lcell) {
+  const int tid = threadIdx.x;
+  const int64_t s0 = cst[c_lo];
+  const int n = (int)(cst[c_hi] - s0);
+  for (int q = tid; q < n; q += 256) pix[q] = keys[s0 + q];
+  if (c_lo + tid < c_hi) {
+    const int lo = (int)(cst[c_lo + tid] - s0), hi = (int)(cst[c_lo + tid + 1] - s0);
+    for (int q = lo; q < hi; ++q) lcell[q] = (uint8_t)(c_lo + tid);
   }
-  if (n > SMALL_SORT) { /* medium cells from the back */
-    const unsigned long long q = atomicAdd(counters + 4, 1ull);
-    biglist[ncells - 1 - (int64_t)q] = (int32_t)cidx;
-    return;
-  }
-  uint64_t v[SMALL_SORT];
-  uint64_t *s = a + start[cidx];
-  for (int q = 0; q < SMALL_SORT; ++q)
-    if (q < n) v[q] = s[q];
-  /* insertion sort in registers (n <= 48) */
-  for (int q = 1; q < SMALL_SORT; ++q) {
-    if (q >= n) break;
-    const uint64_t x = v[q];
-    int r = q - 1;
-    while (r >= 0 && v[r] > x) {
-      v[r + 1] = v[r];
-      --r;
+  __syncthreads();
+  constexpr int PER = (FB_CH + 255) / 256;
+  uint64_t kx[PER];
+  int dst[PER];
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int q = tid + 256 * u;
+    dst[u] = -1;
+    if (q < n) {
+      const int c = lcell[q], lo = (int)(cst[c] - s0), hi = (int)(cst[c + 1] - s0);
+      if (hi - lo <= FB_LDS_SORT) {
+        const uint64_t x = pix[q];
+        int r = 0;
+        for (int w = lo; w < hi; ++w) r += pix[w] < x ? 1 : 0;
+        kx[u] = x;
+        dst[u] = lo + r;
+      }
     }
-    v[r + 1] = x;
   }
-  for (int q = 0; q < SMALL_SORT; ++q)
-    if (q < n) s[q] = v[q];
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < PER; ++u)
+    if (dst[u] >= 0) pix[dst[u]] = kx[u];
+  __syncthreads();
+}
+/* the keys of every cell up to FB_LDS_SORT in order, the others listed */
+__global__ __launch_bounds__(256) void k_sort_cells(const int32_t *__restrict__ cnt, const int64_t *__restrict__ start,
+                                                    int64_t ncells, uint64_t *__restrict__ keys, int32_t *__restrict__ list,
+                                                    unsigned long long *__restrict__ counters) {
+  __shared__ int64_t cst[FB_CELLS + 1];
+  __shared__ uint64_t pix[FB_CH];
+  __shared__ uint8_t lcell[FB_CH];
+  const int tid = threadIdx.x;
+  const int64_t c0 = (int64_t)blockIdx.x * FB_CELLS;
+  const int ncl = (int)min((int64_t)FB_CELLS, ncells - c0);
+  for (int i = tid; i <= ncl; i += 256) cst[i] = start[c0 + i];
+  if (tid < ncl) list_cell(c0 + tid, cnt[c0 + tid], ncells, list, counters);
+  __syncthreads();
+  for (int c_lo = 0; c_lo < ncl;) {
+    const int c_hi = seg_end(cst, ncl, c_lo);
+    const int64_t s0 = cst[c_lo];
+    const int n = (int)min(cst[c_hi] - s0, (int64_t)FB_CH + 1);
+    if (n <= FB_CH) { /* uniform; else one crowded cell */
+      seg_sort(keys, cst, c_lo, c_hi, pix, lcell);
+      for (int q = tid; q < n; q += 256) keys[s0 + q] = pix[q];
+      __syncthreads();
+    }
+    c_lo = c_hi;
+  }
 }
 
 /* bitonic sort of sk[0..m) in LDS, m a power of two */
@@ -448,49 +484,54 @@ __device__ static int lower_bound_u64(const uint64_t *r, int n, uint64_t x) {
   return lo;
 }
 
-/* One wave per medium cell (SMALL_SORT < n <= MED_SORT), four per
-   workgroup: a bitonic sort of the cell's keys (padded to a power of two,
+/* One wave per medium cell (FB_LDS_SORT < n <= MED_SORT), four per
+   workgroup, on a fixed grid (the count stays on the device): a bitonic sort of the cell's keys (padded to a power of two,
    at least 64) in the wave's 8 KB of LDS, the stages ordered by the wave
    itself -- no workgroup barriers, and 32 KB per workgroup so that five
    share a CU where a big cell's workgroup takes 128 KB. */
 __global__ __launch_bounds__(256) void k_sort_med(const int32_t *__restrict__ cnt, const int64_t *__restrict__ start,
-                                                  const int32_t *__restrict__ list, int64_t nlist,
+                                                  const int32_t *__restrict__ list, int64_t ncells,
+                                                  const unsigned long long *__restrict__ counters,
                                                   uint64_t *__restrict__ a) {
   __shared__ uint64_t sm[4 * MED_SORT];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int64_t i = (int64_t)blockIdx.x * 4 + wv;
-  if (i >= nlist) return; /* the whole wave */
   uint64_t *sk = sm + wv * MED_SORT;
-  const int32_t cidx = list[i];
-  const int n = cnt[cidx];
-  uint64_t *s = a + start[cidx];
-  int m = 64;
-  while (m < n) m <<= 1;
-  for (int q = lane; q < m; q += 64) sk[q] = q < n ? s[q] : ~0ull;
-  for (int size = 2; size <= m; size <<= 1)
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      for (int q = lane; q < m; q += 64) { /* each pair (q, q^stride) has one owner */
-        const int o = q ^ stride;
-        if (o > q) {
-          const bool up = (q & size) == 0;
-          const uint64_t x = sk[q], y = sk[o];
-          if ((x > y) == up) {
-            sk[q] = y;
-            sk[o] = x;
+  const int64_t nlist = (int64_t)counters[4];
+  for (int64_t i = (int64_t)blockIdx.x * 4 + wv; i < nlist; i += (int64_t)gridDim.x * 4) {
+    const int32_t cidx = list[ncells - 1 - i];
+    const int n = cnt[cidx];
+    uint64_t *s = a + start[cidx];
+    int m = 64;
+    while (m < n) m <<= 1;
+    for (int q = lane; q < m; q += 64) sk[q] = q < n ? s[q] : ~0ull;
+    for (int size = 2; size <= m; size <<= 1)
+      for (int stride = size >> 1; stride > 0; stride >>= 1) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        for (int q = lane; q < m; q += 64) { /* each pair (q, q^stride) has one owner */
+          const int o = q ^ stride;
+          if (o > q) {
+            const bool up = (q & size) == 0;
+            const uint64_t x = sk[q], y = sk[o];
+            if ((x > y) == up) {
+              sk[q] = y;
+              sk[o] = x;
+            }
           }
         }
       }
-    }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  for (int q = lane; q < n; q += 64) s[q] = sk[q];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (int q = lane; q < n; q += 64) s[q] = sk[q];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); /* the next cell's keys overwrite these */
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
 }
 
-/* One workgroup per big cell.  Up to BIG_SORT keys: a bitonic sort in LDS.
+/* One workgroup per big cell at a time, on a fixed grid.  Up to BIG_SORT keys: a bitonic sort in LDS.
    Larger cells (a collapsed halo core can hold more particles than LDS
    takes): BIG_SORT-key runs sorted in LDS, then pairwise merges of runs in
    global memory between the cell's segment and the same range of tmp (the
@@ -499,58 +540,71 @@ __global__ __launch_bounds__(256) void k_sort_med(const int32_t *__restrict__ cn
    index in its run plus its rank in the other run. */
 __global__ __launch_bounds__(1024) void k_sort_big(const int32_t *__restrict__ cnt,
                                                    const int64_t *__restrict__ start,
-                                                   const int32_t *__restrict__ biglist, uint64_t *__restrict__ a,
-                                                   uint64_t *__restrict__ tmp) {
+                                                   const int32_t *__restrict__ biglist,
+                                                   const unsigned long long *__restrict__ counters,
+                                                   uint64_t *__restrict__ a, uint64_t *__restrict__ tmp) {
   extern __shared__ uint64_t sk[];
-  const int32_t cidx = biglist[blockIdx.x];
-  const int n = cnt[cidx];
-  uint64_t *s = a + start[cidx];
-  if (n <= BIG_SORT) {
-    int m = 1;
-    while (m < n) m <<= 1;
-    for (int q = threadIdx.x; q < m; q += blockDim.x) sk[q] = q < n ? s[q] : ~0ull;
-    __syncthreads();
-    lds_bitonic(sk, m);
-    for (int q = threadIdx.x; q < n; q += blockDim.x) s[q] = sk[q];
-    return;
-  }
-  for (int c0 = 0; c0 < n; c0 += BIG_SORT) {
-    const int len = min(BIG_SORT, n - c0);
-    for (int q = threadIdx.x; q < BIG_SORT; q += blockDim.x) sk[q] = q < len ? s[c0 + q] : ~0ull;
-    __syncthreads();
-    lds_bitonic(sk, BIG_SORT);
-    for (int q = threadIdx.x; q < len; q += blockDim.x) s[c0 + q] = sk[q];
-    __syncthreads();
-  }
-  uint64_t *src = s, *dst = tmp + start[cidx];
-  for (int w = BIG_SORT; w < n; w <<= 1) {
-    for (int lo = 0; lo < n; lo += 2 * w) {
-      const int mid = min(lo + w, n), hi = min(lo + 2 * w, n);
-      for (int q = lo + (int)threadIdx.x; q < hi; q += blockDim.x) {
-        const uint64_t x = src[q];
-        const int pos = q < mid ? (q - lo) + lower_bound_u64(src + mid, hi - mid, x)
-                                : (q - mid) + lower_bound_u64(src + lo, mid - lo, x);
-        dst[lo + pos] = x;
+  const int64_t nlist = (int64_t)counters[3];
+  for (int64_t i = blockIdx.x; i < nlist; i += gridDim.x) {
+    const int32_t cidx = biglist[i];
+    const int n = cnt[cidx];
+    uint64_t *s = a + start[cidx];
+    if (n <= BIG_SORT) {
+      int m = 1;
+      while (m < n) m <<= 1;
+      for (int q = threadIdx.x; q < m; q += blockDim.x) sk[q] = q < n ? s[q] : ~0ull;
+      __syncthreads();
+      lds_bitonic(sk, m);
+      for (int q = threadIdx.x; q < n; q += blockDim.x) s[q] = sk[q];
+      __syncthreads();
+      continue;
+    }
+    for (int c0 = 0; c0 < n; c0 += BIG_SORT) {
+      const int len = min(BIG_SORT, n - c0);
+      for (int q = threadIdx.x; q < BIG_SORT; q += blockDim.x) sk[q] = q < len ? s[c0 + q] : ~0ull;
+      __syncthreads();
+      lds_bitonic(sk, BIG_SORT);
+      for (int q = threadIdx.x; q < len; q += blockDim.x) s[c0 + q] = sk[q];
+      __syncthreads();
+    }
+    uint64_t *src = s, *dst = tmp + start[cidx];
+    for (int w = BIG_SORT; w < n; w <<= 1) {
+      for (int lo = 0; lo < n; lo += 2 * w) {
+        const int mid = min(lo + w, n), hi = min(lo + 2 * w, n);
+        for (int q = lo + (int)threadIdx.x; q < hi; q += blockDim.x) {
+          const uint64_t x = src[q];
+          const int pos = q < mid ? (q - lo) + lower_bound_u64(src + mid, hi - mid, x)
+                                  : (q - mid) + lower_bound_u64(src + lo, mid - lo, x);
+          dst[lo + pos] = x;
+        }
       }
+      __syncthreads();
+      uint64_t *t = src;
+      src = dst;
+      dst = t;
+    }
+    if (src != s) {
+      for (int q = threadIdx.x; q < n; q += blockDim.x) s[q] = src[q];
     }
     __syncthreads();
-    uint64_t *t = src;
-    src = dst;
-    dst = t;
-  }
-  if (src != s) {
-    for (int q = threadIdx.x; q < n; q += blockDim.x) s[q] = src[q];
   }
 }
 
 /* ---------------- per-cell finalize ---------------- */
 /*
  * Finalize by slot ranges: a workgroup owns FB_CELLS consecutive new cells
- * and the contiguous slot range of their particles.  Lanes gather the
- * decoded velocities of consecutive slots into LDS (one lane per slot), one
- * thread per cell then accumulates vfield_new serially in slot order (the
- * reference's order), and lanes write the re-quantised x, v and pid of
- * consecutive slots, so the stores are coalesced.  The velocity statistics
+ * and the contiguous slot range of their particles, and goes through them in
+ * runs of whole cells of at most FB_CH slots.  A run's keys are put in order
+ * in LDS, lanes gather the decoded velocities of consecutive slots (one lane
+ * per slot), one thread per cell then accumulates vfield_new serially in slot
+ * order (the reference's order), and lanes write the re-quantised x, v and pid
+ * of consecutive slots, so the stores are coalesced.  A cell above FB_CH is a
+ * run of its own in pieces, all gathered for the sum and again for the stores.
+ * Ranking every cell up to FB_LDS_SORT here replaced a lane per cell sorting in
+ * scratch memory where a workgroup's cells did not fit in one run: with the
+ * flags and the count read back 15 + 8 us on 16^3 cells, 113 us on 48^3 and 610
+ * us on 128^3 at 16 particles a cell, against nothing but this kernel's own 21
+ * -> 23, 54 -> 58 and 780 -> 820 us.  The velocity statistics
  * of the new state (W/update_particle.f90:172-224) are reduced on the way:
  * per workgroup in a fixed tree, then over workgroups in order.
  */
@@ -558,8 +612,8 @@ template <int IX, int IV>
 __global__ __launch_bounds__(256) void k_drift_final2(
     const typename IntOf<IX>::T *__restrict__ xp, const typename IntOf<IV>::T *__restrict__ vp,
     const int32_t *__restrict__ pid, const float *__restrict__ vfield_old, const int64_t *__restrict__ start,
-    const uint64_t *__restrict__ keys, const uint8_t *__restrict__ flag, const double *__restrict__ vdec, DriftP P,
-    double venc, typename IntOf<IX>::T *__restrict__ xp2, typename IntOf<IV>::T *__restrict__ vp2,
+    const uint64_t *__restrict__ keys, const double *__restrict__ vdec, DriftP P, double venc,
+    typename IntOf<IX>::T *__restrict__ xp2, typename IntOf<IV>::T *__restrict__ vp2,
     int32_t *__restrict__ pid2, float *__restrict__ vfield_new, int64_t ncells, double *__restrict__ part) {
   __shared__ int64_t cst[FB_CELLS + 1];
   __shared__ double vr[FB_CH][3]; /* decoded velocities; the final reduction reuses it */
@@ -580,143 +634,105 @@ __global__ __launch_bounds__(256) void k_drift_final2(
     cgeo[tid][3] = (int)(cidx / ((int64_t)nt * nt * nt));
   }
   __syncthreads();
-  const int64_t S0 = cst[0], S1 = cst[ncl];
-  /* every slot fits (and every cell is small): sort the keys of each cell
-     here and keep the gathers in LDS for the write pass */
-  const bool one = flag[blockIdx.x] != 0;
-  if (one) {
-    for (int64_t s = S0 + tid; s < S1; s += 256) pix[s - S0] = keys[s];
-    if (tid < ncl) {
-      const int lo = (int)(cst[tid] - S0), hi = (int)(cst[tid + 1] - S0);
-      for (int q = lo; q < hi; ++q) lcell[q] = (uint8_t)tid;
-    }
-    __syncthreads();
-    /* each key's place in its cell is the number of smaller keys there
-       (unique: they carry the particle index); every lane ranks its own
-       slots at once instead of one lane per cell sorting serially */
-    constexpr int PER = (FB_CH + 255) / 256;
-    uint64_t kx[PER];
-    int dst[PER];
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int q = tid + 256 * u;
-      dst[u] = -1;
-      if (q < (int)(S1 - S0)) {
-        const int c = lcell[q], lo = (int)(cst[c] - S0), hi = (int)(cst[c + 1] - S0);
-        const uint64_t x = pix[q];
-        int r = 0;
-        for (int w = lo; w < hi; ++w) r += pix[w] < x ? 1 : 0;
-        kx[u] = x;
-        dst[u] = lo + r;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < PER; ++u)
-      if (dst[u] >= 0) pix[dst[u]] = kx[u];
-    __syncthreads();
-  }
-  auto cell_of = [&](int64_t s) -> int {
-    if (one) return lcell[s - S0];
-    int lo = 0, hi = ncl;
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (cst[mid] <= s) lo = mid; else hi = mid;
-    }
-    return lo;
-  };
-
-  /* slot -> (local cell, source particle, decoded velocity) */
-  auto gather = [&](int64_t s, int &lc, int64_t &p, double v[3]) {
-    lc = cell_of(s);
-    const int i = cgeo[lc][0], j = cgeo[lc][1], k = cgeo[lc][2], t = cgeo[lc][3];
-    const uint64_t kk = one ? pix[s - S0] : keys[s];
-    p = (int64_t)(kk & KEY_PMASK);
-    const int rx = (int)((kk >> 40) & 31), ry = (int)((kk >> 45) & 31), rz = (int)((kk >> 50) & 31);
-    /* source cell = destination + (r - 2ncb), in the destination tile frame */
-    const int sx = i + rx - 2 * ncb, sy = j + ry - 2 * ncb, sz = k + rz - 2 * ncb;
-    int64_t sc;
-    if (sx >= 0 && sx < nt && sy >= 0 && sy < nt && sz >= 0 && sz < nt) {
-      sc = g.cid(sx, sy, sz, t);
-    } else {
-      const int tz = t / (g.nnt * g.nnt), ty = (t / g.nnt) % g.nnt, tx = t % g.nnt;
-      sc = cid_global(g, tx * nt + sx, ty * nt + sy, tz * nt + sz);
-    }
-    const V3f vo = *reinterpret_cast<const V3f *>(vfield_old + 3 * sc); /* one 12-byte load */
-    const float vof[3] = {vo.x, vo.y, vo.z};
-#pragma unroll
-    for (int a = 0; a < 3; ++a) v[a] = vdec[(int32_t)vp[3 * p + a] + P.nvh] + (double)vof[a];
-  };
-
+  const int64_t S0 = cst[0];
   /* vfield_new: thread (component aa, cell ca) sums its cell's slots in
      slot order -- three independent serial chains per cell, so a crowded
      cell holds its workgroup a third as long */
   const int ca = tid & 63, aa = tid >> 6;
-  const bool accum = aa < 3 && ca < ncl;
-  float acc = 0.f;
-  if (accum) acc = (float)((double)vfield_old[3 * (c0 + ca) + aa] * WEIGHT_V);
-  for (int64_t ch = S0; ch < S1; ch += FB_CH) {
-    const int64_t ce = min(ch + FB_CH, S1);
-    for (int64_t s = ch + tid; s < ce; s += 256) {
-      int lc;
-      int64_t p;
-      double v[3];
-      gather(s, lc, p, v);
-      vr[s - ch][0] = v[0];
-      vr[s - ch][1] = v[1];
-      vr[s - ch][2] = v[2];
-      pix[s - ch] = (uint64_t)p;
+  double sr = 0, ss = 0;
+  for (int c_lo = 0; c_lo < ncl;) {
+    const int c_hi = seg_end(cst, ncl, c_lo);
+    const int64_t s0 = cst[c_lo], s1 = cst[c_hi];
+    const int np = max(1, (int)((s1 - s0 + FB_CH - 1) / FB_CH)), rounds = np > 1 ? 2 * np : 1; /* uniform */
+    const bool accum = aa < 3 && ca >= c_lo && ca < c_hi;
+    float acc = 0.f;
+    if (accum) acc = (float)((double)vfield_old[3 * (c0 + ca) + aa] * WEIGHT_V);
+#pragma unroll 1
+    for (int u = 0; u < rounds; ++u) {
+      const int64_t ch = s0 + (int64_t)(u < np ? u : u - np) * FB_CH, ce = min(ch + FB_CH, s1);
+      /* slot s always belongs to the same lane: the sums' order */
+      const int first = (tid - (int)(ch - S0)) & 255;
+      if (np == 1) {
+        seg_sort(keys, cst, c_lo, c_hi, pix, lcell);
+      } else {
+        for (int64_t s = ch + tid; s < ce; s += 256) {
+          pix[s - ch] = keys[s];
+          lcell[s - ch] = (uint8_t)c_lo;
+        }
+        __syncthreads();
+      }
+#pragma unroll 1
+      for (int q = tid; q < (int)(ce - ch); q += 256) {
+        const int lc = lcell[q], i = cgeo[lc][0], j = cgeo[lc][1], k = cgeo[lc][2], t = cgeo[lc][3];
+        const uint64_t kk = pix[q];
+        const int64_t p = (int64_t)(kk & KEY_PMASK);
+        const int rx = (int)((kk >> 40) & 31), ry = (int)((kk >> 45) & 31), rz = (int)((kk >> 50) & 31);
+        /* source cell = destination + (r - 2ncb), in the destination tile frame */
+        const int sx = i + rx - 2 * ncb, sy = j + ry - 2 * ncb, sz = k + rz - 2 * ncb;
+        int64_t sc;
+        if (sx >= 0 && sx < nt && sy >= 0 && sy < nt && sz >= 0 && sz < nt) {
+          sc = g.cid(sx, sy, sz, t);
+        } else {
+          const int tz = t / (g.nnt * g.nnt), ty = (t / g.nnt) % g.nnt, tx = t % g.nnt;
+          sc = cid_global(g, tx * nt + sx, ty * nt + sy, tz * nt + sz);
+        }
+        const V3f vo = *reinterpret_cast<const V3f *>(vfield_old + 3 * sc); /* one 12-byte load */
+        const float vof[3] = {vo.x, vo.y, vo.z};
+#pragma unroll
+        for (int a = 0; a < 3; ++a) vr[q][a] = vdec[(int32_t)vp[3 * p + a] + P.nvh] + (double)vof[a];
+        pix[q] = (uint64_t)p;
+      }
+      __syncthreads();
+      if (u < np) { /* uniform */
+        if (accum) {
+          const int lo = (int)(max(cst[ca], ch) - ch), hi = (int)(min(cst[ca + 1], ce) - ch);
+          for (int q = lo; q < hi; ++q) acc = (float)((double)acc + vr[q][aa]);
+          if (u == np - 1) {
+            const double n = (double)(cst[ca + 1] - cst[ca]);
+            vn[ca][aa] = (float)((double)acc / (n + WEIGHT_V));
+            vfield_new[3 * (c0 + ca) + aa] = vn[ca][aa];
+          }
+        }
+        __syncthreads();
+      }
+      if (np == 1 || u >= np) {
+#pragma unroll 1
+        for (int q = first; q < (int)(ce - ch); q += 256) {
+          const int lc = lcell[q];
+          const int64_t p = (int64_t)pix[q], s = ch + q;
+          const double vres[3] = {vr[q][0] - (double)vn[lc][0], vr[q][1] - (double)vn[lc][1],
+                                  vr[q][2] - (double)vn[lc][2]};
+          /* vp_new=nint(...atan(...*(vreal-vfield_new))...) (:116-117) */
+          int32_t code[3];
+#pragma unroll
+          for (int a = 0; a < 3; ++a) code[a] = cube_encode_v(IV, venc, vres[a]);
+          double r[3];
+#pragma unroll
+          for (int a = 0; a < 3; ++a) {
+            /* xp_new=xp+nint(dt_mid*vreal/(x_resolution*ncell)) (:115) */
+            const double qx = ((double)P.dt_mid * vr[q][a]) * P.inv_xres4;
+            xp2[3 * s + a] = (typename IntOf<IX>::T)cube_wrap(IX, (int64_t)xp[3 * p + a] + (int64_t)cube_nint(qx));
+            vp2[3 * s + a] = (typename IntOf<IV>::T)code[a];
+            r[a] = vdec[code[a] + P.nvh];
+          }
+          if (pid) pid2[s] = pid[p];
+          sr += (r[0] * r[0] + r[1] * r[1]) + r[2] * r[2];
+          r[0] += (double)vn[lc][0];
+          r[1] += (double)vn[lc][1];
+          r[2] += (double)vn[lc][2];
+          ss += (r[0] * r[0] + r[1] * r[1]) + r[2] * r[2];
+        }
+      }
+      __syncthreads();
     }
-    __syncthreads();
-    if (accum) {
-      const int64_t lo = max(cst[ca], ch), hi = min(cst[ca + 1], ce);
-      for (int64_t q = lo; q < hi; ++q) acc = (float)((double)acc + vr[q - ch][aa]);
-    }
-    __syncthreads();
+    c_lo = c_hi;
   }
-  if (accum) {
-    const double n = (double)(cst[ca + 1] - cst[ca]);
-    vn[ca][aa] = (float)((double)acc / (n + WEIGHT_V));
-    vfield_new[3 * (c0 + ca) + aa] = vn[ca][aa];
-  }
-  __syncthreads();
-  double sc = 0, sr = 0, ss = 0;
+  double sc = 0;
   if (tid < ncl) {
     const float v0 = vn[tid][0], v1 = vn[tid][1], v2 = vn[tid][2];
     sc = (double)((v0 * v0 + v1 * v1) + v2 * v2);
   }
-  for (int64_t s = S0 + tid; s < S1; s += 256) {
-    int lc;
-    int64_t p;
-    double v[3];
-    if (one) {
-      lc = lcell[s - S0];
-      p = (int64_t)pix[s - S0];
-      v[0] = vr[s - S0][0];
-      v[1] = vr[s - S0][1];
-      v[2] = vr[s - S0][2];
-    } else {
-      gather(s, lc, p, v);
-    }
-    double r[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      /* xp_new=xp+nint(dt_mid*vreal/(x_resolution*ncell)) (:115) */
-      const double qx = ((double)P.dt_mid * v[a]) * P.inv_xres4;
-      xp2[3 * s + a] = (typename IntOf<IX>::T)cube_wrap(IX, (int64_t)xp[3 * p + a] + (int64_t)cube_nint(qx));
-      /* vp_new=nint(...atan(...*(vreal-vfield_new))...) (:116-117) */
-      const int32_t code = cube_encode_v(IV, venc, v[a] - (double)vn[lc][a]);
-      vp2[3 * s + a] = (typename IntOf<IV>::T)code;
-      r[a] = vdec[(int32_t)(typename IntOf<IV>::T)code + P.nvh];
-    }
-    if (pid) pid2[s] = pid[p];
-    sr += (r[0] * r[0] + r[1] * r[1]) + r[2] * r[2];
-    r[0] += (double)vn[lc][0];
-    r[1] += (double)vn[lc][1];
-    r[2] += (double)vn[lc][2];
-    ss += (r[0] * r[0] + r[1] * r[1]) + r[2] * r[2];
-  }
-  __syncthreads(); /* vr is free: reduce through it */
+  /* vr is free: reduce through it */
   double(*red)[256] = reinterpret_cast<double(*)[256]>(&vr[0][0]);
   red[0][tid] = sc;
   red[1][tid] = sr;
@@ -829,32 +845,29 @@ __global__ void k_place_keys(const int32_t *dest, const uint64_t *key, int64_t n
     out[start[d] + s] = key[p];
   }
 }
-/* sort every cell's key segment ascending (small ones in registers, medium
-   ones with a wave's bitonic sort, big ones with a workgroup's, huge ones by
-   merging sorted runs);
-   c->key, dead once the keys are placed, is the merge buffer */
+/* the cells that are listed: medium ones with a wave's bitonic sort, big ones
+   with a workgroup's, huge ones by merging sorted runs, tmp the merge buffer.
+   Fixed grids that the lists' counts cut short, so the host need not know them */
+static int sort_listed(cube_ctx *c, const int32_t *cnt, const int64_t *start, uint64_t *keys, const int32_t *list,
+                       const unsigned long long *ctr, uint64_t *tmp) {
+  hipLaunchKernelGGL(k_sort_med, dim3((unsigned)std::min<int64_t>((c->ncells + 3) / 4, 1280)), dim3(256), 0, c->stream, cnt,
+                     start, list, c->ncells, ctr, keys);
+  CUBE_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_sort_big, dim3((unsigned)std::min<int64_t>(c->ncells, 256)), dim3(1024), BIG_SORT * sizeof(uint64_t),
+                     c->stream, cnt, start, list, ctr, keys, tmp);
+  CUBE_LAUNCH_CHECK();
+  return CUBE_OK;
+}
+/* sort every cell's key segment ascending; c->key, dead once the keys are
+   placed, is the merge buffer */
 extern "C" int cube_sort_small_segments(cube_ctx *c, const int32_t *cnt, const int64_t *start, uint64_t *keys) {
   unsigned long long *ctr = (unsigned long long *)c->ured;
   int st = fill_i64(c, (int64_t *)ctr + 3, 2, 0);
   if (st) return st;
-  const unsigned nbc = (unsigned)((c->ncells + 255) / 256);
-  int32_t *biglist = (int32_t *)c->dest;
-  hipLaunchKernelGGL(k_sort_small, dim3(nbc), dim3(256), 0, c->stream, cnt, start, c->ncells, keys, biglist, ctr,
-                     (const uint8_t *)nullptr);
+  hipLaunchKernelGGL(k_sort_cells, dim3((unsigned)((c->ncells + FB_CELLS - 1) / FB_CELLS)), dim3(256), 0, c->stream, cnt,
+                     start, c->ncells, keys, (int32_t *)c->dest, ctr);
   CUBE_LAUNCH_CHECK();
-  unsigned long long hc[8];
-  CUBE_CHECK(hipMemcpy(hc, ctr, sizeof(hc), hipMemcpyDeviceToHost));
-  if (hc[4]) {
-    hipLaunchKernelGGL(k_sort_med, dim3((unsigned)((hc[4] + 3) / 4)), dim3(256), 0, c->stream, cnt, start,
-                       biglist + c->ncells - (int64_t)hc[4], (int64_t)hc[4], keys);
-    CUBE_LAUNCH_CHECK();
-  }
-  if (hc[3]) {
-    hipLaunchKernelGGL(k_sort_big, dim3((unsigned)hc[3]), dim3(1024), BIG_SORT * sizeof(uint64_t), c->stream, cnt,
-                       start, biglist, keys, c->key);
-    CUBE_LAUNCH_CHECK();
-  }
-  return CUBE_OK;
+  return sort_listed(c, cnt, start, keys, (const int32_t *)c->dest, ctr, c->key);
 }
 
 /* ---------------- driver ---------------- */
@@ -879,37 +892,21 @@ template <int IX, int IV> static int drift_impl(cube_ctx *c, DriftP P, double ve
   if (hc[2] & DERR_XOVER) return CUBE_ERR_IMAGE_OVERFLOW;
   if (total > c->cap) return CUBE_ERR_IMAGE_OVERFLOW;
   *nxtra = (int64_t)hc[0];
+  int32_t *list = c->fill; /* the initial sort's, free here */
   hipLaunchKernelGGL(k_place_ranked, dim3(4096), dim3(256), 0, c->stream, c->dest, c->rank, c->key, c->nplocal,
-                     c->cstart2, c->sortbuf);
+                     c->cstart2, c->sortbuf, c->rhoc2, c->ncells, list, ctr);
   CUBE_LAUNCH_CHECK();
   if (hc[0]) {
     hipLaunchKernelGGL(k_place_ranked, dim3(64), dim3(256), 0, c->stream, c->xdest, c->xrank, c->xkey,
-                       (int64_t)hc[0], c->cstart2, c->sortbuf);
+                       (int64_t)hc[0], c->cstart2, c->sortbuf, (const int32_t *)nullptr, c->ncells, list, ctr);
     CUBE_LAUNCH_CHECK();
   }
-  const unsigned nbc = (unsigned)((c->ncells + 255) / 256);
+  /* key is dead after placement: the merge buffer */
+  if ((st = sort_listed(c, c->rhoc2, c->cstart2, c->sortbuf, list, ctr, c->key))) return st;
   const int64_t nfb = (c->ncells + FB_CELLS - 1) / FB_CELLS;
-  hipLaunchKernelGGL(k_fb_flags, dim3((unsigned)((nfb + 255) / 256)), dim3(256), 0, c->stream, c->rhoc2, c->cstart2,
-                     c->ncells, c->fbflag);
-  CUBE_LAUNCH_CHECK();
-  int32_t *biglist = (int32_t *)c->dest; /* dest is dead after placement */
-  hipLaunchKernelGGL(k_sort_small, dim3(nbc), dim3(256), 0, c->stream, c->rhoc2, c->cstart2, c->ncells, c->sortbuf,
-                     biglist, ctr, c->fbflag);
-  CUBE_LAUNCH_CHECK();
-  CUBE_CHECK(hipMemcpy(hc, ctr, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost));
-  if (hc[4]) {
-    hipLaunchKernelGGL(k_sort_med, dim3((unsigned)((hc[4] + 3) / 4)), dim3(256), 0, c->stream, c->rhoc2,
-                       c->cstart2, biglist + c->ncells - (int64_t)hc[4], (int64_t)hc[4], c->sortbuf);
-    CUBE_LAUNCH_CHECK();
-  }
-  if (hc[3]) {
-    hipLaunchKernelGGL(k_sort_big, dim3((unsigned)hc[3]), dim3(1024), BIG_SORT * sizeof(uint64_t), c->stream,
-                       c->rhoc2, c->cstart2, biglist, c->sortbuf, c->key); /* key is dead after placement */
-    CUBE_LAUNCH_CHECK();
-  }
   hipLaunchKernelGGL((k_drift_final2<IX, IV>), dim3((unsigned)nfb), dim3(256), 0, c->stream, (const TX *)c->xp,
                      (const TV *)c->vp, c->p.has_pid ? c->pid : nullptr, c->vfield, c->cstart2, c->sortbuf,
-                     c->fbflag, c->vdec0, P, venc, (TX *)c->xp2, (TV *)c->vp2, c->pid2, c->vfield2, c->ncells,
+                     c->vdec0, P, venc, (TX *)c->xp2, (TV *)c->vp2, c->pid2, c->vfield2, c->ncells,
                      c->vpart);
   CUBE_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_sum_parts_tree, dim3(1), dim3(1024), 0, c->stream, c->vpart, nfb, c->dred);
@@ -928,7 +925,7 @@ int cube_drift(cube_ctx *c, float dt_old, float dt, float vz_max, float sigma_vi
      tile's extended region must fit np_tile_max */
   int64_t *sums = (int64_t *)malloc(c->ntiles * sizeof(int64_t));
   tbeg(c);
-  int st = cube_tile_boxsum(c, c->rhoc, (int)c->ncb, sums);
+  int st = cube_tile_boxsum(c, (int)c->ncb, sums);
   tend(c, CUBE_T_CHECKS);
   double ov = 0;
   int64_t mx = 0;

@@ -64,7 +64,6 @@ struct cube_ctx {
   int32_t *xdest;           /* extra copies (duplicates in the reference)      */
   uint64_t *xkey;
   int32_t *rank, *xrank;    /* slot of each (extra) copy inside its new cell, arrival order */
-  uint8_t *fbflag;          /* per finalize block: 1 = sorted and finished in LDS */
   int64_t xcap;
   /* codec tables */
   float *tanf_tab;          /* nvbin: tanf(pi*code/(nvbin-1)), index code+nvbin/2 */
@@ -94,7 +93,7 @@ struct cube_ctx {
   double *fdheavy;          /* and FDH_W sums of its crowded cells */
   int32_t *fdlist;          /* and its list of blocks with crowded cells (length in ured) */
   uint64_t *fdmask;         /* those cells, by block */
-  int64_t *ired;            /* 4096 */
+  int64_t *ired;            /* the tiles' box sums, BOX_WG parts each */
   int64_t *scanbuf;         /* ncells/1024 + 2 block sums of the scan */
   double *vpart;            /* 3 per finalize block of the drift (velocity sums) */
   /* host-side persistent state */
@@ -297,7 +296,8 @@ __device__ static inline float cube_kfac(int d, int mx, int my, int mz, int n) {
 int cube_drift(cube_ctx *c, float dt_old, float dt, float vz_max, float sigma_vi, cube_vstats *out);
 int cube_vdec_table(cube_ctx *c, double *dst, float sigma);
 int cube_scan_counts(cube_ctx *c, const int32_t *cnt, int64_t *start, int64_t n, int64_t *total);
-int cube_tile_boxsum(cube_ctx *c, const int32_t *rhoc, int w, int64_t *host_out);
+#define BOX_WG 8 /* workgroups per tile */
+int cube_tile_boxsum(cube_ctx *c, int w, int64_t *host_out);
 
 /* 1 when the line-FFT kernels are built for size n (12..2048, factors 2, 3, 5) */
 int cube_fft_supported(int64_t n);

@@ -704,8 +704,7 @@ __global__ __launch_bounds__(256) void k_drift_final2(
                                   vr[q][2] - (double)vn[lc][2]};
           /* vp_new=nint(...atan(...*(vreal-vfield_new))...) (:116-117) */
           int32_t code[3];
-#pragma unroll
-          for (int a = 0; a < 3; ++a) code[a] = cube_encode_v(IV, venc, vres[a]);
+          cube_encode_v3(IV, venc, vres, code);
           double r[3];
 #pragma unroll
           for (int a = 0; a < 3; ++a) {

@@ -168,10 +168,14 @@ __global__ void k_xv_encode(const double *x, const float *v, const int32_t *cnt,
   const double res = IX == 1 ? 256.0 : 65536.0;
   for (int q = 0; q < n; ++q) {
     const int64_t p = (int64_t)(keys[s0 + q] & KEY_PMASK);
+    const double vres[3] = {(double)v[3 * p] - (double)vfield[3 * c], (double)v[3 * p + 1] - (double)vfield[3 * c + 1],
+                            (double)v[3 * p + 2] - (double)vfield[3 * c + 2]};
+    int32_t code[3];
+    cube_encode_v3(IV, venc, vres, code);
+#pragma unroll
     for (int a = 0; a < 3; ++a) {
       xp[3 * (s0 + q) + a] = (typename IntOf<IX>::T)cube_wrap(IX, (int64_t)floor(x[3 * p + a] * res));
-      vp[3 * (s0 + q) + a] =
-          (typename IntOf<IV>::T)cube_encode_v(IV, venc, (double)v[3 * p + a] - (double)vfield[3 * c + a]);
+      vp[3 * (s0 + q) + a] = (typename IntOf<IV>::T)code[a];
     }
     if (pid && ng <= 0) {
       pid[s0 + q] = (int32_t)(p + 1); /* host-given particles: input index */

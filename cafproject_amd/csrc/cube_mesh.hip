@@ -1155,24 +1155,25 @@ __global__ __launch_bounds__(KT) void k_kick(const typename IntOf<IX>::T *__rest
     kick_particle<IX, FINE, FINE && NKICK == 2>(code, loc, tt, g, force, a_mid, dt, vreal);
     if (NKICK == 2) {
       /* the code the fine kick would store, decoded again for the coarse kick */
+      int32_t v1[3];
+      cube_encode_v3(IV, venc, vreal, v1);
 #pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        const int32_t v1 = (int32_t)(typename IntOf<IV>::T)cube_encode_v(IV, venc, vreal[a]);
-        vreal[a] = vdec2[v1 + nvh];
-      }
+      for (int a = 0; a < 3; ++a) vreal[a] = vdec2[v1[a] + nvh];
       kick_particle<IX, false>(code, loc, tt, g, force2, a_mid, dt, vreal);
     }
     const double ve = NKICK == 2 ? venc2 : venc;
     F3 vc = {0.f, 0.f, 0.f};
     if (VMAX) vc = *reinterpret_cast<const F3 *>(vfield + 3 * (c0 + lo)); /* one 12-byte load */
     const float vcf[3] = {vc.x, vc.y, vc.z};
+    int32_t vcode[3];
+    cube_encode_v3(IV, ve, vreal, vcode);
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       if (VMAX) {
         const double av = fabs(vreal[a] + (double)vcf[a]);
         vm[a] = av > vm[a] ? av : vm[a];
       }
-      vp[3 * p + a] = (typename IntOf<IV>::T)cube_encode_v(IV, ve, vreal[a]);
+      vp[3 * p + a] = (typename IntOf<IV>::T)vcode[a];
     }
   }
   if (VMAX) vmax_reduce(vm, vmax_bits);

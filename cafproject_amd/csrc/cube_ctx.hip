@@ -166,12 +166,12 @@ extern "C" int cube_ctx_create(const cube_params *p, cube_ctx **out) {
     if (hipMemGetInfo(&fr, &tot) == hipSuccess && full > fr / 100 * 97) compact = 1;
   }
   c->fine_nspec = compact ? 1 : 3;
-  /* 16 bytes of padding: the deposits read a particle's 3 or 6 code bytes
-     with one 4- or 8-byte load, which ends past the last particle */
+  /* 16 bytes of padding: kernels read a particle's 3 or 6 code bytes with one
+     4- or 8-byte load, which ends past the last particle */
   st |= dalloc_bytes(&c->xp, c->cap * xb + 16);
-  st |= dalloc_bytes(&c->vp, c->cap * vb);
+  st |= dalloc_bytes(&c->vp, c->cap * vb + 16);
   st |= dalloc_bytes(&c->xp2, c->cap * xb + 16);
-  st |= dalloc_bytes(&c->vp2, c->cap * vb);
+  st |= dalloc_bytes(&c->vp2, c->cap * vb + 16);
   if (p->has_pid) {
     st |= dalloc(&c->pid, c->cap);
     st |= dalloc(&c->pid2, c->cap);

@@ -1013,12 +1013,11 @@ __global__ void k_kick_prescale(const float *__restrict__ F, int64_t n, float a_
    the 8 corners in the order of W/pm.f90:146-153 (fine: force_f with
    ((((F*a_mid)*dt)/6)/pi)*wx*wy*wz per term; coarse: the prescaled G with
    G*wx*wy*wz, W/pm.f90:341-348).  loc: 1-based cell in the tile, tt: tile. */
-template <int IX, bool FINE, bool PRE = false>
+template <int IX, bool FINE>
 __device__ __forceinline__ void kick_particle(const int32_t code[3], const int loc[3], const int tt[3],
                                               const Geo &g, const float *__restrict__ force, float a_mid,
                                               float dt, double vreal[3]) {
-  /* PRE: the fine mesh already holds (((F*a_mid)*dt)/6)/pi per value */
-  constexpr bool DIV = FINE && !PRE;
+  constexpr bool DIV = FINE;
   const int nt = g.nt, nfine = 4 * g.nc, nft = 4 * nt;
   int i1[3];
   float d1[3], d2[3];
@@ -1082,40 +1081,34 @@ __device__ __forceinline__ void kick_particle(const int32_t code[3], const int l
 /* max of |v + v_c| over the workgroup: wave shuffles, then the waves
    through LDS, one atomic per component into its slot region of
    vmax_bits (W/pm.f90:349) */
-__device__ __forceinline__ void vmax_reduce(double vm[3], unsigned long long *__restrict__ vmax_bits) {
+template <int THREADS> __device__ __forceinline__ void vmax_reduce(double vm[3], unsigned long long *__restrict__ vmax_bits) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1)
 #pragma unroll
     for (int a = 0; a < 3; ++a) vm[a] = fmax(vm[a], __shfl_xor(vm[a], o, 64));
-  __shared__ double red[3][KT / 64];
+  __shared__ double red[3][THREADS / 64];
   if ((threadIdx.x & 63) == 0)
     for (int a = 0; a < 3; ++a) red[a][threadIdx.x >> 6] = vm[a];
   __syncthreads();
   if (threadIdx.x < 3) {
     double m = red[threadIdx.x][0];
-    for (int w = 1; w < KT / 64; ++w) m = fmax(m, red[threadIdx.x][w]);
+    for (int w = 1; w < THREADS / 64; ++w) m = fmax(m, red[threadIdx.x][w]);
     atomicMax(cube_slot(vmax_bits + threadIdx.x * CUBE_SLOTS), (unsigned long long)__double_as_longlong(m));
   }
 }
 
 /* kicks, one workgroup per cell row (tile, k, j): particles of the row are
-   contiguous; each thread finds its cell by binary search in LDS.
-   NKICK = 1: the one kick of FINE (decode with vdec, encode with venc);
-   NKICK = 2: the fine kick (vdec, venc) from the prescaled fine mesh that
-   the step's force pipeline leaves in force_f, then the coarse one on the
-   re-decoded code (vdec2, venc2) in the same pass, which is the step's
-   sequence W/pm.f90:129-159 then 322-354 with the intermediate codes kept
-   in registers instead of going through vp. */
+   contiguous; each thread finds its cell by binary search in LDS.  The one
+   kick of FINE (decode with vdec, encode with venc), for callers that take
+   the stages one by one; a step takes k_kicks. */
 #define KICK_ROW 2048 /* particles of a row whose cells the kick tables in LDS (else a binary search) */
-template <int IX, int IV, bool FINE, int NKICK>
+template <int IX, int IV, bool FINE>
 __global__ __launch_bounds__(KT) void k_kick(const typename IntOf<IX>::T *__restrict__ xp,
                                              typename IntOf<IV>::T *__restrict__ vp,
                                              const int64_t *__restrict__ cstart, const float *__restrict__ vfield,
                                              const float *__restrict__ force, const double *__restrict__ vdec,
                                              Geo g, int nvh, float a_mid, float dt, double venc,
-                                             unsigned long long *__restrict__ vmax_bits,
-                                             const float *__restrict__ force2, const double *__restrict__ vdec2,
-                                             double venc2) {
+                                             unsigned long long *__restrict__ vmax_bits) {
   const int nt = g.nt;
   const int64_t row = blockIdx.x;
   const int j = (int)(row % nt), k = (int)((row / nt) % nt), t = (int)(row / ((int64_t)nt * nt));
@@ -1131,7 +1124,7 @@ __global__ __launch_bounds__(KT) void k_kick(const typename IntOf<IX>::T *__rest
       for (int64_t q = cs[i]; q < cs[i + 1]; ++q) lcell[q - cs[0]] = (uint16_t)i;
     __syncthreads();
   }
-  constexpr bool VMAX = !FINE || NKICK == 2; /* the coarse kick reports vmax */
+  constexpr bool VMAX = !FINE; /* the coarse kick reports vmax */
   double vm[3] = {0, 0, 0};
   for (int64_t p = cs[0] + threadIdx.x; p < cs[nt]; p += KT) {
     int lo = 0, hi = nt;
@@ -1152,21 +1145,12 @@ __global__ __launch_bounds__(KT) void k_kick(const typename IntOf<IX>::T *__rest
       code[a] = (int32_t)xp[3 * p + a];
       vreal[a] = vdec[(int32_t)vp[3 * p + a] + nvh];
     }
-    kick_particle<IX, FINE, FINE && NKICK == 2>(code, loc, tt, g, force, a_mid, dt, vreal);
-    if (NKICK == 2) {
-      /* the code the fine kick would store, decoded again for the coarse kick */
-      int32_t v1[3];
-      cube_encode_v3(IV, venc, vreal, v1);
-#pragma unroll
-      for (int a = 0; a < 3; ++a) vreal[a] = vdec2[v1[a] + nvh];
-      kick_particle<IX, false>(code, loc, tt, g, force2, a_mid, dt, vreal);
-    }
-    const double ve = NKICK == 2 ? venc2 : venc;
+    kick_particle<IX, FINE>(code, loc, tt, g, force, a_mid, dt, vreal);
     F3 vc = {0.f, 0.f, 0.f};
     if (VMAX) vc = *reinterpret_cast<const F3 *>(vfield + 3 * (c0 + lo)); /* one 12-byte load */
     const float vcf[3] = {vc.x, vc.y, vc.z};
     int32_t vcode[3];
-    cube_encode_v3(IV, ve, vreal, vcode);
+    cube_encode_v3(IV, venc, vreal, vcode);
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       if (VMAX) {
@@ -1176,27 +1160,208 @@ __global__ __launch_bounds__(KT) void k_kick(const typename IntOf<IX>::T *__rest
       vp[3 * p + a] = (typename IntOf<IV>::T)vcode[a];
     }
   }
-  if (VMAX) vmax_reduce(vm, vmax_bits);
+  if (VMAX) vmax_reduce<KT>(vm, vmax_bits);
 }
 
-template <int IX, int IV, bool FINE, int NKICK>
-static int kick_impl(cube_ctx *c, const float *force, float a_mid, float dt, double venc,
-                     unsigned long long *vmb, const float *force2, double venc2) {
-  const int64_t nrows = c->ncells / c->nt;
-  hipLaunchKernelGGL((k_kick<IX, IV, FINE, NKICK>), dim3((unsigned)nrows), dim3(KT), 0, c->stream,
-                     (const typename IntOf<IX>::T *)c->xp, (typename IntOf<IV>::T *)c->vp, c->cstart, c->vfield, force,
-                     c->vdec0, geo_of(c), c->nvbin / 2, a_mid, dt, venc, vmb, force2, c->vdec1, venc2);
+/*
+ * The step's two kicks in one pass, W/pm.f90:129-159 then 322-354: the fine one
+ * (decode with vdec) from the prescaled mesh that the step's force pipeline
+ * leaves in force_f, then the coarse one on the code the fine one would store
+ * (decoded again with vdec2), the intermediate codes in registers instead of
+ * going through vp.
+ *
+ * One workgroup per block of 4x2x2 coarse cells of a tile.  Gathering 16
+ * corners per particle from global memory, the mesh of a row of cells never in
+ * L1 for long, was bound by those gathers.  Here the block's mesh values
+ * (planes 0..16, 0..8, 0..8 of its 16x8x8 fine cells, and its coarse cells with
+ * a ring) go to LDS in rows of 16-byte loads, and the gathers are LDS reads.
+ * The first particles' words fly with them.  8 workgroups a CU hide one
+ * another's loads; what bounds it now is VALU issue (some 840 instructions per
+ * wave, at 4 ms of 7.4).  8x2x2 and 4x4x2 cells (4 workgroups a CU) took 8.7
+ * and 7.7 ms, several blocks per workgroup 7.6 (99 registers).  With a
+ * workgroup per row of cells, before -> after: 8.1 -> 7.4 ms on the 1024^3
+ * fine mesh with 512^3 particles (13 GB of mesh), 1.29 -> 1.00 ms on
+ * 512^3 with 256^3, 157 -> 141 us on 256^3 and 201 -> 148 us on its clustered
+ * z = 0 state, 74 -> 51 us on 192^3; 8.9 -> 9.7 us on 64^3.
+ */
+#define KB 192 /* 16 cells at the usual 8 particles, and half as many again; 12 rows of 16 lanes load a plane */
+template <int IX, int IV, bool EX>
+__global__ __launch_bounds__(KB) void k_kicks(const typename IntOf<IX>::T *__restrict__ xp,
+                                              typename IntOf<IV>::T *__restrict__ vp, const int64_t *__restrict__ cstart,
+                                              const float *__restrict__ vfield, const float *__restrict__ force,
+                                              const double *__restrict__ vdec, Geo g, int nvh, double venc,
+                                              unsigned long long *__restrict__ vmax_bits,
+                                              const float *__restrict__ force2, const double *__restrict__ vdec2) {
+  /* EX: the real(4) coordinate is exact, so a particle's second plane is at
+     most the first one past its cell; else it can round up to the one after.
+     A row is CH chunks of 16 bytes, loaded by 16 lanes */
+  constexpr int PL = EX ? 9 : 10, CH = EX ? 13 : 14, RF = 4 * CH;
+  __shared__ float4 fm[PL * PL * CH];
+  __shared__ float cm[4 * 4 * 18];
+  __shared__ int64_t cs[4][5];
+  __shared__ int pre[5];
+  const int nt = g.nt, tid = threadIdx.x;
+  /* consecutive blocks on one XCD, whose L2 then holds the planes they share */
+  const unsigned nq = gridDim.x >> 3, nr = gridDim.x & 7, xcd = blockIdx.x & 7;
+  const unsigned b = xcd * nq + min(xcd, nr) + (blockIdx.x >> 3);
+  const unsigned nbx = (nt + 3) / 4, nby = (nt + 1) / 2, nbz = (nt + 1) / 2, q1 = b / nbx, q2 = q1 / nby, t = q2 / nbz;
+  const int x0 = 4 * (int)(b - q1 * nbx), y0 = 2 * (int)(q1 - q2 * nby), z0 = 2 * (int)(q2 - t * nbz);
+  const unsigned t1 = t / (unsigned)g.nnt;
+  const int gx = (int)(t - t1 * g.nnt) * nt + x0, gy = (int)(t1 % (unsigned)g.nnt) * nt + y0,
+            gz = (int)(t1 / (unsigned)g.nnt) * nt + z0; /* the block's first cell in the box */
+  const int nf = 4 * g.nc, rowb = 12 * nf;
+  if (tid < 64) { /* starts of the 4 rows' cells; those past the tile are empty */
+    const int r = tid / 5, y = y0 + (r & 1), z = z0 + (r >> 1);
+    int64_t v = 0;
+    if (tid < 20) {
+      const bool in = y < nt && z < nt;
+      v = cstart[g.cid(0, in ? y : 0, in ? z : 0, (int)t) + (in ? min(x0 + tid % 5, nt) : 0)];
+      cs[r][tid % 5] = v;
+    }
+    const int lo = 5 * min(tid, 3);
+    const int n = (int)(__shfl(v, lo + 4, 64) - __shfl(v, lo, 64)); /* by the whole wave */
+    const int sc = wave_incl_scan(tid < 4 ? n : 0);
+    if (tid < 4) pre[tid + 1] = sc;
+    if (tid == 63) pre[0] = 0;
+  }
+  __syncthreads();
+  /* the mesh and the first particles fly together.  This lane's chunk of a
+     plane; its row's bytes are a multiple of 48, so no chunk straddles its end */
+  const int ry = tid >> 4, rc = tid & 15;
+  const bool on = rc < CH && ry < PL;
+  float4 raw[PL];
+  {
+    int x = 48 * gx + 16 * rc, y = 4 * gy + ry;
+    while (x >= rowb) x -= rowb;
+    while (y >= nf) y -= nf;
+    const uint32_t off = (uint32_t)y * (uint32_t)rowb + (uint32_t)x; /* a plane is below 2^32 bytes */
+#pragma unroll
+    for (int z = 0; z < PL; ++z) raw[z] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (on)
+#pragma unroll
+      for (int z = 0; z < PL; ++z) {
+        const int zz = 4 * gz + z;
+        const char *plane = reinterpret_cast<const char *>(force) + (int64_t)(zz < nf ? zz : zz - nf) * nf * rowb;
+        raw[z] = *reinterpret_cast<const float4 *>(plane + off);
+      }
+  }
+  float rawc[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int q = min(tid + KB * u, 287), r = q / 18, f = q - 18 * r;
+    int m[3] = {gx - 1 + f / 3, gy - 1 + (r & 3), gz - 1 + (r >> 2)};
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      m[a] += m[a] < 0 ? g.nc : 0;
+      while (m[a] >= g.nc) m[a] -= g.nc;
+    }
+    rawc[u] = force2[3 * ((int64_t)(m[2] * g.nc + m[1]) * g.nc + m[0]) + f % 3];
+  }
+  const int n = pre[4];
+  int r = 0, ci = 0; /* the particle's row, its cell of the row's 4 */
+  int64_t p = 0;
+  int32_t code[3] = {0, 0, 0};
+  double vreal[3] = {0, 0, 0};
+  F3 vc = {0.f, 0.f, 0.f};
+  auto fetch = [&](int q) {
+    r = pre[2] <= q ? 2 : 0;
+    r += pre[r + 1] <= q ? 1 : 0;
+    p = cs[r][0] + (q - pre[r]);
+    ci = (cs[r][1] <= p ? 1 : 0) + (cs[r][2] <= p ? 1 : 0) + (cs[r][3] <= p ? 1 : 0);
+    const typename CdWord<IX>::T wx = cd_load<IX>(reinterpret_cast<const char *>(xp) + 3 * IX * p);
+    const typename CdWord<IV>::T wv = cd_load<IV>(reinterpret_cast<const char *>(vp) + 3 * IV * p);
+    vc = *reinterpret_cast<const F3 *>(vfield + 3 * g.cid(x0 + ci, y0 + (r & 1), z0 + (r >> 1), (int)t));
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      code[a] = (int32_t)fd_code<IX>(wx, a);
+      vreal[a] = vdec[(int32_t)(typename IntOf<IV>::T)fd_code<IV>(wv, a) + nvh];
+    }
+  };
+  if (tid < n) fetch(tid);
+  if (on)
+#pragma unroll
+    for (int z = 0; z < PL; ++z) fm[(z * PL + ry) * CH + rc] = raw[z];
+  cm[tid] = rawc[0];
+  if (tid + KB < 288) cm[tid + KB] = rawc[1];
+  __syncthreads();
+  const float *ff = reinterpret_cast<const float *>(fm);
+  /* corner order of W/pm.f90:146-153 */
+  constexpr int ox[8] = {0, 1, 0, 0, 0, 1, 1, 1}, oy[8] = {0, 0, 1, 0, 1, 0, 1, 1}, oz[8] = {0, 0, 0, 1, 1, 1, 0, 1};
+  double vm[3] = {0, 0, 0};
+  for (int q = tid; q < n;) {
+    const int lc[3] = {ci, r & 1, r >> 1}, l0[3] = {x0, y0, z0}, g0[3] = {gx, gy, gz};
+    const float vcf[3] = {vc.x, vc.y, vc.z};
+#pragma unroll
+    for (int k = 0; k < 2; ++k) { /* the fine kick, the coarse kick */
+      int m[3];
+      float d1[3], d2[3];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        /* as in kick_particle; m: the first of the two planes in the staged block */
+        const float tempx = k == 0 ? (float)(4 * (l0[a] + lc[a])) + ((float)cube_ucode(IX, code[a]) + 0.5f) * (IX == 1 ? 0x1p-6f : 0x1p-14f)
+                                   : coarse_tempx<IX>(g0[a] + lc[a], code[a]);
+        const float fl = floorf(tempx);
+        m[a] = (int)fl - (k == 0 ? 4 * l0[a] : g0[a] - 1);
+        d1[a] = (float)((int)fl + 1) - tempx;
+        d2[a] = 1.0f - d1[a];
+      }
+      const float *F0 = k == 0 ? ff + (m[2] * PL + m[1]) * RF + 3 * m[0] : cm + (m[2] * 4 + m[1]) * 18 + 3 * m[0];
+      const int sy = k == 0 ? RF : 18, sz = k == 0 ? PL * RF : 72;
+#pragma unroll
+      for (int q8 = 0; q8 < 8; ++q8) {
+        const float *F = F0 + oz[q8] * sz + oy[q8] * sy + ox[q8] * 3;
+        const float wx = ox[q8] ? d2[0] : d1[0], wy = oy[q8] ? d2[1] : d1[1], wz = oz[q8] ? d2[2] : d1[2];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          const float inc = ((F[a] * wx) * wy) * wz;
+          vreal[a] = vreal[a] + (double)inc;
+        }
+      }
+      int32_t vcode[3];
+      cube_encode_v3(IV, venc, vreal, vcode);
+      if (k == 0) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) vreal[a] = vdec2[vcode[a] + nvh];
+      } else {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          const double av = fabs(vreal[a] + (double)vcf[a]);
+          vm[a] = av > vm[a] ? av : vm[a];
+          vp[3 * p + a] = (typename IntOf<IV>::T)vcode[a];
+        }
+      }
+    }
+    q += KB;
+    if (q < n) fetch(q);
+  }
+  vmax_reduce<KB>(vm, vmax_bits);
+}
+template <int IX, int IV> static int kicks_impl(cube_ctx *c, const float *G, double venc, unsigned long long *vmb) {
+  const int64_t nt = c->nt, grid = ((nt + 3) / 4) * ((nt + 1) / 2) * ((nt + 1) / 2) * c->ntiles;
+  auto kern = IX == 1 || nt <= 128 ? k_kicks<IX, IV, true> : k_kicks<IX, IV, IX == 1>; /* as in cube_fine_deposit */
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(KB), 0, c->stream, (const typename IntOf<IX>::T *)c->xp,
+                     (typename IntOf<IV>::T *)c->vp, c->cstart, c->vfield, c->force_f, c->vdec0, geo_of(c), c->nvbin / 2,
+                     venc, vmb, G, c->vdec1);
   CUBE_LAUNCH_CHECK();
   return CUBE_OK;
 }
-template <bool FINE, int NKICK = 1>
-static int kick(cube_ctx *c, const float *force, float a_mid, float dt, double venc, unsigned long long *vmb,
-                const float *force2 = nullptr, double venc2 = 0.0) {
+
+template <int IX, int IV, bool FINE>
+static int kick_impl(cube_ctx *c, const float *force, float a_mid, float dt, double venc, unsigned long long *vmb) {
+  const int64_t nrows = c->ncells / c->nt;
+  hipLaunchKernelGGL((k_kick<IX, IV, FINE>), dim3((unsigned)nrows), dim3(KT), 0, c->stream,
+                     (const typename IntOf<IX>::T *)c->xp, (typename IntOf<IV>::T *)c->vp, c->cstart, c->vfield, force,
+                     c->vdec0, geo_of(c), c->nvbin / 2, a_mid, dt, venc, vmb);
+  CUBE_LAUNCH_CHECK();
+  return CUBE_OK;
+}
+template <bool FINE>
+static int kick(cube_ctx *c, const float *force, float a_mid, float dt, double venc, unsigned long long *vmb) {
   const int x = c->p.izipx, v = c->p.izipv;
-  if (x == 1 && v == 1) return kick_impl<1, 1, FINE, NKICK>(c, force, a_mid, dt, venc, vmb, force2, venc2);
-  if (x == 1) return kick_impl<1, 2, FINE, NKICK>(c, force, a_mid, dt, venc, vmb, force2, venc2);
-  if (v == 1) return kick_impl<2, 1, FINE, NKICK>(c, force, a_mid, dt, venc, vmb, force2, venc2);
-  return kick_impl<2, 2, FINE, NKICK>(c, force, a_mid, dt, venc, vmb, force2, venc2);
+  if (x == 1 && v == 1) return kick_impl<1, 1, FINE>(c, force, a_mid, dt, venc, vmb);
+  if (x == 1) return kick_impl<1, 2, FINE>(c, force, a_mid, dt, venc, vmb);
+  if (v == 1) return kick_impl<2, 1, FINE>(c, force, a_mid, dt, venc, vmb);
+  return kick_impl<2, 2, FINE>(c, force, a_mid, dt, venc, vmb);
 }
 
 /* fine kick, W/pm.f90:129-159: decode with sigma_vi, encode with sigma_vi_new */
@@ -1226,7 +1391,11 @@ int cube_pm_kicks(cube_ctx *c, float a_mid, float dt, float sigma_vi, float sigm
   hipLaunchKernelGGL(k_kick_prescale, dim3(2048), dim3(256), 0, c->stream, c->force_c, 3 * c->ncells, a_mid, dt, G);
   CUBE_LAUNCH_CHECK();
   const double venc = cube_vconst(sigma_vi_new);
-  st = kick<true, 2>(c, c->force_f, a_mid, dt, venc, vsl, G, venc);
+  const int ix = c->p.izipx, iv = c->p.izipv;
+  if (ix == 1 && iv == 1) st = kicks_impl<1, 1>(c, G, venc, vsl);
+  else if (ix == 1) st = kicks_impl<1, 2>(c, G, venc, vsl);
+  else if (iv == 1) st = kicks_impl<2, 1>(c, G, venc, vsl);
+  else st = kicks_impl<2, 2>(c, G, venc, vsl);
   if (st) return st;
   if ((st = cube_slots_fold(c, vsl, 3, 0, vmb, nullptr))) return st;
   unsigned long long h[3];

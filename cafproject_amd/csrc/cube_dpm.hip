@@ -67,12 +67,6 @@ template <int NC> __device__ __forceinline__ Pair<NC> ld_pair(const float *row, 
   return r;
 }
 
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 /* the particle lattice: ng^3 points r mesh cells apart, in nb^3 blocks of 4^3 */
 struct Lat {
   int ng, r, nb, nblk;

@@ -170,6 +170,12 @@ template <int B> struct IntOf;
 template <> struct IntOf<1> { typedef int8_t T; };
 template <> struct IntOf<2> { typedef int16_t T; };
 
+/* LDS writes of a wave's lanes before it, reads after it */
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 /* inclusive prefix sum over the 64 lanes of a wave (shuffles, no LDS) */
 __device__ __forceinline__ int wave_incl_scan(int v) {
   const int lane = threadIdx.x & 63;

@@ -156,11 +156,6 @@ template <int IX> struct CdLds { /* per wave */
   int rb[12];     /* first batch of each row of the phase */
   int cax[3][6];  /* a source cell's id is the sum of its three axes' parts */
 };
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 /* bits [0, p), p clipped to [0, 64] */
 __device__ __forceinline__ uint64_t bits_below(int p) {
   p = max(p, 0);

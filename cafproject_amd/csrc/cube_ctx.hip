@@ -26,17 +26,15 @@ extern "C" const char *cube_strerror(int code) {
   return "unknown error";
 }
 
-__global__ void k_slots_zero(unsigned long long *s, int n) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) s[i] = 0ull;
-}
-__global__ __launch_bounds__(CUBE_SLOTS) void k_slots_fold(const unsigned long long *s, int add,
+__global__ __launch_bounds__(CUBE_SLOTS) void k_slots_fold(unsigned long long *s, int add,
                                                           unsigned long long *d64, unsigned *d32) {
   __shared__ unsigned long long r[CUBE_SLOTS];
   const int t = threadIdx.x, reg = blockIdx.x;
   r[t] = s[reg * CUBE_SLOTS + t];
+  s[reg * CUBE_SLOTS + t] = 0ull;
   __syncthreads();
   for (int o = CUBE_SLOTS / 2; o > 0; o >>= 1) {
-    if (t < o) r[t] = add ? r[t] + r[t + o] : (r[t] > r[t + o] ? r[t] : r[t + o]);
+    if (t < o) r[t] = (add >> reg) & 1 ? r[t] + r[t + o] : (r[t] > r[t + o] ? r[t] : r[t + o]);
     __syncthreads();
   }
   if (t == 0) {
@@ -44,12 +42,7 @@ __global__ __launch_bounds__(CUBE_SLOTS) void k_slots_fold(const unsigned long l
     if (d32) d32[reg] = (unsigned)r[0];
   }
 }
-int cube_slots_zero(cube_ctx *c, unsigned long long *region, int nreg) {
-  hipLaunchKernelGGL(k_slots_zero, dim3(1), dim3(256), 0, c->stream, region, nreg * CUBE_SLOTS);
-  CUBE_LAUNCH_CHECK();
-  return CUBE_OK;
-}
-int cube_slots_fold(cube_ctx *c, const unsigned long long *region, int nreg, int add, unsigned long long *d64,
+int cube_slots_fold(cube_ctx *c, unsigned long long *region, int nreg, int add, unsigned long long *d64,
                     unsigned *d32) {
   hipLaunchKernelGGL(k_slots_fold, dim3(nreg), dim3(CUBE_SLOTS), 0, c->stream, region, add, d64, d32);
   CUBE_LAUNCH_CHECK();
@@ -63,9 +56,10 @@ static void free_all(cube_ctx *c) {
                   c->cstart, c->cstart2, c->dest, c->key, c->sortbuf, c->fill, c->xdest, c->xkey, c->rank, c->xrank,
                   c->tanf_tab, c->venc_tab, c->vdec0, c->vdec1, c->rho_f, c->spec_f, c->specd_f, c->force_f,
                   c->kern_f, c->rho_c, c->spec_c, c->specd_c, c->force_c, c->kern_c, c->dred,
-                  c->ured, c->fdsum, c->fdheavy, c->fdlist, c->fdmask, c->ired, c->scanbuf, c->vpart, c->slots, c->ppdefer, c->ppitems};
+                  c->ured, c->fdsum, c->fdheavy, c->fdlist, c->fdmask, c->scanbuf, c->vpart, c->slots, c->ppdefer, c->ppitems};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
+  if (c->hres) (void)hipHostFree(c->hres);
   cube_fft_destroy(c->plan_f);
   cube_fft_destroy(c->plan_c);
   for (int k = 0; k < 2 * CUBE_TEV; ++k)
@@ -234,7 +228,12 @@ extern "C" int cube_ctx_create(const cube_params *p, cube_ctx **out) {
   }
   if (!st && hipMemset(c->ured, 0, 64 * sizeof(uint64_t)) != hipSuccess) st = CUBE_ERR_HIP;
   st |= dalloc(&c->slots, CUBE_NSLOTREG * CUBE_SLOTS);
-  st |= dalloc(&c->ired, c->ntiles * BOX_WG);
+  if (!st && hipMemset(c->slots, 0, CUBE_NSLOTREG * CUBE_SLOTS * sizeof(unsigned long long)) != hipSuccess) st = CUBE_ERR_HIP;
+  if (!st && hipHostMalloc((void **)&c->hres, (HR_BOX + c->ntiles * BOX_WG) * sizeof(unsigned long long),
+                           hipHostMallocMapped) != hipSuccess) {
+    c->hres = nullptr;
+    st = CUBE_ERR_ALLOC;
+  }
   st |= dalloc(&c->scanbuf, c->ncells / 1024 + 4);
   st |= dalloc(&c->vpart, 3 * (c->ncells / 64 + 2));
   if (st) {
@@ -617,20 +616,10 @@ extern "C" int cube_particle_mesh(cube_ctx *c, float a_mid, float dt, float sigm
   st = cube_pm_kicks(c, a_mid, dt, sigma_vi, sigma_vi_new, o.vmax); /* synchronises */
   tend(c, CUBE_T_FINE_KICK);
   if (st) return st;
-  {
-    double sums[2];
-    unsigned f2[2];
-    CUBE_CHECK(hipMemcpyAsync(&sums[0], c->dred + CUBE_DRED_FINE_SUM, sizeof(double), hipMemcpyDeviceToHost,
-                              c->stream));
-    CUBE_CHECK(hipMemcpyAsync(&sums[1], c->dred + CUBE_DRED_COARSE_SUM, sizeof(double), hipMemcpyDeviceToHost,
-                              c->stream));
-    CUBE_CHECK(hipMemcpyAsync(f2, c->ured, 2 * sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
-    CUBE_CHECK(hipStreamSynchronize(c->stream));
-    o.testrhof = sums[0];
-    o.testrhoc = sums[1];
-    memcpy(&o.f2_max_fine, &f2[0], sizeof(float));
-    memcpy(&o.f2_max_coarse, &f2[1], sizeof(float));
-  }
+  memcpy(&o.testrhof, &c->hres[HR_SUM], sizeof(double));
+  memcpy(&o.testrhoc, &c->hres[HR_SUM + 1], sizeof(double));
+  memcpy(&o.f2_max_fine, &c->hres[HR_F2], sizeof(float));
+  memcpy(&o.f2_max_coarse, reinterpret_cast<const char *>(&c->hres[HR_F2]) + sizeof(float), sizeof(float));
   /* W/pm.f90:395-398 in real(4) */
   const float GG = 1.0f / 6.0f / CUBE_PI_F;
   o.dt_fine = sqrtf(1.0f / (sqrtf(o.f2_max_fine) * a_mid * GG));

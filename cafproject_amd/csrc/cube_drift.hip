@@ -29,7 +29,6 @@
 #include <stdlib.h>
 #include <string.h>
 #include <algorithm>
-#include <vector>
 
 #define DT 256
 static const double WEIGHT_V = (double)0.1f; /* real(8),parameter :: weight_v=0.1 */
@@ -37,18 +36,9 @@ static const double WEIGHT_V = (double)0.1f; /* real(8),parameter :: weight_v=0.
 enum { DERR_RANGE = 1, DERR_KEY = 2, DERR_XOVER = 8 };
 
 /* ---------------- small utilities ---------------- */
-__global__ void k_fill_i32(int32_t *p, int64_t n, int32_t v) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = v;
-}
 __global__ void k_fill_i64(int64_t *p, int64_t n, int64_t v) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     p[i] = v;
-}
-static int fill_i32(cube_ctx *c, int32_t *p, int64_t n, int32_t v) {
-  hipLaunchKernelGGL(k_fill_i32, dim3(1024), dim3(256), 0, c->stream, p, n, v);
-  CUBE_LAUNCH_CHECK();
-  return CUBE_OK;
 }
 static int fill_i64(cube_ctx *c, int64_t *p, int64_t n, int64_t v) {
   hipLaunchKernelGGL(k_fill_i64, dim3(64), dim3(256), 0, c->stream, p, n, v);
@@ -58,24 +48,38 @@ static int fill_i64(cube_ctx *c, int64_t *p, int64_t n, int64_t v) {
 
 /* decoded residual velocity table: vdec[code+nvbin/2] =
    tan(pi*real(code)/real(nvbin-1)) / (sqrt(pi/2)/(sigma*vrel_boost)) */
-__global__ void k_vdec(const float *tanf_tab, double *vdec, int nv, double vc) {
+__global__ void k_vdec(const float *tanf_tab, double *vdec, int nv, double vc, unsigned long long *zero, int nz) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < nv) vdec[i] = (double)tanf_tab[i] / vc;
+  if (i < nz) zero[i] = 0ull;
 }
-int cube_vdec_table(cube_ctx *c, double *dst, float sigma) {
+/* the table, and nz words cleared in the same launch */
+int cube_vdec_table(cube_ctx *c, double *dst, float sigma, unsigned long long *zero, int nz) {
   const int nv = c->nvbin;
   hipLaunchKernelGGL(k_vdec, dim3((nv + 255) / 256), dim3(256), 0, c->stream, c->tanf_tab, dst, nv,
-                     cube_vconst(sigma));
+                     cube_vconst(sigma), zero, nz);
   CUBE_LAUNCH_CHECK();
   return CUBE_OK;
 }
 
 /* ---------------- exclusive scan of int32 counts -> int64 ---------------- */
 #define SCAN_B 1024
-__global__ __launch_bounds__(SCAN_B) void k_scan_blocks(const int32_t *cnt, int64_t n, int64_t *bsum) {
+/* largest cell whose keys the drift's finalize pass ranks, and that one wave sorts */
+#define FB_LDS_SORT 64
+#define MED_SORT 1024
+__global__ __launch_bounds__(SCAN_B) void k_scan_blocks(const int32_t *cnt, int64_t n, int64_t *bsum,
+                                                        unsigned long long *ctr) {
   __shared__ int64_t s[SCAN_B];
   const int64_t i = blockIdx.x * (int64_t)SCAN_B + threadIdx.x;
-  s[threadIdx.x] = i < n ? cnt[i] : 0;
+  const int v = i < n ? cnt[i] : 0;
+  s[threadIdx.x] = v;
+  if (ctr) { /* cells that will be listed: big in ctr[5], medium in ctr[6] */
+    const uint64_t big = __ballot(v > MED_SORT), med = __ballot(v > FB_LDS_SORT) & ~big;
+    if ((threadIdx.x & 63) == 0) {
+      if (big) atomicAdd(ctr + 5, (unsigned long long)__popcll(big));
+      if (med) atomicAdd(ctr + 6, (unsigned long long)__popcll(med));
+    }
+  }
   __syncthreads();
   for (int o = SCAN_B / 2; o > 0; o >>= 1) {
     if (threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
@@ -83,7 +87,8 @@ __global__ __launch_bounds__(SCAN_B) void k_scan_blocks(const int32_t *cnt, int6
   }
   if (threadIdx.x == 0) bsum[blockIdx.x] = s[0];
 }
-__global__ __launch_bounds__(SCAN_B) void k_scan_partials(int64_t *bsum, int64_t nb, int64_t *total) {
+__global__ __launch_bounds__(SCAN_B) void k_scan_partials(int64_t *bsum, int64_t nb, int64_t *total,
+                                                          const unsigned long long *ctr, unsigned long long *hres) {
   /* exclusive scan of nb block sums, one block, chunked */
   __shared__ int64_t s[SCAN_B];
   __shared__ int64_t carry;
@@ -105,7 +110,11 @@ __global__ __launch_bounds__(SCAN_B) void k_scan_partials(int64_t *bsum, int64_t
     if (threadIdx.x == SCAN_B - 1) carry += s[SCAN_B - 1];
     __syncthreads();
   }
-  if (threadIdx.x == 0) *total = carry;
+  if (threadIdx.x == 0) {
+    *total = carry;
+    hres[HR_TOTAL] = (unsigned long long)carry;
+  }
+  if (ctr && threadIdx.x < 8) hres[HR_CTR + threadIdx.x] = ctr[threadIdx.x];
 }
 __global__ __launch_bounds__(SCAN_B) void k_scan_final(const int32_t *cnt, int64_t n, const int64_t *boff,
                                                      int64_t *start, const int64_t *total) {
@@ -123,20 +132,20 @@ __global__ __launch_bounds__(SCAN_B) void k_scan_final(const int32_t *cnt, int64
   if (i < n) start[i] = boff[blockIdx.x] + s[threadIdx.x] - v;
   if (i == n - 1) start[n] = *total;
 }
-int cube_scan_counts(cube_ctx *c, const int32_t *cnt, int64_t *start, int64_t n, int64_t *total) {
+int cube_scan_counts(cube_ctx *c, const int32_t *cnt, int64_t *start, int64_t n, int64_t *total,
+                     unsigned long long *ctr) {
   const int64_t nb = (n + SCAN_B - 1) / SCAN_B;
   int64_t *bsum = c->scanbuf;   /* nb + 1 entries */
   int64_t *tot = c->scanbuf + nb;
-  hipLaunchKernelGGL(k_scan_blocks, dim3((unsigned)nb), dim3(SCAN_B), 0, c->stream, cnt, n, bsum);
+  hipLaunchKernelGGL(k_scan_blocks, dim3((unsigned)nb), dim3(SCAN_B), 0, c->stream, cnt, n, bsum, ctr);
   CUBE_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_scan_partials, dim3(1), dim3(SCAN_B), 0, c->stream, bsum, nb, tot);
+  hipLaunchKernelGGL(k_scan_partials, dim3(1), dim3(SCAN_B), 0, c->stream, bsum, nb, tot, (const unsigned long long *)ctr,
+                     c->hres);
   CUBE_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_scan_final, dim3((unsigned)nb), dim3(SCAN_B), 0, c->stream, cnt, n, bsum, start, tot);
   CUBE_LAUNCH_CHECK();
-  if (total) {
-    CUBE_CHECK(hipMemcpyAsync(total, tot, sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
-  }
   CUBE_CHECK(hipStreamSynchronize(c->stream));
+  if (total) *total = (int64_t)c->hres[HR_TOTAL];
   return CUBE_OK;
 }
 
@@ -144,7 +153,7 @@ int cube_scan_counts(cube_ctx *c, const int32_t *cnt, int64_t *start, int64_t n,
 /* particles of local cells [1-w, nt+w]^3 of tile t (periodic): a row of the
    box is a run of cells in each tile it crosses, so its sum is a difference of
    their starts.  BOX_WG workgroups share a tile's rows, the host adds their
-   sums.  Latency bound: some 10 us with the copy back for any tile, where
+   sums.  Latency bound: 4 us for small tiles, 9 for 8 of 128^3, where
    reading the cells' counts took 28 us on 8 tiles of 16^3 cells (784 rows of
    28 cells each, w = 6) and 83 us on 8 of 128^3 */
 __global__ __launch_bounds__(256) void k_tile_boxsum(const int64_t *__restrict__ cstart, Geo g, int w,
@@ -172,11 +181,10 @@ __global__ __launch_bounds__(256) void k_tile_boxsum(const int64_t *__restrict__
 }
 int cube_tile_boxsum(cube_ctx *c, int w, int64_t *host_out) {
   hipLaunchKernelGGL(k_tile_boxsum, dim3(BOX_WG, (unsigned)c->ntiles), dim3(256), 0, c->stream, c->cstart, geo_of(c), w,
-                     c->ired);
+                     (int64_t *)c->hres + HR_BOX);
   CUBE_LAUNCH_CHECK();
-  std::vector<int64_t> part(c->ntiles * BOX_WG);
-  CUBE_CHECK(hipMemcpyAsync(part.data(), c->ired, part.size() * sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
   CUBE_CHECK(hipStreamSynchronize(c->stream));
+  const int64_t *part = (const int64_t *)c->hres + HR_BOX;
   for (int64_t t = 0; t < c->ntiles; ++t) {
     host_out[t] = 0;
     for (int b = 0; b < BOX_WG; ++b) host_out[t] += part[t * BOX_WG + b];
@@ -349,14 +357,12 @@ __global__ __launch_bounds__(DT) void k_drift_dest(const typename IntOf<IX>::T *
 }
 
 /* ---------------- per-cell sort ---------------- */
-#define MED_SORT 1024
 #define BIG_SORT 16384
 #define FB_CELLS 64      /* cells per finalize workgroup (the context sizes vpart for it) */
 /* slots staged in LDS at once: 640 (10 per cell against the 8 of an average
    cell) keeps the finalize workgroup at ~22 KB of LDS, 7 per CU; a workgroup
    with more goes through its cells in runs of at most that many */
 #define FB_CH 640
-#define FB_LDS_SORT 64   /* largest cell whose keys are ranked there */
 /* cells above FB_LDS_SORT, for the sorts of their own: big ones (above
    MED_SORT) from the front of the list, counted in counters[3], the others
    from its back, counted in counters[4] */
@@ -846,15 +852,19 @@ __global__ void k_place_keys(const int32_t *dest, const uint64_t *key, int64_t n
 }
 /* the cells that are listed: medium ones with a wave's bitonic sort, big ones
    with a workgroup's, huge ones by merging sorted runs, tmp the merge buffer.
-   Fixed grids that the lists' counts cut short, so the host need not know them */
+   nmed and nbig bound their numbers; the lists' own counts are on the device */
 static int sort_listed(cube_ctx *c, const int32_t *cnt, const int64_t *start, uint64_t *keys, const int32_t *list,
-                       const unsigned long long *ctr, uint64_t *tmp) {
-  hipLaunchKernelGGL(k_sort_med, dim3((unsigned)std::min<int64_t>((c->ncells + 3) / 4, 1280)), dim3(256), 0, c->stream, cnt,
-                     start, list, c->ncells, ctr, keys);
-  CUBE_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_sort_big, dim3((unsigned)std::min<int64_t>(c->ncells, 256)), dim3(1024), BIG_SORT * sizeof(uint64_t),
-                     c->stream, cnt, start, list, ctr, keys, tmp);
-  CUBE_LAUNCH_CHECK();
+                       const unsigned long long *ctr, uint64_t *tmp, int64_t nmed, int64_t nbig) {
+  if (nmed) {
+    hipLaunchKernelGGL(k_sort_med, dim3((unsigned)std::min<int64_t>((nmed + 3) / 4, 1280)), dim3(256), 0, c->stream, cnt,
+                       start, list, c->ncells, ctr, keys);
+    CUBE_LAUNCH_CHECK();
+  }
+  if (nbig) {
+    hipLaunchKernelGGL(k_sort_big, dim3((unsigned)std::min<int64_t>(nbig, 256)), dim3(1024), BIG_SORT * sizeof(uint64_t),
+                       c->stream, cnt, start, list, ctr, keys, tmp);
+    CUBE_LAUNCH_CHECK();
+  }
   return CUBE_OK;
 }
 /* sort every cell's key segment ascending; c->key, dead once the keys are
@@ -866,18 +876,28 @@ extern "C" int cube_sort_small_segments(cube_ctx *c, const int32_t *cnt, const i
   hipLaunchKernelGGL(k_sort_cells, dim3((unsigned)((c->ncells + FB_CELLS - 1) / FB_CELLS)), dim3(256), 0, c->stream, cnt,
                      start, c->ncells, keys, (int32_t *)c->dest, ctr);
   CUBE_LAUNCH_CHECK();
-  return sort_listed(c, cnt, start, keys, (const int32_t *)c->dest, ctr, c->key);
+  return sort_listed(c, cnt, start, keys, (const int32_t *)c->dest, ctr, c->key, c->ncells, c->ncells);
 }
 
 /* ---------------- driver ---------------- */
+/* what the first pass reads: the decode table (as k_vdec), counts and counters cleared */
+__global__ __launch_bounds__(256) void k_drift_prep(const float *__restrict__ tanf_tab, double *__restrict__ vdec, int nv,
+                                                    double vc, int32_t *__restrict__ cnt, int64_t ncells,
+                                                    unsigned long long *__restrict__ ctr) {
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, nthr = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = t; i < nv; i += nthr) vdec[i] = (double)tanf_tab[i] / vc;
+  for (int64_t i = t; i < ncells; i += nthr) cnt[i] = 0;
+  if (t < 8) ctr[t] = 0ull;
+}
 template <int IX, int IV> static int drift_impl(cube_ctx *c, DriftP P, double venc, int64_t *nxtra,
                                                 unsigned long long *hc) {
   typedef typename IntOf<IX>::T TX;
   typedef typename IntOf<IV>::T TV;
   unsigned long long *ctr = (unsigned long long *)c->ured;
   int st;
-  if ((st = fill_i32(c, c->rhoc2, c->ncells, 0))) return st;
-  if ((st = fill_i64(c, (int64_t *)ctr, 8, 0))) return st;
+  hipLaunchKernelGGL(k_drift_prep, dim3(1024), dim3(256), 0, c->stream, c->tanf_tab, c->vdec0, (int)c->nvbin, venc, c->rhoc2,
+                     c->ncells, ctr);
+  CUBE_LAUNCH_CHECK();
   const int64_t nrows = c->ncells / c->nt;
   const size_t dyn = (size_t)(9 * c->nt + P.agg_cap) * sizeof(int);
   hipLaunchKernelGGL((k_drift_dest<IX, IV>), dim3((unsigned)nrows), dim3(DT), dyn, c->stream, (const TX *)c->xp,
@@ -885,8 +905,8 @@ template <int IX, int IV> static int drift_impl(cube_ctx *c, DriftP P, double ve
                      c->xdest, c->xkey, c->xrank, c->xcap, ctr);
   CUBE_LAUNCH_CHECK();
   int64_t total = 0;
-  if ((st = cube_scan_counts(c, c->rhoc2, c->cstart2, c->ncells, &total))) return st;
-  CUBE_CHECK(hipMemcpy(hc, ctr, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost));
+  if ((st = cube_scan_counts(c, c->rhoc2, c->cstart2, c->ncells, &total, ctr))) return st;
+  memcpy(hc, c->hres + HR_CTR, 8 * sizeof(unsigned long long));
   if (hc[2] & (DERR_RANGE | DERR_KEY)) return CUBE_ERR_DISPLACEMENT;
   if (hc[2] & DERR_XOVER) return CUBE_ERR_IMAGE_OVERFLOW;
   if (total > c->cap) return CUBE_ERR_IMAGE_OVERFLOW;
@@ -901,14 +921,14 @@ template <int IX, int IV> static int drift_impl(cube_ctx *c, DriftP P, double ve
     CUBE_LAUNCH_CHECK();
   }
   /* key is dead after placement: the merge buffer */
-  if ((st = sort_listed(c, c->rhoc2, c->cstart2, c->sortbuf, list, ctr, c->key))) return st;
+  if ((st = sort_listed(c, c->rhoc2, c->cstart2, c->sortbuf, list, ctr, c->key, (int64_t)hc[6], (int64_t)hc[5]))) return st;
   const int64_t nfb = (c->ncells + FB_CELLS - 1) / FB_CELLS;
   hipLaunchKernelGGL((k_drift_final2<IX, IV>), dim3((unsigned)nfb), dim3(256), 0, c->stream, (const TX *)c->xp,
                      (const TV *)c->vp, c->p.has_pid ? c->pid : nullptr, c->vfield, c->cstart2, c->sortbuf,
                      c->vdec0, P, venc, (TX *)c->xp2, (TV *)c->vp2, c->pid2, c->vfield2, c->ncells,
                      c->vpart);
   CUBE_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_sum_parts_tree, dim3(1), dim3(1024), 0, c->stream, c->vpart, nfb, c->dred);
+  hipLaunchKernelGGL(k_sum_parts_tree, dim3(1), dim3(1024), 0, c->stream, c->vpart, nfb, (double *)c->hres + HR_S3);
   CUBE_LAUNCH_CHECK();
   CUBE_CHECK(hipStreamSynchronize(c->stream));
   c->nplocal = total;
@@ -937,7 +957,6 @@ int cube_drift(cube_ctx *c, float dt_old, float dt, float vz_max, float sigma_vi
   if (st) return st;
   if (mx > c->np_tile_max) return CUBE_ERR_TILE_OVERFLOW;
   tbeg(c);
-  if ((st = cube_vdec_table(c, c->vdec0, sigma_vi))) return st;
   DriftP P;
   P.g = geo_of(c);
   P.nlayer = nlayer;
@@ -969,7 +988,7 @@ int cube_drift(cube_ctx *c, float dt_old, float dt, float vz_max, float sigma_vi
   /* std of the velocity field, FP64 sums (:171-224), reduced by the
      finalize kernel of the drift */
   double s3[3];
-  CUBE_CHECK(hipMemcpy(s3, c->dred, 3 * sizeof(double), hipMemcpyDeviceToHost));
+  memcpy(s3, c->hres + HR_S3, sizeof(s3));
   const double npg = (double)c->npglobal;
   cube_vstats v;
   memset(&v, 0, sizeof(v));

@@ -93,7 +93,9 @@ struct cube_ctx {
   double *fdheavy;          /* and FDH_W sums of its crowded cells */
   int32_t *fdlist;          /* and its list of blocks with crowded cells (length in ured) */
   uint64_t *fdmask;         /* those cells, by block */
-  int64_t *ired;            /* the tiles' box sums, BOX_WG parts each */
+  /* pinned host words that kernels store a call's scalars into (HR_*), read
+     after the stream is waited for: no copies back */
+  unsigned long long *hres;
   int64_t *scanbuf;         /* ncells/1024 + 2 block sums of the scan */
   double *vpart;            /* 3 per finalize block of the drift (velocity sums) */
   /* host-side persistent state */
@@ -281,9 +283,9 @@ enum { CUBE_SLOT_F2_FINE = 0, CUBE_SLOT_F2_COARSE = 1, CUBE_SLOT_PP = 2 /* f2, c
 __device__ __forceinline__ unsigned long long *cube_slot(unsigned long long *region) {
   return region + blockIdx.x % CUBE_SLOTS;
 }
-int cube_slots_zero(cube_ctx *c, unsigned long long *region, int nreg);
-/* region r folded into d64[r] (or the low 32 bits into d32[r]): max, or sum when add */
-int cube_slots_fold(cube_ctx *c, const unsigned long long *region, int nreg, int add, unsigned long long *d64,
+/* region r folded into d64[r] (or the low 32 bits into d32[r]): max, or sum
+   where bit r of add is set.  It leaves the region cleared for its next use */
+int cube_slots_fold(cube_ctx *c, unsigned long long *region, int nreg, int add, unsigned long long *d64,
                     unsigned *d32);
 
 /* K_d = k_d/k^2 for the mode (mx, my, mz), mx in [0, n/2], of an n^3 mesh,
@@ -300,9 +302,13 @@ __device__ static inline float cube_kfac(int d, int mx, int my, int mz, int n) {
 
 /* launchers (one file each) */
 int cube_drift(cube_ctx *c, float dt_old, float dt, float vz_max, float sigma_vi, cube_vstats *out);
-int cube_vdec_table(cube_ctx *c, double *dst, float sigma);
-int cube_scan_counts(cube_ctx *c, const int32_t *cnt, int64_t *start, int64_t n, int64_t *total);
+int cube_vdec_table(cube_ctx *c, double *dst, float sigma, unsigned long long *zero = nullptr, int nz = 0);
+/* ctr: the drift's counters, stored to hres with the numbers of cells to be listed */
+int cube_scan_counts(cube_ctx *c, const int32_t *cnt, int64_t *start, int64_t n, int64_t *total,
+                     unsigned long long *ctr = nullptr);
 #define BOX_WG 8 /* workgroups per tile */
+enum { HR_TOTAL = 0, HR_CTR = 1 /* 8 */, HR_S3 = 9 /* 3 */, HR_PP = 12 /* 2 */, HR_VMAX = 14 /* 3 */, HR_SUM = 17 /* 2 */,
+       HR_F2 = 19, HR_BOX = 32 /* BOX_WG per tile */ };
 int cube_tile_boxsum(cube_ctx *c, int w, int64_t *host_out);
 
 /* 1 when the line-FFT kernels are built for size n (12..2048, factors 2, 3, 5) */
@@ -333,6 +339,7 @@ int cube_fft_filter3_t(cube_ctx *c, FFTPlan *p, const float *in3, const float *a
 
 int cube_fine_deposit(cube_ctx *c, float mass_p, double *testrhof);
 /* device slots (in dred) of the deposits' mesh sums */
+#define CUBE_URED_PP 24 /* words of ured: the PP pass's deferred blocks and claimed items */
 #define CUBE_URED_FDHEAVY 32 /* words of ured: the fine deposit's listed blocks, and its sum's finished workgroups */
 #define FDH_W 16             /* waves that share a listed block */
 #define FDS_W 64             /* most workgroups of its sum */

@@ -995,13 +995,48 @@ struct F3 {
 /* G = (((F*a_mid)*dt)/6)/pi per mesh value, the factor of every kick term
    (W/pm.f90:341-348); the coarse kick reads G so each coarse cell's value is
    formed once instead of by every particle whose cloud touches it */
-__global__ void k_kick_prescale(const float *__restrict__ F, int64_t n, float a_mid, float dt, float *__restrict__ G) {
+__device__ __forceinline__ void kick_prescale(const float *__restrict__ F, int64_t n, float a_mid, float dt,
+                                              float *__restrict__ G) {
   for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x) {
     const float a = (F[q] * a_mid) * dt;
     bool ok = true;
     const float v = div_6pi(a, ok);
     G[q] = ok ? v : (a / 6.0f) / CUBE_PI_F;
   }
+}
+__global__ void k_kick_prescale(const float *__restrict__ F, int64_t n, float a_mid, float dt, float *__restrict__ G) {
+  kick_prescale(F, n, a_mid, dt, G);
+}
+/* all that the one-pass kicks read besides the state and the fine mesh, in one
+   launch: G and both decode tables */
+__global__ __launch_bounds__(256) void k_kick_prep(const float *__restrict__ F, int64_t n, float a_mid, float dt,
+                                                   float *__restrict__ G, const float *__restrict__ tanf_tab, int nv,
+                                                   double vc0, double vc1, double *__restrict__ vdec0,
+                                                   double *__restrict__ vdec1) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nv; i += gridDim.x * blockDim.x) {
+    vdec0[i] = (double)tanf_tab[i] / vc0; /* as k_vdec */
+    vdec1[i] = (double)tanf_tab[i] / vc1;
+  }
+  kick_prescale(F, n, a_mid, dt, G);
+}
+/* a step's scalars to the host: vmax folded from its slots (left cleared), the
+   mesh sums and max |F|^2 of both meshes */
+__global__ __launch_bounds__(CUBE_SLOTS) void k_pm_result(unsigned long long *__restrict__ vsl, const double *__restrict__ dred,
+                                                          const uint64_t *__restrict__ ured,
+                                                          unsigned long long *__restrict__ hres) {
+  __shared__ unsigned long long r[CUBE_SLOTS];
+  const int t = threadIdx.x, reg = blockIdx.x;
+  r[t] = vsl[reg * CUBE_SLOTS + t];
+  vsl[reg * CUBE_SLOTS + t] = 0ull;
+  __syncthreads();
+  for (int o = CUBE_SLOTS / 2; o > 0; o >>= 1) {
+    if (t < o) r[t] = r[t] > r[t + o] ? r[t] : r[t + o];
+    __syncthreads();
+  }
+  if (t == 0) hres[HR_VMAX + reg] = r[0];
+  if (reg == 0 && t == 1) hres[HR_SUM] = (unsigned long long)__double_as_longlong(dred[CUBE_DRED_FINE_SUM]);
+  if (reg == 0 && t == 2) hres[HR_SUM + 1] = (unsigned long long)__double_as_longlong(dred[CUBE_DRED_COARSE_SUM]);
+  if (reg == 0 && t == 3) hres[HR_F2] = ured[0]; /* two floats */
 }
 
 /* One kick of one particle: vreal[a] += the CIC gather of the mesh over
@@ -1377,13 +1412,11 @@ int cube_fine_kick(cube_ctx *c, float a_mid, float dt, float sigma_vi, float sig
    this a_mid and dt.  Equal to cube_fine_kick then
    cube_coarse_kick(sigma_vi_new) on the plain force bit for bit. */
 int cube_pm_kicks(cube_ctx *c, float a_mid, float dt, float sigma_vi, float sigma_vi_new, float *vmax) {
-  int st = cube_vdec_table(c, c->vdec0, sigma_vi);
-  if (!st) st = cube_vdec_table(c, c->vdec1, sigma_vi_new);
-  if (st) return st;
-  unsigned long long *vmb = (unsigned long long *)c->ured + 8, *vsl = c->slots + CUBE_SLOT_VMAX * CUBE_SLOTS;
-  if ((st = cube_slots_zero(c, vsl, 3))) return st;
+  int st;
+  unsigned long long *vsl = c->slots + CUBE_SLOT_VMAX * CUBE_SLOTS;
   float *G = reinterpret_cast<float *>(c->specd_c);
-  hipLaunchKernelGGL(k_kick_prescale, dim3(2048), dim3(256), 0, c->stream, c->force_c, 3 * c->ncells, a_mid, dt, G);
+  hipLaunchKernelGGL(k_kick_prep, dim3(2048), dim3(256), 0, c->stream, c->force_c, 3 * c->ncells, a_mid, dt, G, c->tanf_tab,
+                     (int)c->nvbin, cube_vconst(sigma_vi), cube_vconst(sigma_vi_new), c->vdec0, c->vdec1);
   CUBE_LAUNCH_CHECK();
   const double venc = cube_vconst(sigma_vi_new);
   const int ix = c->p.izipx, iv = c->p.izipv;
@@ -1392,10 +1425,10 @@ int cube_pm_kicks(cube_ctx *c, float a_mid, float dt, float sigma_vi, float sigm
   else if (iv == 1) st = kicks_impl<2, 1>(c, G, venc, vsl);
   else st = kicks_impl<2, 2>(c, G, venc, vsl);
   if (st) return st;
-  if ((st = cube_slots_fold(c, vsl, 3, 0, vmb, nullptr))) return st;
-  unsigned long long h[3];
-  CUBE_CHECK(hipMemcpyAsync(h, vmb, sizeof(h), hipMemcpyDeviceToHost, c->stream));
+  hipLaunchKernelGGL(k_pm_result, dim3(3), dim3(CUBE_SLOTS), 0, c->stream, vsl, c->dred, c->ured, c->hres);
+  CUBE_LAUNCH_CHECK();
   CUBE_CHECK(hipStreamSynchronize(c->stream));
+  const unsigned long long *h = c->hres + HR_VMAX;
   for (int a = 0; a < 3; ++a) {
     double d;
     memcpy(&d, &h[a], sizeof(d));
@@ -1408,18 +1441,16 @@ int cube_pm_kicks(cube_ctx *c, float a_mid, float dt, float sigma_vi, float sigm
 int cube_coarse_kick(cube_ctx *c, float a_mid, float dt, float sigma_vi, float *vmax) {
   int st = cube_vdec_table(c, c->vdec0, sigma_vi);
   if (st) return st;
-  unsigned long long *vmb = (unsigned long long *)c->ured + 8, *vsl = c->slots + CUBE_SLOT_VMAX * CUBE_SLOTS;
-  if ((st = cube_slots_zero(c, vsl, 3))) return st;
+  unsigned long long *vsl = c->slots + CUBE_SLOT_VMAX * CUBE_SLOTS;
   /* G in the coarse spectra scratch, free once force_c is formed */
   float *G = reinterpret_cast<float *>(c->specd_c);
   hipLaunchKernelGGL(k_kick_prescale, dim3(2048), dim3(256), 0, c->stream, c->force_c, 3 * c->ncells, a_mid, dt, G);
   CUBE_LAUNCH_CHECK();
   st = kick<false>(c, G, a_mid, dt, cube_vconst(sigma_vi), vsl);
   if (st) return st;
-  if ((st = cube_slots_fold(c, vsl, 3, 0, vmb, nullptr))) return st;
-  unsigned long long h[3];
-  CUBE_CHECK(hipMemcpyAsync(h, vmb, sizeof(h), hipMemcpyDeviceToHost, c->stream));
+  if ((st = cube_slots_fold(c, vsl, 3, 0, c->hres + HR_VMAX, nullptr))) return st;
   CUBE_CHECK(hipStreamSynchronize(c->stream));
+  const unsigned long long *h = c->hres + HR_VMAX;
   for (int a = 0; a < 3; ++a) {
     double d;
     memcpy(&d, &h[a], sizeof(d));

@@ -787,10 +787,6 @@ __global__ __launch_bounds__(PPC_T) void k_pp_cell(const typename IntOf<IX>::T *
   pp_reduce<PPC_T>(f2m, ntest, out);
 }
 
-__global__ void k_zero_u64(unsigned long long *p, int n) {
-  if ((int)threadIdx.x < n) p[threadIdx.x] = 0ull;
-}
-
 template <int IX, int IV>
 static int pp_impl(cube_ctx *c, float a_mid, float dt, float sigma_vi, float mass_p, unsigned long long *out) {
   const int pr = (int)c->p.pp_range;
@@ -820,9 +816,7 @@ static int pp_impl(cube_ctx *c, float a_mid, float dt, float sigma_vi, float mas
     if (const char *e = getenv("CUBE_PP_CELL_CAP"); e && *e)
       cap = std::max(1, std::min((ldsmax - 1024 - (2 * nregc + 1) * 4) / 8, atoi(e)));
     const int64_t nb = c->nt / 4, nblk = nb * nb * nb * c->ntiles;
-    unsigned long long *dcount = (unsigned long long *)c->ured + 24, *claim = (unsigned long long *)c->ured + 25;
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c->stream, dcount, 2);
-    CUBE_LAUNCH_CHECK();
+    unsigned long long *dcount = (unsigned long long *)c->ured + CUBE_URED_PP, *claim = dcount + 1; /* cleared by cube_pp */
     hipLaunchKernelGGL((k_pp_blk<IX, IV>), dim3((unsigned)nblk), dim3(PPB_T), (size_t)maxs * 8 + table, c->stream,
                        (const typename IntOf<IX>::T *)c->xp, (typename IntOf<IV>::T *)c->vp, c->rhoc, c->cstart,
                        c->vdec0, c->venc_tab, geo_of(c), c->nvbin / 2, pr, (double)c->p.rsoft, (double)mass_p, (double)a_mid,
@@ -853,21 +847,18 @@ static int pp_impl(cube_ctx *c, float a_mid, float dt, float sigma_vi, float mas
 }
 
 int cube_pp(cube_ctx *c, float a_mid, float dt, float sigma_vi, float mass_p, float *f2_max_pp, int64_t *itest1) {
-  int st = cube_vdec_table(c, c->vdec0, sigma_vi);
+  int st = cube_vdec_table(c, c->vdec0, sigma_vi, (unsigned long long *)c->ured + CUBE_URED_PP, 2);
   if (st) return st;
-  unsigned long long *out = (unsigned long long *)c->ured + 16, *osl = c->slots + CUBE_SLOT_PP * CUBE_SLOTS;
-  if ((st = cube_slots_zero(c, osl, 2))) return st;
+  unsigned long long *osl = c->slots + CUBE_SLOT_PP * CUBE_SLOTS;
   const int x = c->p.izipx, v = c->p.izipv;
   if (x == 1 && v == 1) st = pp_impl<1, 1>(c, a_mid, dt, sigma_vi, mass_p, osl);
   else if (x == 1) st = pp_impl<1, 2>(c, a_mid, dt, sigma_vi, mass_p, osl);
   else if (v == 1) st = pp_impl<2, 1>(c, a_mid, dt, sigma_vi, mass_p, osl);
   else st = pp_impl<2, 2>(c, a_mid, dt, sigma_vi, mass_p, osl);
   if (st) return st;
-  if ((st = cube_slots_fold(c, osl, 1, 0, out, nullptr)) || (st = cube_slots_fold(c, osl + CUBE_SLOTS, 1, 1, out + 1, nullptr)))
-    return st;
-  unsigned long long h[2];
-  CUBE_CHECK(hipMemcpyAsync(h, out, sizeof(h), hipMemcpyDeviceToHost, c->stream));
+  if ((st = cube_slots_fold(c, osl, 2, 2, c->hres + HR_PP, nullptr))) return st; /* max, sum */
   CUBE_CHECK(hipStreamSynchronize(c->stream));
+  const unsigned long long *h = c->hres + HR_PP;
   double f2;
   memcpy(&f2, &h[0], sizeof(f2));
   /* ftemp=max(ftemp,sum(f_tot**2)) with a `save`d real(4) ftemp that is

@@ -453,14 +453,16 @@ __global__ __launch_bounds__(RC<N>::NT) void k_c2c_r(float2 *__restrict__ a, con
   }
 }
 
+#define GREEN_SPLIT 256 /* largest mesh with a line set per workgroup, see green() */
 /* Green's function pass along z, register version of k_green_z; OCT selects
    the blocked octant kernel storage (fine mesh, cube_kernf_index) over the
    full one (coarse mesh).  A workgroup does the lines y and N-y, which read
-   the same kernel block, for two adjacent column blocks. */
-template <int N, bool OCT>
+   the same kernel block, for two adjacent column blocks and components d0..d1;
+   or (SPLIT) one line set, components d0 + blockIdx.z*nd .. +nd. */
+template <int N, bool OCT, bool SPLIT>
 __global__ __launch_bounds__(RC<N>::NT) void k_green_r(const float2 *spec, float2 *outd,
                                                      const float *__restrict__ kern,
-                                                     const float2 *__restrict__ tw, int d0, int d1) {
+                                                     const float2 *__restrict__ tw, int d0, int d1, int nd) {
   using G = RC<N>;
   constexpr int NH = N / 2 + 1, H = N / 2, R1 = G::R1, R2 = G::R2, H1 = H + 1, SP = cube_spec_pitch(N);
   constexpr int64_t stride = (int64_t)N * SP, plane = (int64_t)SP * N * N;
@@ -480,13 +482,14 @@ __global__ __launch_bounds__(RC<N>::NT) void k_green_r(const float2 *spec, float
      spectrum v dies as w is formed from it and the two share registers */
   if constexpr (G::ONE) d1 = d0 + 1;
   const int yp = blockIdx.y;
-  const int ny = (yp == 0 || yp == H) ? 1 : 2;
+  const int ny = SPLIT || yp == 0 || yp == H ? 1 : 2;
+  const int da = SPLIT ? d0 + (int)blockIdx.z * nd : d0, db = SPLIT ? da + nd : d1;
 #pragma unroll 1
-  for (int cb = 0; cb < 2; ++cb) {
+  for (int cb = 0; cb < (SPLIT ? 1 : 2); ++cb) {
 #pragma unroll 1
     for (int iy = 0; iy < ny; ++iy) {
       const int y = iy == 0 ? yp : N - yp;
-      const int kx0 = (2 * blockIdx.x + cb) * G::CB + c;
+      const int kx0 = ((SPLIT ? 1 : 2) * blockIdx.x + cb) * G::CB + c;
       const bool ok = kx0 < NH;
       const int kx = ok ? kx0 : NH - 1;
       const uint32_t lo = (uint32_t)(((int64_t)t * stride + kx) * 8);
@@ -502,7 +505,7 @@ __global__ __launch_bounds__(RC<N>::NT) void k_green_r(const float2 *spec, float
       const int ky = y <= H ? y : N - y;
       const float sy = y <= H ? 1.f : -1.f;
 #pragma unroll 1
-      for (int d = d0; d < d1; ++d) {
+      for (int d = da; d < db; ++d) {
         /* at N=2048 the kernel loads wait for the forward transform, whose
            peak register use they would otherwise add to */
         const int z0 = G::ONE ? opaque_zero_after(v[R2 - 1].x) : opaque_zero();
@@ -625,9 +628,9 @@ __global__ __launch_bounds__(FFT_T) void k_c2c_s(float2 *__restrict__ a, const f
    workgroup reads its lines whole before it writes them (k_green_r
    likewise). */
 template <int N>
-__global__ __launch_bounds__(FFT_T) void k_green_z(const float2 *spec, float2 *outd,
+__global__ __launch_bounds__(FFT_T, 3) void k_green_z(const float2 *spec, float2 *outd,
                                                  const float *__restrict__ kern, int octant,
-                                                 const float2 *__restrict__ tw, int d0, int d1) {
+                                                 const float2 *__restrict__ tw, int d0, int nd) {
   constexpr int B = Cfg<N>::BS, TL = FFT_T / B, NP = lspan(N), NH = N / 2 + 1, H = N / 2, SP = cube_spec_pitch(N);
   constexpr int EPT = (B * N + FFT_T - 1) / FFT_T;
   __shared__ float2 sm[B * NP];
@@ -636,13 +639,19 @@ __global__ __launch_bounds__(FFT_T) void k_green_z(const float2 *spec, float2 *o
   const int64_t stride = (int64_t)N * SP;   /* between z planes */
   const int64_t plane = (int64_t)SP * N * N;
   const float2 *src = spec + (int64_t)y * SP + col0;
-  for (int idx = tid; idx < B * N; idx += FFT_T) {
-    const int l = idx % B, n = idx / B;
-    sm[l * NP + lpad(n)] = (col0 + l < NH) ? src[n * stride + l] : make_float2(0.f, 0.f);
+  float2 keep[EPT];
+#pragma unroll
+  for (int s = 0; s < EPT; ++s) { /* every load in flight before the first LDS store */
+    const int idx = tid + s * FFT_T, l = idx % B, n = idx / B;
+    keep[s] = idx < B * N && col0 + l < NH ? src[n * stride + l] : make_float2(0.f, 0.f);
+  }
+#pragma unroll
+  for (int s = 0; s < EPT; ++s) {
+    const int idx = tid + s * FFT_T;
+    if (idx < B * N) sm[(idx % B) * NP + lpad(idx / B)] = keep[s];
   }
   __syncthreads();
   line_fft<N, -1, TL>(sm + line * NP, tl, tw, N);
-  float2 keep[EPT];
 #pragma unroll
   for (int s = 0; s < EPT; ++s) {
     const int idx = tid + s * FFT_T;
@@ -650,21 +659,22 @@ __global__ __launch_bounds__(FFT_T) void k_green_z(const float2 *spec, float2 *o
   }
   const int ky = y <= H ? y : N - y;
   const float sy = y <= H ? 1.f : -1.f;
-  for (int d = d0; d < d1; ++d) {
+  const int da = d0 + (int)blockIdx.z * nd;
+#pragma unroll 1
+  for (int d = da; d < da + nd; ++d) {
     __syncthreads();
 #pragma unroll
     for (int s = 0; s < EPT; ++s) {
       const int idx = tid + s * FFT_T;
       if (idx < B * N) {
-        const int l = idx % B, n = idx / B, kx = col0 + l;
+        const int l = FFT_T % B == 0 ? tid % B : idx % B, n = idx / B, kx = col0 + l;
         float K = 0.f;
         if (kx < NH) {
           if (octant) {
-            const int kz = n <= H ? n : N - n;
-            const float sz = n <= H ? 1.f : -1.f;
-            K = kern[cube_kernf_index(H + 1, d, kz, ky, kx)];
+            /* kernel elements of a column lie 16 apart in kz */
+            K = kern[cube_kernf_index(H + 1, d, 0, ky, kx) + 16 * (n <= H ? n : N - n)];
             if (d == 1) K *= sy;
-            if (d == 2) K *= sz;
+            if (d == 2 && n > H) K = -K;
           } else {
             K = kern[(((int64_t)d * N + n) * N + y) * NH + kx];
           }
@@ -1261,7 +1271,22 @@ template <int N> struct Launch {
   static int green(cube_ctx *c, FFTPlan *p, const float2 *spec, const float *kern, int oct, float2 *work3,
                    int d0 = 0, int d1 = 3) {
     constexpr int NH = N / 2 + 1;
-    if constexpr (RC<N>::ok) {
+    /* Below 192^3 a line set does one component per workgroup, the forward
+       transform redone, because a workgroup per line set alone would leave CUs
+       without work (64^3: 192 line sets); up to GREEN_SPLIT a workgroup per line
+       set, above it one per four (512^3: 515 us that way, 511 this).  Against
+       four line sets and all components per workgroup: 28 -> 7.6 us on 64^3 (37
+       -> 12 with the full kernel), 108 -> 68 on 128^3, 110 -> 94 on 256^3, 24 ->
+       18.5 on 48^3 (beside other kernels of a step) */
+    const int nd = N < 192 ? 1 : d1 - d0;
+    if constexpr (RC<N>::ok && N <= GREEN_SPLIT) {
+      using G = RC<N>;
+      dim3 g((NH + G::CB - 1) / G::CB, N, (d1 - d0) / nd);
+      if (oct)
+        hipLaunchKernelGGL((k_green_r<N, true, true>), g, dim3(G::NT), 0, c->stream, spec, work3, kern, p->tw, d0, d1, nd);
+      else
+        hipLaunchKernelGGL((k_green_r<N, false, true>), g, dim3(G::NT), 0, c->stream, spec, work3, kern, p->tw, d0, d1, nd);
+    } else if constexpr (RC<N>::ok) {
       /* pairs of column blocks x the line pairs (y, N-y), y = 0..N/2 */
       using G = RC<N>;
       dim3 g(((NH + G::CB - 1) / G::CB + 1) / 2, N / 2 + 1);
@@ -1270,14 +1295,14 @@ template <int N> struct Launch {
         const int e1 = G::ONE ? e + 1 : d1;
         float2 *o = work3 + (e - d0) * plane;
         if (oct)
-          hipLaunchKernelGGL((k_green_r<N, true>), g, dim3(G::NT), 0, c->stream, spec, o, kern, p->tw, e, e1);
+          hipLaunchKernelGGL((k_green_r<N, true, false>), g, dim3(G::NT), 0, c->stream, spec, o, kern, p->tw, e, e1, 0);
         else
-          hipLaunchKernelGGL((k_green_r<N, false>), g, dim3(G::NT), 0, c->stream, spec, o, kern, p->tw, e, e1);
+          hipLaunchKernelGGL((k_green_r<N, false, false>), g, dim3(G::NT), 0, c->stream, spec, o, kern, p->tw, e, e1, 0);
         CUBE_LAUNCH_CHECK();
       }
     } else {
-      dim3 g((NH + Cfg<N>::BS - 1) / Cfg<N>::BS, N);
-      hipLaunchKernelGGL(k_green_z<N>, g, dim3(FFT_T), 0, c->stream, spec, work3, kern, oct, p->tw, d0, d1);
+      dim3 g((NH + Cfg<N>::BS - 1) / Cfg<N>::BS, N, (d1 - d0) / nd);
+      hipLaunchKernelGGL(k_green_z<N>, g, dim3(FFT_T), 0, c->stream, spec, work3, kern, oct, p->tw, d0, nd);
     }
     CUBE_LAUNCH_CHECK();
     return CUBE_OK;

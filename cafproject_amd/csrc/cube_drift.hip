@@ -266,10 +266,13 @@ __global__ __launch_bounds__(DT) void k_drift_dest(const typename IntOf<IX>::T *
     int err = 0;
     const V3f vcell = *reinterpret_cast<const V3f *>(vfield + 3 * (c0 + i)); /* one 12-byte load */
     const float vcf[3] = {vcell.x, vcell.y, vcell.z};
+    int32_t xcode[3], vcode[3];
+    code_split<IX>(code_word<IX>(xp, p), xcode);
+    code_split<IV>(code_word<IV>(vp, p), vcode);
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      const int32_t xc = (int32_t)xp[3 * p + a];
-      const int32_t vc = (int32_t)vp[3 * p + a];
+      const int32_t xc = xcode[a];
+      const int32_t vc = (int32_t)(typename IntOf<IV>::T)vcode[a];
       const double off = ((double)cube_ucode(IX, xc) + 0.5) * P.xres;
       const double vreal = vdec[vc + P.nvh] + (double)vcf[a];
       const double dx = ((double)P.dt_mid * vreal) / 4.0;
@@ -684,8 +687,11 @@ __global__ __launch_bounds__(256) void k_drift_final2(
         }
         const V3f vo = *reinterpret_cast<const V3f *>(vfield_old + 3 * sc); /* one 12-byte load */
         const float vof[3] = {vo.x, vo.y, vo.z};
+        int32_t vcode[3];
+        code_split<IV>(code_word<IV>(vp, p), vcode);
 #pragma unroll
-        for (int a = 0; a < 3; ++a) vr[q][a] = vdec[(int32_t)vp[3 * p + a] + P.nvh] + (double)vof[a];
+        for (int a = 0; a < 3; ++a)
+          vr[q][a] = vdec[(int32_t)(typename IntOf<IV>::T)vcode[a] + P.nvh] + (double)vof[a];
         pix[q] = (uint64_t)p;
       }
       __syncthreads();
@@ -711,12 +717,14 @@ __global__ __launch_bounds__(256) void k_drift_final2(
           /* vp_new=nint(...atan(...*(vreal-vfield_new))...) (:116-117) */
           int32_t code[3];
           cube_encode_v3(IV, venc, vres, code);
+          int32_t xcode[3];
+          code_split<IX>(code_word<IX>(xp, p), xcode);
           double r[3];
 #pragma unroll
           for (int a = 0; a < 3; ++a) {
             /* xp_new=xp+nint(dt_mid*vreal/(x_resolution*ncell)) (:115) */
             const double qx = ((double)P.dt_mid * vr[q][a]) * P.inv_xres4;
-            xp2[3 * s + a] = (typename IntOf<IX>::T)cube_wrap(IX, (int64_t)xp[3 * p + a] + (int64_t)cube_nint(qx));
+            xp2[3 * s + a] = (typename IntOf<IX>::T)cube_wrap(IX, (int64_t)xcode[a] + (int64_t)cube_nint(qx)); /* modulo 2^8izipx */
             vp2[3 * s + a] = (typename IntOf<IV>::T)code[a];
             r[a] = vdec[code[a] + P.nvh];
           }

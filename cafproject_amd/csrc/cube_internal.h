@@ -172,6 +172,25 @@ template <int B> struct IntOf;
 template <> struct IntOf<1> { typedef int8_t T; };
 template <> struct IntOf<2> { typedef int16_t T; };
 
+/* a particle's position or velocity codes, unsigned, with one 4- or 8-byte read
+   of its 3 or 6 bytes, which ends in the array's padding for the last one.
+   Single codes were three reads per particle in every loop of the PP kernels
+   and the drift; with words (and the cell path's 27 cells counted as one run) a
+   32^3-particle run went from 4.34 to 3.97 ms, the compact 256^3 one from 90.5
+   to 88.8, 512^3 from 356 to 351 (to 344 with the drift's, whose finalize pass
+   went from 4.51 to 4.44 ms and first pass from 2.63 to 2.57) */
+template <int B> struct CodeWord { typedef uint64_t T; };
+template <> struct CodeWord<1> { typedef uint32_t T; };
+template <int B>
+__device__ __forceinline__ typename CodeWord<B>::T code_word(const typename IntOf<B>::T *__restrict__ x, int64_t p) {
+  typename CodeWord<B>::T w;
+  __builtin_memcpy(&w, x + 3 * p, sizeof(w));
+  return w;
+}
+template <int B> __device__ __forceinline__ void code_split(typename CodeWord<B>::T w, int32_t code[3]) {
+#pragma unroll
+  for (int a = 0; a < 3; ++a) code[a] = (int32_t)((w >> (8 * B * a)) & (B == 1 ? 0xffu : 0xffffu));
+}
 /* LDS writes of a wave's lanes before it, reads after it */
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

@@ -207,23 +207,6 @@ __global__ __launch_bounds__(PT) void k_pp(const typename IntOf<IX>::T *__restri
  * clustered region -- is left to the cell path below: it goes to the list
  * `dlist` with its number of work items in `ditems`.
  */
-/* a particle's position (or velocity) codes, unsigned, with one 4- or 8-byte
-   read of its 3 or 6 bytes, which ends in the array's padding for the last one.
-   Single codes were three reads per particle in every loop here; with them and
-   the cell path's 27 cells counted one after another, a 32^3-particle run took
-   4.34 ms (now 3.97), the compact 256^3 one 90.5 (88.8), 512^3 356 (351) */
-template <int IX> struct PpWord { typedef uint64_t T; };
-template <> struct PpWord<1> { typedef uint32_t T; };
-template <int IX>
-__device__ __forceinline__ typename PpWord<IX>::T pp_word(const typename IntOf<IX>::T *__restrict__ xp, int64_t p) {
-  typename PpWord<IX>::T w;
-  __builtin_memcpy(&w, xp + 3 * p, sizeof(w));
-  return w;
-}
-template <int IX> __device__ __forceinline__ void pp_codes(typename PpWord<IX>::T w, int32_t code[3]) {
-#pragma unroll
-  for (int a = 0; a < 3; ++a) code[a] = (int32_t)((w >> (8 * IX * a)) & (IX == 1 ? 0xffu : 0xffffu));
-}
 #define PPB_T 256
 #define PP_HEAVY 32 /* default heavy_at of the block kernel: staged cells above it are placed by their wave */
 #define PPC_T 256
@@ -371,7 +354,7 @@ __global__ __launch_bounds__(PPB_T) void k_pp_blk(const typename IntOf<IX>::T *_
         int32_t code[3] = {0, 0, 0};
         int ri = -1;
         if (l >= 0 && l < hnp) {
-          pp_codes<IX>(pp_word<IX>(xp, hp0 + l), code);
+          code_split<IX>(code_word<IX>(xp, hp0 + l), code);
           ri = region_in(hsc, code);
         }
         const int sub = (int)((cube_ucode(IX, code[2]) >> sh) << 4 | (cube_ucode(IX, code[1]) >> sh) << 2 |
@@ -404,7 +387,7 @@ __global__ __launch_bounds__(PPB_T) void k_pp_blk(const typename IntOf<IX>::T *_
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int l = min(max(l0 + d * u, 0), np - 1);
-      pp_codes<IX>(pp_word<IX>(xp, p0 + l), c4[u]);
+      code_split<IX>(code_word<IX>(xp, p0 + l), c4[u]);
     }
   };
   /* count per fine cell: the cell's owner thread (or wave) only, no atomics */
@@ -491,8 +474,8 @@ __global__ __launch_bounds__(PPB_T) void k_pp_blk(const typename IntOf<IX>::T *_
     int gf[3];
     double x1[3];
     int32_t xc[3], vc[3];
-    pp_codes<IX>(pp_word<IX>(xp, p), xc);
-    pp_codes<IV>(pp_word<IV>(vp, p), vc);
+    code_split<IX>(code_word<IX>(xp, p), xc);
+    code_split<IV>(code_word<IV>(vp, p), vc);
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       x1[a] = (double)(pp_fix(IX, loc[a], xc[a]) - X0[a]) * 0x1p-15;
@@ -682,7 +665,7 @@ __global__ __launch_bounds__(PPC_T) void k_pp_cell(const typename IntOf<IX>::T *
 #pragma unroll
       for (int b = 16; b > 0; b >>= 1) q += q + b < 27 && spre[q + b] <= i ? b : 0;
       int32_t cd[3];
-      pp_codes<IX>(pp_word<IX>(xp, sp0[q] + (i - spre[q])), cd);
+      code_split<IX>(code_word<IX>(xp, sp0[q] + (i - spre[q])), cd);
       const int ri = region(q, cd);
       if (ri >= 0) atomicAdd(&cnt[ri], 1);
     }
@@ -721,10 +704,10 @@ __global__ __launch_bounds__(PPC_T) void k_pp_cell(const typename IntOf<IX>::T *
       }
       __syncthreads();
       /* the wave's next 64 particles are read while it places these */
-      typename PpWord<IX>::T next = 0;
+      typename CodeWord<IX>::T next = 0;
       auto read = [&](int q, int base) {
         const int l = snp[q] - 1 - (base + lane);
-        if (l >= 0) next = pp_word<IX>(xp, sp0[q] + l);
+        if (l >= 0) next = code_word<IX>(xp, sp0[q] + l);
       };
       read(wv, 0);
       for (int q = wv; q < 27; q += PPC_T / 64) {
@@ -733,7 +716,7 @@ __global__ __launch_bounds__(PPC_T) void k_pp_cell(const typename IntOf<IX>::T *
         if (np == 0 && q + PPC_T / 64 < 27) read(q + PPC_T / 64, 0);
         for (int base = 0; base < np; base += 64) { /* uniform over the wave */
           const int l = np - 1 - (base + lane);
-          const typename PpWord<IX>::T word = next;
+          const typename CodeWord<IX>::T word = next;
           if (base + 64 < np)
             read(q, base + 64);
           else if (q + PPC_T / 64 < 27)
@@ -741,7 +724,7 @@ __global__ __launch_bounds__(PPC_T) void k_pp_cell(const typename IntOf<IX>::T *
           int ri = -1;
           int32_t cd[3] = {0, 0, 0};
           if (l >= 0) {
-            pp_codes<IX>(word, cd);
+            code_split<IX>(word, cd);
             ri = region(q, cd);
           }
           const unsigned key = (unsigned)(ri + 1);
@@ -777,8 +760,8 @@ __global__ __launch_bounds__(PPC_T) void k_pp_cell(const typename IntOf<IX>::T *
         p = sp0[13] + tgt[tid];
         int gf[3];
         int32_t xc[3], vc[3];
-        pp_codes<IX>(pp_word<IX>(xp, p), xc);
-        pp_codes<IV>(pp_word<IV>(vp, p), vc);
+        code_split<IX>(code_word<IX>(xp, p), xc);
+        code_split<IV>(code_word<IV>(vp, p), vc);
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
           x1[a] = (double)(pp_fix(IX, C[a], xc[a]) - X0[a]) * 0x1p-15;

@@ -177,8 +177,8 @@ template <> struct IntOf<2> { typedef int16_t T; };
    Single codes were three reads per particle in every loop of the PP kernels
    and the drift; with words (and the cell path's 27 cells counted as one run) a
    32^3-particle run went from 4.34 to 3.97 ms, the compact 256^3 one from 90.5
-   to 88.8, 512^3 from 356 to 351 (to 344 with the drift's, whose finalize pass
-   went from 4.51 to 4.44 ms and first pass from 2.63 to 2.57) */
+   to 88.8, 512^3 from 356 to 351; the drift's finalize pass of 512^3 particles
+   went from 4.51 to 4.44 ms and its first pass from 2.63 to 2.57 */
 template <int B> struct CodeWord { typedef uint64_t T; };
 template <> struct CodeWord<1> { typedef uint32_t T; };
 template <int B>

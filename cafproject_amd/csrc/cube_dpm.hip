@@ -283,6 +283,17 @@ __global__ __launch_bounds__(NT) void k_dpm_tile(const float *__restrict__ x, co
       int l[3];
       (void)lat_of(L, blk_pack(L, slot >> 6), slot & 63, l);
       const Cic c = cic_of(ld3(x + 3 * (int64_t)slot), l, L.r, n);
+      float g[3] = {0.f, 0.f, 0.f};
+      /* not finite: the weights (of a displacement that is not) or the
+         cotangent.  Such a particle adds nothing: its terms have no integer */
+      float odd = (c.w[0][1] + c.w[1][1]) + c.w[2][1];
+      if constexpr (NC == 3) {
+        const V3 pb = ld3(pbar + 3 * (int64_t)slot);
+        g[0] = coef * pb.x;
+        g[1] = coef * pb.y;
+        g[2] = coef * pb.z;
+        odd += (0.f * g[0] + 0.f * g[1]) + 0.f * g[2];
+      }
       int rel[3][2];
       bool in[3][2];
 #pragma unroll
@@ -291,14 +302,8 @@ __global__ __launch_bounds__(NT) void k_dpm_tile(const float *__restrict__ x, co
         for (int u = 0; u < 2; ++u) {
           rel[a][u] = c.i[a][u] - t0[a];
           in[a][u] = (unsigned)rel[a][u] < (unsigned)te[a];
+          if (a == 2) in[a][u] = in[a][u] && odd == odd;
         }
-      float g[3] = {0.f, 0.f, 0.f};
-      if constexpr (NC == 3) {
-        const V3 pb = ld3(pbar + 3 * (int64_t)slot);
-        g[0] = coef * pb.x;
-        g[1] = coef * pb.y;
-        g[2] = coef * pb.z;
-      }
 #pragma unroll
       for (int z = 0; z < 2; ++z)
 #pragma unroll

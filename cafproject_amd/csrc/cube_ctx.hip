@@ -46,6 +46,19 @@ int cube_slots_fold(cube_ctx *c, unsigned long long *region, int nreg, int add, 
                     unsigned *d32) {
   hipLaunchKernelGGL(k_slots_fold, dim3(nreg), dim3(CUBE_SLOTS), 0, c->stream, region, add, d64, d32);
   CUBE_LAUNCH_CHECK();
+  cube_words_close(c, cube_slots_bits(c, region, nreg));
+  return CUBE_OK;
+}
+__global__ void k_words_clear(unsigned long long *w, int n) {
+  for (int i = threadIdx.x; i < n; i += blockDim.x) w[i] = 0ull;
+}
+int cube_words_open(cube_ctx *c, unsigned bits, unsigned long long *w, int n) {
+  if (c->unfolded & bits) {
+    CUBE_CHECK(hipDeviceSynchronize()); /* the pass may have run on a side stream */
+    hipLaunchKernelGGL(k_words_clear, dim3(1), dim3(256), 0, c->stream, w, n);
+    CUBE_LAUNCH_CHECK();
+  }
+  c->unfolded |= bits;
   return CUBE_OK;
 }
 

@@ -1493,6 +1493,8 @@ int cube_fft_green_c2r_3d(cube_ctx *c, FFTPlan *p, float2 *spec, const float *ke
   const float pa = prescale ? prescale[0] : 0.f, pdt = prescale ? prescale[1] : 0.f;
   /* max |F|^2 as float bits: per workgroup into the slots, folded into the
      device word f2dev */
+  int sst = cube_slots_open(c, f2slots, 1);
+  if (sst) return sst;
   const int64_t plane = (int64_t)cube_spec_pitch(p->n) * p->n * p->n;
   switch (p->n) {
 #define CASE(N)                                                                   \
@@ -1532,8 +1534,7 @@ int cube_fft_green_c2r_3d(cube_ctx *c, FFTPlan *p, float2 *spec, const float *ke
     default:
       return CUBE_ERR_INVALID;
   }
-  const int sst = cube_slots_fold(c, f2slots, 1, 0, nullptr, f2dev);
-  if (sst) return sst;
+  if ((sst = cube_slots_fold(c, f2slots, 1, 0, nullptr, f2dev))) return sst;
   if (!f2max) return CUBE_OK; /* no readback: stays asynchronous (and capturable) */
   unsigned bits = 0;
   CUBE_CHECK(hipMemcpyAsync(&bits, f2dev, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));

@@ -109,6 +109,7 @@ struct cube_ctx {
   int pm_ahead;
   float pm_mass, pm_amid, pm_dt; /* force_f then holds the kick factors of this a_mid, dt */
   unsigned long long *slots; /* CUBE_NSLOTREG regions of CUBE_SLOTS words, see cube_slots_fold */
+  unsigned unfolded;         /* what a pass has been queued to fill and not to clear, see cube_words_open */
   /* stage timers: event pairs recorded without waiting, resolved when the
      ring is full or the timers are read */
   int profiling;
@@ -302,8 +303,25 @@ enum { CUBE_SLOT_F2_FINE = 0, CUBE_SLOT_F2_COARSE = 1, CUBE_SLOT_PP = 2 /* f2, c
 __device__ __forceinline__ unsigned long long *cube_slot(unsigned long long *region) {
   return region + blockIdx.x % CUBE_SLOTS;
 }
+/* The regions, and the fine deposit's list length, are cleared by the kernel
+   that uses them up, not before they are filled.  A pass therefore opens its
+   words (a bit of `unfolded` each) before its first kernel and closes them once
+   the last one is queued.  Words found open belong to a pass that an error
+   ended in between: whatever it queued is waited for and they are cleared.
+   (Left as they were, maxima would carry over, and the list would grow past
+   its end.) */
+#define CUBE_OPEN_FDLIST (1u << CUBE_NSLOTREG)
+int cube_words_open(cube_ctx *c, unsigned bits, unsigned long long *w, int n);
+static inline void cube_words_close(cube_ctx *c, unsigned bits) { c->unfolded &= ~bits; }
+static inline unsigned cube_slots_bits(const cube_ctx *c, const unsigned long long *region, int nreg) {
+  return ((1u << nreg) - 1u) << ((region - c->slots) / CUBE_SLOTS);
+}
+static inline int cube_slots_open(cube_ctx *c, unsigned long long *region, int nreg) {
+  return cube_words_open(c, cube_slots_bits(c, region, nreg), region, nreg * CUBE_SLOTS);
+}
 /* region r folded into d64[r] (or the low 32 bits into d32[r]): max, or sum
-   where bit r of add is set.  It leaves the region cleared for its next use */
+   where bit r of add is set.  It leaves the region cleared for its next use,
+   and closes it */
 int cube_slots_fold(cube_ctx *c, unsigned long long *region, int nreg, int add, unsigned long long *d64,
                     unsigned *d32);
 

@@ -924,6 +924,8 @@ template <int IX, bool EX> static int fine_dep(cube_ctx *c, float mass, double *
   const int64_t nbt = (c->nt + 3) / 4, nblk = nbt * nbt * nbt * c->ntiles;
   const typename IntOf<IX>::T *xp = (const typename IntOf<IX>::T *)c->xp;
   unsigned long long *hcount = (unsigned long long *)c->ured + CUBE_URED_FDHEAVY;
+  const int st = cube_words_open(c, CUBE_OPEN_FDLIST, hcount, 2);
+  if (st) return st;
   hipLaunchKernelGGL((k_fine_deposit<IX, EX>), dim3((unsigned)std::min<int64_t>(nblk, FD_GRID)), dim3(64), 0, c->stream,
                      xp, c->rhoc, c->cstart, geo_of(c), mass, c->rho_f, c->fdsum, (int)nblk, heavy_at, c->fdlist,
                      c->fdmask, hcount);
@@ -936,6 +938,7 @@ template <int IX, bool EX> static int fine_dep(cube_ctx *c, float mass, double *
   hipLaunchKernelGGL(k_sum_blocks, dim3(nw), dim3(256), 0, c->stream, c->fdsum, c->fdmask, c->fdheavy, (int)nblk, per,
                      c->fdsum + nblk, c->dred + CUBE_DRED_FINE_SUM, hcount);
   CUBE_LAUNCH_CHECK();
+  cube_words_close(c, CUBE_OPEN_FDLIST);
   if (t) {
     CUBE_CHECK(hipMemcpyAsync(t, c->dred + CUBE_DRED_FINE_SUM, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     CUBE_CHECK(hipStreamSynchronize(c->stream));
@@ -1414,6 +1417,7 @@ int cube_fine_kick(cube_ctx *c, float a_mid, float dt, float sigma_vi, float sig
 int cube_pm_kicks(cube_ctx *c, float a_mid, float dt, float sigma_vi, float sigma_vi_new, float *vmax) {
   int st;
   unsigned long long *vsl = c->slots + CUBE_SLOT_VMAX * CUBE_SLOTS;
+  if ((st = cube_slots_open(c, vsl, 3))) return st;
   float *G = reinterpret_cast<float *>(c->specd_c);
   hipLaunchKernelGGL(k_kick_prep, dim3(2048), dim3(256), 0, c->stream, c->force_c, 3 * c->ncells, a_mid, dt, G, c->tanf_tab,
                      (int)c->nvbin, cube_vconst(sigma_vi), cube_vconst(sigma_vi_new), c->vdec0, c->vdec1);
@@ -1427,6 +1431,7 @@ int cube_pm_kicks(cube_ctx *c, float a_mid, float dt, float sigma_vi, float sigm
   if (st) return st;
   hipLaunchKernelGGL(k_pm_result, dim3(3), dim3(CUBE_SLOTS), 0, c->stream, vsl, c->dred, c->ured, c->hres);
   CUBE_LAUNCH_CHECK();
+  cube_words_close(c, cube_slots_bits(c, vsl, 3));
   CUBE_CHECK(hipStreamSynchronize(c->stream));
   const unsigned long long *h = c->hres + HR_VMAX;
   for (int a = 0; a < 3; ++a) {
@@ -1442,6 +1447,7 @@ int cube_coarse_kick(cube_ctx *c, float a_mid, float dt, float sigma_vi, float *
   int st = cube_vdec_table(c, c->vdec0, sigma_vi);
   if (st) return st;
   unsigned long long *vsl = c->slots + CUBE_SLOT_VMAX * CUBE_SLOTS;
+  if ((st = cube_slots_open(c, vsl, 3))) return st;
   /* G in the coarse spectra scratch, free once force_c is formed */
   float *G = reinterpret_cast<float *>(c->specd_c);
   hipLaunchKernelGGL(k_kick_prescale, dim3(2048), dim3(256), 0, c->stream, c->force_c, 3 * c->ncells, a_mid, dt, G);

@@ -870,6 +870,7 @@ int cube_pp(cube_ctx *c, float a_mid, float dt, float sigma_vi, float mass_p, fl
   int st = cube_vdec_table(c, c->vdec0, sigma_vi, (unsigned long long *)c->ured + CUBE_URED_PP, 2);
   if (st) return st;
   unsigned long long *osl = c->slots + CUBE_SLOT_PP * CUBE_SLOTS;
+  if ((st = cube_slots_open(c, osl, 2))) return st;
   const int x = c->p.izipx, v = c->p.izipv;
   if (x == 1 && v == 1) st = pp_impl<1, 1>(c, a_mid, dt, sigma_vi, mass_p, osl);
   else if (x == 1) st = pp_impl<1, 2>(c, a_mid, dt, sigma_vi, mass_p, osl);

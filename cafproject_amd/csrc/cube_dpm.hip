@@ -24,6 +24,7 @@
  * transforms are exact transposes of each other.
  */
 #include "cube_dpm_internal.h"
+#include "cube_dpm_mem.h"
 #include <math.h>
 #include <stdlib.h>
 #include <string.h>
@@ -726,50 +727,61 @@ extern "C" int cube_dpm_create(const cube_dpm_params *p, cube_dpm **out) {
     d->tcap = (int)std::min<double>(d->nblk, std::max(64.0, 24.0 * mean));
   }
   const int64_t np3 = d->npp * 3;
-  /* What the adjoint finds.  checkpoint: the positions of every step, and the
-     force mesh of every step while all of them take no more than an eighth of
-     the free memory (else it is formed again).  No checkpoint: within 24 bytes
-     per mesh point, the positions of every step if they fit, else position
-     and momentum of every `every`-th step, recomputed from there. */
+  /* What the adjoint finds.  checkpoint: the positions of every step, and
+     their force meshes while there is room (dpm_keep_force), else they are
+     formed again.  No checkpoint: the positions of every step if those after
+     the initial ones take at most 24 bytes per mesh point, else position and
+     momentum of every `every`-th step within those 24 bytes (of one step at
+     least), recomputed from there with 36 bytes per slot to work in. */
   d->every = 1;
-  int64_t nx = p->nsteps + 1, nps = 0, nforce = 1;
-  if (p->checkpoint) {
-    size_t fr = 0, tot = 0;
-    const size_t all = (size_t)p->nsteps * 3 * d->nf3 * sizeof(float);
-    if (hipMemGetInfo(&fr, &tot) == hipSuccess && all <= fr / 8) {
-      d->keep_force = 1;
-      nforce = p->nsteps;
-    }
-  } else if (p->nsteps * 12 * d->npp > 24 * d->nf3) {
+  int64_t nx = p->nsteps + 1, nps = 0;
+  if (!p->checkpoint && p->nsteps * 12 * d->npp > 24 * d->nf3) {
     const int64_t k = std::max<int64_t>(1, 24 * d->nf3 / (24 * d->npp));
     d->every = (int)((p->nsteps + k - 1) / k);
     nx = (p->nsteps - 1) / d->every + 1;
     nps = nx;
   }
   const bool own_end = d->every > 1;
-  if (!st) st |= dalloc_f(&d->amp, (int64_t)p->ng * p->ng * (p->ng / 2 + 1));
-  if (!st) st |= dalloc_f(&d->xs, nx * np3);
-  if (!st && nps) st |= dalloc_f(&d->ps, nps * np3);
-  if (!st && own_end) st |= dalloc_f(&d->xend_own, np3);
+  int64_t base = 0; /* bytes of the arrays below */
+  auto get = [&](float **q, int64_t n) {
+    if (!st) st = dalloc_f(q, n);
+    base += n * (int64_t)sizeof(float);
+  };
+  get(&d->amp, (int64_t)p->ng * p->ng * (p->ng / 2 + 1));
+  get(&d->xs, nx * np3);
+  if (nps) get(&d->ps, nps * np3);
+  if (own_end) get(&d->xend_own, np3);
   if (!st) d->xend = own_end ? d->xend_own : d->xs + (int64_t)p->nsteps * np3;
-  if (!st && own_end) st |= dalloc_f(&d->x, np3);
-  if (!st && own_end) st |= dalloc_f(&d->pw, np3);
-  if (!st) st |= dalloc_f(&d->pm, np3);
-  if (!st) st |= dalloc_f(&d->rho, d->nf3);
-  if (!st) st |= dalloc_f(&d->force, nforce * 3 * d->nf3);
-  if (!st) st |= dalloc_f(&d->S, 3 * d->nf3);
-  if (!st) st |= dalloc_f(reinterpret_cast<float **>(&d->gmx), 2 * DPM_GMX);
-  if (!st) st |= dalloc_f(&d->lam, d->nf3);
-  if (!st) st |= dalloc_f((float **)&d->spec_f, 2 * d->sf);
-  if (!st) st |= dalloc_f((float **)&d->work3_f, 6 * d->sf);
-  if (!st) st |= dalloc_f((float **)&d->spec_g, 2 * d->sg);
-  if (!st) st |= dalloc_f((float **)&d->work3_g, 6 * d->sg);
-  if (!st) st |= dalloc_f(&d->psi, 3 * d->ng3);
-  if (!st) st |= dalloc_f(&d->xbar, np3);
-  if (!st) st |= dalloc_f(&d->pbar, np3);
-  if (!st) st |= dalloc_f(reinterpret_cast<float **>(&d->tcnt), 2 * nt3);
-  if (!st) st |= dalloc_f(reinterpret_cast<float **>(&d->tlist), (int64_t)nt3 * d->tcap);
-  if (!st) st |= dalloc_f(reinterpret_cast<float **>(&d->trange), 2 * (int64_t)d->nblk);
+  if (own_end) get(&d->x, np3);
+  if (own_end) get(&d->pw, np3);
+  get(&d->pm, np3);
+  get(&d->rho, d->nf3);
+  get(&d->S, 3 * d->nf3);
+  get(reinterpret_cast<float **>(&d->gmx), 2 * DPM_GMX);
+  get(&d->lam, d->nf3);
+  get((float **)&d->spec_f, 2 * d->sf);
+  get((float **)&d->work3_f, 6 * d->sf);
+  get((float **)&d->spec_g, 2 * d->sg);
+  get((float **)&d->work3_g, 6 * d->sg);
+  get(&d->psi, 3 * d->ng3);
+  get(&d->xbar, np3);
+  get(&d->pbar, np3);
+  get(reinterpret_cast<float **>(&d->tcnt), 2 * nt3);
+  get(reinterpret_cast<float **>(&d->tlist), (int64_t)nt3 * d->tcap);
+  get(reinterpret_cast<float **>(&d->trange), 2 * (int64_t)d->nblk);
+  if (p->checkpoint && p->nsteps == 1) d->keep_force = 1; /* in the one mesh */
+  if (!st && p->checkpoint && p->nsteps > 1) {
+    const int64_t mesh = 3 * d->nf3 * (int64_t)sizeof(float), extra = (p->nsteps - 1) * mesh;
+    size_t fr = 0, tot = 0;
+    if (hipMemGetInfo(&fr, &tot) == hipSuccess && (int64_t)fr > mesh &&
+        dpm_keep_force(fr - mesh, tot, base + mesh, extra, d->nf3, d->np)) {
+      if (dalloc_f(&d->force, p->nsteps * 3 * d->nf3) == CUBE_OK)
+        d->keep_force = 1;
+      else
+        (void)hipGetLastError(); /* no room after all: the one mesh below */
+    }
+  }
+  if (!d->force) get(&d->force, 3 * d->nf3);
   if (!st && hipStreamSynchronize(d->c.stream) != hipSuccess) st = CUBE_ERR_HIP;
   if (st) {
     cube_dpm_destroy(d);

@@ -21,12 +21,15 @@
  * conjugate factor -i k/k^2, the CIC weight-gradient gather (the position
  * derivative of deposit and gather), the transposed drift and kicks, and
  * the transposed IC filter.  With checkpoint=1 the forward keeps the
- * positions of every step (12 bytes per particle per step) and, while those
- * of all steps take at most an eighth of the device's free memory when the
- * box is created, the force meshes (12 bytes per mesh point per step), which
- * the adjoint else forms again.  With checkpoint=0 it keeps within 24 bytes
- * per mesh point: the positions of every step if they fit, else position and
- * momentum of every k-th step, from which the others are recomputed.
+ * positions of every step (12 bytes per particle per step) and, if three
+ * quarters of the device's memory (more where positions are most of a box)
+ * stay free behind them when the box is created, the force meshes (12 bytes
+ * per mesh point per step), which the adjoint else forms again: the same
+ * results, later.  With checkpoint=0 it keeps the positions of every step if
+ * those after the initial ones take at most 24 bytes per mesh point; else
+ * position and momentum of every k-th step within those 24 bytes (of one step
+ * at least), from which the others are recomputed, and 36 bytes per particle to
+ * do so.  A lattice that is no multiple of 4 takes the room of one that is.
  *
  * Array arguments of forward/adjoint are DEVICE pointers on the context's
  * device (e.g. torch tensors' data_ptr()); the amplitude and schedule are
@@ -45,7 +48,7 @@ typedef struct {
   int32_t ng;         /* particles per dimension (lattice), power of two or 2^a 3^b */
   int32_t nf;         /* density / force mesh per dimension, a multiple of ng */
   int32_t nsteps;     /* KDK steps */
-  int32_t checkpoint; /* 1: keep every step; 0: keep what fits 24 bytes per mesh point, recompute the rest */
+  int32_t checkpoint; /* 1: keep every step; 0: what fits 24 bytes per mesh point (see above), the rest recomputed */
   int32_t device;
   int32_t reserved;
 } cube_dpm_params;

@@ -295,7 +295,8 @@ static int power_args(cube_ctx *c, int32_t ng, int32_t nbin, const double *ksum,
   if (!c || !ksum || !psum || !count || ng < 4 || ng > c->nf || c->nf % ng || nbin < 1) return CUBE_ERR_INVALID;
   if (!c->has_state) return CUBE_ERR_STATE;
   if (c->nt > 519) return CUBE_ERR_INVALID; /* k_pw_deposit stages nt+1 row offsets in LDS */
-  /* the FP64 mesh lives in the force spectra */
+  /* room for an FP64 mesh in the force spectra, where ng < nc deposits (meshes
+     refused for it stay refused where the gathering deposit needs none) */
   if ((size_t)ng * ng * ng * sizeof(double) >
       (size_t)c->fine_nspec * cube_spec_pitch((int)c->nf) * c->nf * c->nf * sizeof(float2))
     return CUBE_ERR_INVALID;
@@ -313,8 +314,13 @@ static void power_deposit(cube_ctx *c, int32_t ng) {
   const typename IntOf<IX>::T *xp = (const typename IntOf<IX>::T *)c->xp;
   if (ng >= c->nc) {
     /* 16^3 mesh cells a workgroup, 8^3 (half the particles read are its own)
-       where that would be too few for 256 CUs */
-    const int n16 = (ng + PG_B - 1) / PG_B, lb = n16 * n16 * n16 >= 512 ? 4 : 3, nb = (ng + (1 << lb) - 1) >> lb;
+       where that would be too few for 256 CUs, 4^3 where even these would be 64
+       at most and each would go through its rows of particles one by one: a call
+       on 16^3 of 32^3 particles takes 121 us with 8^3, 98 with 4^3 (103 by the
+       atomics below), on 32^3 of 64^3 123 and 104 (140); on 48^3 of 24^3, 216
+       workgroups of 8^3, 102 and 107 (108) */
+    const int n16 = (ng + PG_B - 1) / PG_B, n8 = (ng + 7) / 8;
+    const int lb = n16 * n16 * n16 >= 512 ? 4 : (n8 * n8 * n8 > 64 ? 3 : 2), nb = (ng + (1 << lb) - 1) >> lb;
     hipLaunchKernelGGL(k_pw_gather<IX>, dim3((unsigned)(nb * nb * nb)), dim3(PG_T), 0, c->stream, xp, c->cstart, geo_of(c),
                        ng, lb, inv_mean, c->rho_f);
     return;

@@ -71,6 +71,13 @@ __device__ __forceinline__ int rl_i(int v, int l) { return __builtin_amdgcn_read
  * and each lane adds its column, two instructions per particle, so a halo of
  * thousands of particles costs its additions and not a walk each.
  *
+ * PACK, for boxes of few particles: a phase of at most CD_PACK particles is
+ * staged with its rows one behind the other, where a batch of its own for each
+ * row of 6 cells was nearly empty.  One particle a cell: 210 instead of 260 us
+ * on 128^3, 290 instead of 470 on one tile of 144^3 with 2-byte codes (where
+ * rounding makes a slot's fields longest); 152 instead of 202 on 128^3 with one
+ * particle in 8 cells.
+ *
  * What bounds it: VALU work (the hit loop above all) at 16 waves per CU (9.4
  * KB of LDS per wave, 4 waves per SIMD by registers), on small meshes the one
  * chain of dependent loads of a wave, and with halos the additions of the
@@ -153,7 +160,7 @@ template <int IX> struct CdLds { /* per wave */
   uint64_t up[CdWord<IX>::NB][3];
   int64_t start[36][3]; /* a row's first particle, and that of its cells iL and iE */
   int pre[36][7]; /* first particle of each cell of a row, counted from the row's first */
-  int rb[12];     /* first batch of each row of the phase */
+  int rb[12];     /* first slot (PACK) or batch of each row of the phase */
   int cax[3][6];  /* a source cell's id is the sum of its three axes' parts */
 };
 /* bits [0, p), p clipped to [0, 64] */
@@ -165,7 +172,9 @@ __device__ __forceinline__ int64_t rl_i64(int64_t v, int l) {
   return (int64_t)(((uint64_t)(uint32_t)rl_i((int)(v >> 32), l) << 32) | (uint64_t)(uint32_t)rl_i((int)(v & 0xffffffff), l));
 }
 
-template <int IX, bool EX, int NW>
+#define CD_PACK 128 /* largest phase whose rows are staged without padding */
+
+template <int IX, bool EX, int NW, bool PACK>
 __global__ __launch_bounds__(64 * NW, 4) void k_coarse_deposit(const typename IntOf<IX>::T *__restrict__ xp,
                                                             const int32_t *__restrict__ rhoc,
                                                             const int64_t *__restrict__ cstart, Geo g, float mass,
@@ -257,8 +266,10 @@ __global__ __launch_bounds__(64 * NW, 4) void k_coarse_deposit(const typename In
       }
       const int nbr = (nrow + 63) >> 6;
       const int bsc = wave_incl_scan(nbr), psc = wave_incl_scan(nrow);
-      if (lane < 12) S.rb[lane] = bsc - nbr;
       const int nbat = rl_i(bsc, 11), npart = rl_i(psc, 11);
+      const bool packed = PACK && npart <= CD_PACK && npart <= heavy_at; /* uniform */
+      const int rb = packed ? psc - nrow : (PACK ? 64 : 1) * (bsc - nbr); /* see CdLds */
+      if (lane < 12) S.rb[lane] = rb;
       /* row tr of the phase, wave-uniform (read from its lane before any
          branch that turns lanes off), and its particle l's codes as stored */
       struct Seg {
@@ -294,34 +305,55 @@ __global__ __launch_bounds__(64 * NW, 4) void k_coarse_deposit(const typename In
         return cd_fields<IX, EX>(raw, c, up);
       };
       wave_lds_sync();
-      if (nbat <= CdWord<IX>::NB && npart <= heavy_at) {
-        auto stage = [&](W raw, int tr, int o) {
-          const int q = rl_i(bsc - nbr, tr) + (o >> 6);
+      if (packed || (nbat <= CdWord<IX>::NB && npart <= heavy_at)) {
+        auto put = [&](W raw, int q, int tr, int l) {
           bool up[3];
-          const W w = fields(raw, tr, o + lane, up);
+          const W w = fields(raw, tr, l, up);
           const uint64_t u0 = __ballot(up[0]), u1 = __ballot(up[1]), u2 = __ballot(up[2]);
           S.word[q * 64 + lane] = w;
           if (lane < 3) S.up[q][lane] = lane == 0 ? u0 : (lane == 1 ? u1 : u2);
         };
-        /* the first batch of every row is on its way before one is used */
-        W raw[12];
-#pragma unroll
-        for (int tr = 0; tr < 12; ++tr) {
-          raw[tr] = 0;
-          const Seg e = seg(tr);
-          if (lane < e.n) raw[tr] = load(e, lane);
-        }
-#pragma unroll
-        for (int tr = 0; tr < 12; ++tr)
-          if (rl_i(nrow, tr) > 0) stage(raw[tr], tr, 0);
-        if (__ballot(nrow > 64)) {
+        if (packed) {
 #pragma unroll 1
+          for (int q = 0; q * 64 < npart; ++q) {
+            const int i = q * 64 + lane;
+            int tr = 0; /* its row */
+#pragma unroll
+            for (int t = 1; t < 12; ++t) tr += rl_i(rb, t) <= i ? 1 : 0;
+            const int l = i - S.rb[tr], r = (s0 + 3 * (tr & 1)) * 6 + (tr >> 1);
+            W raw = 0;
+            if (i < npart) {
+              int64_t d = S.start[r][0];
+              if (!oneseg) {
+                const int eB = iL ? S.pre[r][1] : 0, eC = iE < 6 ? S.pre[r][iE] : npart;
+                if (l >= eB) d = S.start[r][1] - eB;
+                if (l >= eC) d = S.start[r][2] - eC;
+              }
+              raw = cd_load<IX>(xb8 + (d + l) * PB);
+            }
+            put(raw, q, tr, l);
+          }
+        } else {
+          /* the first batch of every row is on its way before one is used */
+          W raw[12];
+#pragma unroll
           for (int tr = 0; tr < 12; ++tr) {
+            raw[tr] = 0;
             const Seg e = seg(tr);
-            for (int o = 64; o < e.n; o += 64) {
-              W w = 0;
-              if (o + lane < e.n) w = load(e, o + lane);
-              stage(w, tr, o);
+            if (lane < e.n) raw[tr] = load(e, lane);
+          }
+#pragma unroll
+          for (int tr = 0; tr < 12; ++tr)
+            if (rl_i(nrow, tr) > 0) put(raw[tr], rl_i(rb, tr) >> (PACK ? 6 : 0), tr, lane);
+          if (__ballot(nrow > 64)) {
+#pragma unroll 1
+            for (int tr = 0; tr < 12; ++tr) {
+              const Seg e = seg(tr);
+              for (int o = 64; o < e.n; o += 64) {
+                W w = 0;
+                if (o + lane < e.n) w = load(e, o + lane);
+                put(w, (rl_i(rb, tr) >> (PACK ? 6 : 0)) + (o >> 6), tr, o + lane);
+              }
             }
           }
         }
@@ -331,11 +363,11 @@ __global__ __launch_bounds__(64 * NW, 4) void k_coarse_deposit(const typename In
 #pragma unroll 1
         for (int j = 0; j < 3; ++j) { /* rows y-1, y, y+1 */
           const int sy = yi + j, r = sz * 6 + sy, tr = 2 * sy + (sz >= 3 ? 1 : 0);
-          const int pA = S.pre[r][xi], pB = S.pre[r][xi + 1], pC = S.pre[r][xi + 2], pD = S.pre[r][xi + 3];
-          const int rb = S.rb[tr];
+          const int rb = S.rb[tr], r0 = PACK ? rb : 0, q0 = PACK ? 0 : rb;
+          const int pA = r0 + S.pre[r][xi], pB = r0 + S.pre[r][xi + 1], pC = r0 + S.pre[r][xi + 2], pD = r0 + S.pre[r][xi + 3];
           const float ys = j == 1 ? 1.f : -1.f, my = cd_mul<IX>(ys), ay = cd_add<IX>(ys);
           for (int bb = pA >> 6; bb * 64 < pD; ++bb) {
-            const int q = rb + bb, o = 64 * bb;
+            const int q = q0 + bb, o = 64 * bb;
             const uint64_t ux = S.up[q][0], uy = S.up[q][1], uz = S.up[q][2];
             const uint64_t fA = bits_below(pA - o), fB = bits_below(pB - o), fC = bits_below(pC - o), fD = bits_below(pD - o);
             uint64_t m = ((fB & ~fA) & ux) | (fC & ~fB) | ((fD & ~fC) & ~ux);
@@ -967,12 +999,14 @@ template <int IX, bool EX> static int coarse_dep(cube_ctx *c, float mass, double
   const int64_t want = small ? nblk : (nblk + 3) / 4;
   const unsigned grid = (unsigned)std::min<int64_t>(want, DEP_BLOCKS);
   const typename IntOf<IX>::T *xp = (const typename IntOf<IX>::T *)c->xp;
-  if (small)
-    hipLaunchKernelGGL((k_coarse_deposit<IX, EX, 1>), dim3(grid), dim3(64), 0, c->stream, xp, c->rhoc, c->cstart,
-                       geo_of(c), mass, c->rho_c, part, (int)nblk, heavy_at);
-  else
-    hipLaunchKernelGGL((k_coarse_deposit<IX, EX, 4>), dim3(grid), dim3(256), 0, c->stream, xp, c->rhoc, c->cstart,
-                       geo_of(c), mass, c->rho_c, part, (int)nblk, heavy_at);
+  /* few particles: the 72 source cells of an average phase fit CD_PACK.  With 8
+     a cell a phase never does, and the other variant's slots need no offset (1
+     to 2 % of the kernel) */
+  const bool pack = 72 * c->nplocal <= CD_PACK * c->ncells;
+  auto kern = small ? (pack ? k_coarse_deposit<IX, EX, 1, true> : k_coarse_deposit<IX, EX, 1, false>)
+                    : (pack ? k_coarse_deposit<IX, EX, 4, true> : k_coarse_deposit<IX, EX, 4, false>);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(small ? 64 : 256), 0, c->stream, xp, c->rhoc, c->cstart, geo_of(c), mass,
+                     c->rho_c, part, (int)nblk, heavy_at);
   CUBE_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_sum_parts1, dim3(1), dim3(64), 0, c->stream, part, (int)grid, c->dred + CUBE_DRED_COARSE_SUM);
   CUBE_LAUNCH_CHECK();

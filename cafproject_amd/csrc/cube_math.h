@@ -128,6 +128,20 @@ CUBE_HD static inline double cube_rcp(double a) {
   return (double)(1.0f / (float)a);
 #endif
 }
+/* P of cube_encode_v3: atan(x) = x*P(x^2) on [0,1] */
+CUBE_HD static inline double cube_atan_poly(double z) {
+  double p = 0.000937563612006803;
+  p = __builtin_fma(p, z, -0.006394792927109298);
+  p = __builtin_fma(p, z, 0.0204678832131648);
+  p = __builtin_fma(p, z, -0.042088155301232);
+  p = __builtin_fma(p, z, 0.06541381456030451);
+  p = __builtin_fma(p, z, -0.08713861532823457);
+  p = __builtin_fma(p, z, 0.11028651356204722);
+  p = __builtin_fma(p, z, -0.1427443216339156);
+  p = __builtin_fma(p, z, 0.19999129800465953);
+  p = __builtin_fma(p, z, -0.3333330208965988);
+  return __builtin_fma(p, z, 0.9999999966724514);
+}
 /*
  * cube_encode_v of three components, the same integers: the code needs
  * y = (nvbin-1)*atan(c*v)/pi only to the nearest integer, so a shorter atan
@@ -149,18 +163,7 @@ CUBE_HD static inline void cube_encode_v3(int bytes, double c, const double v[3]
     const double u = c * (i == 0 ? v0 : (i == 1 ? v1 : v2)), a = __builtin_fabs(u);
     const double r0 = cube_rcp(a), r = __builtin_fma(__builtin_fma(-a, r0, 1.0), r0, r0);
     const double x = a > 1.0 ? r : a, z = x * x;
-    double p = 0.000937563612006803;
-    p = __builtin_fma(p, z, -0.006394792927109298);
-    p = __builtin_fma(p, z, 0.0204678832131648);
-    p = __builtin_fma(p, z, -0.042088155301232);
-    p = __builtin_fma(p, z, 0.06541381456030451);
-    p = __builtin_fma(p, z, -0.08713861532823457);
-    p = __builtin_fma(p, z, 0.11028651356204722);
-    p = __builtin_fma(p, z, -0.1427443216339156);
-    p = __builtin_fma(p, z, 0.19999129800465953);
-    p = __builtin_fma(p, z, -0.3333330208965988);
-    p = __builtin_fma(p, z, 0.9999999966724514);
-    const double t = x * p, y = (a > 1.0 ? 1.5707963267948966 - t : t) * scale, k = __builtin_rint(y);
+    const double t = x * cube_atan_poly(z), y = (a > 1.0 ? 1.5707963267948966 - t : t) * scale, k = __builtin_rint(y);
     if (!(__builtin_fabs(y - k) < 0.5 - 0x1p-17)) far |= 1 << i; /* a NaN too */
     code[i] = (int32_t)(u < 0.0 ? -k : k);
   }

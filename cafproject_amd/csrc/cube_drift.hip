@@ -362,9 +362,10 @@ __global__ __launch_bounds__(DT) void k_drift_dest(const typename IntOf<IX>::T *
 /* ---------------- per-cell sort ---------------- */
 #define BIG_SORT 16384
 #define FB_CELLS 64      /* cells per finalize workgroup (the context sizes vpart for it) */
-/* slots staged in LDS at once: 640 (10 per cell against the 8 of an average
-   cell) keeps the finalize workgroup at ~22 KB of LDS, 7 per CU; a workgroup
-   with more goes through its cells in runs of at most that many */
+/* slots staged in LDS at once: an average workgroup's 512 and a quarter more, so
+   that most go through their cells in one run; one with more takes runs of at
+   most that many.  23.4 KB, 6 finalize workgroups a CU, which does not bind:
+   their 93 registers allow 5 */
 #define FB_CH 640
 /* cells above FB_LDS_SORT, for the sorts of their own: big ones (above
    MED_SORT) from the front of the list, counted in counters[3], the others

@@ -1340,7 +1340,7 @@ template <int N> struct Launch {
     }
     return CUBE_OK;
   }
-  /* The model's z passes.  Below 256^3 a line set does one component per
+  /* The model's z passes.  Below 192^3 a line set does one component per
      workgroup, forward transform redone, because a workgroup per line set
      alone would leave CUs without work (64^3: 192 line sets). */
   template <bool KA> static int pois(cube_ctx *c, FFTPlan *p, const float2 *spec, const float *amp, float2 *work3) {

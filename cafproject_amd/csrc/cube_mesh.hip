@@ -66,7 +66,7 @@ __device__ __forceinline__ int rl_i(int v, int l) { return __builtin_amdgcn_read
  * terms unchanged, so nothing is lost by not visiting it.
  *
  * A phase with more than `heavy_at` particles (a clustered region) or more
- * batches than are staged at once goes through its particles 32 at a time
+ * batches than are staged at once goes through its particles 64 at a time
  * instead: the wave forms the 27 terms of each (zero where it misses) in LDS
  * and each lane adds its column, two instructions per particle, so a halo of
  * thousands of particles costs its additions and not a walk each.
@@ -120,8 +120,8 @@ __device__ __forceinline__ typename CdWord<IX>::T cd_fields(typename CdWord<IX>:
       uint32_t q;
       if constexpr (EX) {
         up[a] = u >= 32768u;
-        q = (2u * u + 1u) ^ (up[a] ? 0x1ffffu : 0u); /* 131071 - 2u - ... : 131072-(2u+1), 17 bits */
-        q += up[a] ? 1u : 0u;
+        q = (2u * u + 1u) ^ (up[a] ? 0x1ffffu : 0u); /* upper: 131071 - (2u+1), */
+        q += up[a] ? 1u : 0u;                        /* so 131072 - (2u+1), 17 bits */
       } else {
         const float tempx = coarse_tempx<2>(c[a], (int32_t)u);
         const int i1 = (int)floorf(tempx) + 1;
@@ -134,13 +134,13 @@ __device__ __forceinline__ typename CdWord<IX>::T cd_fields(typename CdWord<IX>:
     return w;
   }
 }
-/* weight of axis a in units of 1/(2H) times k: s = 1 the own cell's, -1 the
-   neighbour's; (k, s) come folded as (ks, kh), see CdWord */
+/* axis a's field of a staged word, q of CdWord */
 template <int IX> __device__ __forceinline__ float cd_q(typename CdWord<IX>::T w, int a) {
   if constexpr (IX == 1) return (float)((w >> (8 * a)) & 0xff);
   else return (float)(uint32_t)((w >> (21 * a)) & 0x1fffff);
 }
-/* H + s*t as q*cd_mul(s) + cd_add(s): t = 2q+1 (1-byte codes) or q */
+/* a weight in units of 1/(2H), s = 1 the own cell's and -1 the neighbour's: H +
+   s*t as q*cd_mul(s) + cd_add(s), t = 2q+1 (1-byte codes) or q */
 template <int IX> __device__ __forceinline__ float cd_mul(float s) { return IX == 1 ? 2.f * s : s; }
 template <int IX> __device__ __forceinline__ float cd_add(float s) { return IX == 1 ? CdWord<IX>::H + s : CdWord<IX>::H; }
 /* the codes of particle p as stored: one 4- or 8-byte read of its 3 or 6

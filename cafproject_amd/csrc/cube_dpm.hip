@@ -330,7 +330,7 @@ __global__ __launch_bounds__(NT) void k_dpm_tile(const float *__restrict__ x, co
         g[0] = coef * pb.x;
         g[1] = coef * pb.y;
         g[2] = coef * pb.z;
-        odd += (0.f * g[0] + 0.f * g[1]) + 0.f * g[2];
+        odd = fmaf(0.f, g[0], fmaf(0.f, g[1], fmaf(0.f, g[2], odd)));
       }
       int rel[3][2];
       bool in[3][2];
@@ -340,8 +340,8 @@ __global__ __launch_bounds__(NT) void k_dpm_tile(const float *__restrict__ x, co
         for (int u = 0; u < 2; ++u) {
           rel[a][u] = c.i[a][u] - t0[a];
           in[a][u] = (unsigned)rel[a][u] < (unsigned)te[a];
-          if (a == 2) in[a][u] = in[a][u] && odd == odd;
         }
+      if (odd == odd)
 #pragma unroll
       for (int z = 0; z < 2; ++z)
 #pragma unroll

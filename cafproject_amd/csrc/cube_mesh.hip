@@ -503,6 +503,16 @@ __global__ __launch_bounds__(64 * NW, 4) void k_coarse_deposit(const typename In
  * wave up: its lane sits out, and the block goes to a list for
  * k_fine_deposit_heavy with the mask of such cells.
  *
+ * A row takes batches of its own, ten of which hold a phase of the usual 8
+ * particles a cell; slots then need no offsets and no lane's rows straddle
+ * batches.  PACK stages a phase's rows one behind the other instead.  With one
+ * particle a cell the ten batches were nearly empty: 416 -> 322 us on 128^3
+ * cells, 588 -> 470 on one tile of 144^3 with 2-byte codes.  With 27 a phase is
+ * 30 batches, and staged ten at a time each window has work for the lanes of a
+ * few rows only; packed into 24 at once 275 -> 141 us on 32^3, 670 -> 440 on 64^3
+ * (11, 14 and 18 at a time 512, 516 and 569, however many more waves fit), 1.08
+ * -> 0.97 ms with halos.
+ *
  * Bound by VALU issue (some 4,000 instructions a block, half of them the hits)
  * with the 16 KiB of sums leaving 7 waves a CU to hide the rest.  Both kernels
  * and the sum, against a thread per coarse cell walking its 8 cells in global
@@ -511,14 +521,13 @@ __global__ __launch_bounds__(64 * NW, 4) void k_coarse_deposit(const typename In
  * 128^3 at z = 3, 0.117 -> 0.086 ms on 64^3, 0.057 -> 0.045 ms on 16^3, 1.48
  * -> 0.68 ms on the clustered 128^3 at z = 0 with 1-byte codes.
  */
-template <int IX> struct FdLds { /* per wave */
-  static constexpr int NB = 10; /* batches staged at once: a phase's 10 rows of up to 64 */
+template <int IX, int NB> struct FdLds { /* per wave; NB: batches staged at once */
   float acc[64 * 64];                         /* fine cell q of lane t at q*64 + t: conflict free */
   typename CdWord<IX>::T word[NB * 64];
   uint64_t top[NB][3];
   int64_t start[25][2]; /* a row's first particle, and that of its second cell */
   int pre[25][6];
-  int rb[2][10]; /* a row's first batch, by phase parity */
+  int rb[2][10]; /* a row's first batch (PACK: first slot), by phase parity */
   int cax[3][5];
 };
 /* the two planes b, b+1 of an axis and their weights: a particle of code u in
@@ -585,7 +594,7 @@ __device__ __forceinline__ void blk4(int b, const Geo &g, int nbt, int T[3], int
   m0[2] = 4 * (int)(q2 - t * un);
 }
 
-template <int IX, bool EX>
+template <int IX, bool EX, bool PACK, int NB>
 __global__ __launch_bounds__(64) void k_fine_deposit(const typename IntOf<IX>::T *__restrict__ xp,
                                                      const int32_t *__restrict__ rhoc,
                                                      const int64_t *__restrict__ cstart, Geo g, float mass,
@@ -594,8 +603,8 @@ __global__ __launch_bounds__(64) void k_fine_deposit(const typename IntOf<IX>::T
                                                      uint64_t *__restrict__ hmask,
                                                      unsigned long long *__restrict__ hcount) {
   typedef typename CdWord<IX>::T W;
-  constexpr int PB = 3 * IX, sh = IX == 1 ? 6 : 14, NB = FdLds<IX>::NB;
-  __shared__ FdLds<IX> S;
+  constexpr int PB = 3 * IX, sh = IX == 1 ? 6 : 14;
+  __shared__ FdLds<IX, NB> S;
   const int lane = threadIdx.x;
   const char *xb8 = reinterpret_cast<const char *>(xp);
   const int nt = g.nt, nbt = (nt + 3) / 4;
@@ -665,6 +674,7 @@ __global__ __launch_bounds__(64) void k_fine_deposit(const typename IntOf<IX>::T
     struct Phase {
       int nrow, sB, bsc, rb, nb;
       int64_t dA, dB;
+      int p0, n; /* PACK: first plane, particles */
     };
     auto phase = [&](int il) -> Phase {
       const int p0 = (il - kz + 3) % 3; /* planes p0 and p0+3 (if below 5) have this ilayer */
@@ -672,6 +682,15 @@ __global__ __launch_bounds__(64) void k_fine_deposit(const typename IntOf<IX>::T
       const int rt = on ? (p0 + 3 * (lane & 1)) * 5 + (lane >> 1) : 0;
       Phase h;
       h.nrow = on ? S.pre[rt][5] : 0;
+      if constexpr (PACK) {
+        const int psc = wave_incl_scan(h.nrow);
+        h.p0 = p0;
+        h.rb = psc - h.nrow;
+        h.n = rl_i(psc, 9);
+        h.nb = (h.n + 63) >> 6;
+        if (lane < 10) S.rb[il & 1][lane] = h.rb;
+        return h;
+      }
       h.sB = i2 ? S.pre[rt][1] : 0;
       h.dA = S.start[rt][0];
       h.dB = S.start[rt][1] - S.pre[rt][1];
@@ -688,7 +707,27 @@ __global__ __launch_bounds__(64) void k_fine_deposit(const typename IntOf<IX>::T
 #pragma unroll
       for (int q = 0; q < NB; ++q) {
         raw[q] = 0;
-        if (q0 + q < h.nb) {
+        if (PACK && q0 + q < h.nb) {
+          const int i = 64 * (q0 + q) + lane;
+          int tr = 0, first = 0; /* its row and that row's first slot */
+#pragma unroll
+          for (int t = 1; t < 10; ++t) {
+            const int f = rl_i(h.rb, t);
+            if (f <= i) {
+              tr = t;
+              first = f;
+            }
+          }
+          const int l = i - first, r = (h.p0 + 3 * (tr & 1)) * 5 + (tr >> 1);
+          if (i < h.n) {
+            int64_t p = S.start[r][0];
+            if (i2) {
+              const int sB = S.pre[r][1];
+              if (l >= sB) p = S.start[r][1] - sB;
+            }
+            raw[q] = cd_load<IX>(xb8 + (p + l) * PB);
+          }
+        } else if (!PACK && q0 + q < h.nb) {
           const int tr = __popcll(__ballot(lane < 10 && h.bsc <= q0 + q)); /* its row */
           const int l = 64 * (q0 + q - rl_i(h.rb, tr)) + lane, n = rl_i(h.nrow, tr);
           int64_t p = rl_i64(h.dA, tr);
@@ -731,8 +770,9 @@ __global__ __launch_bounds__(64) void k_fine_deposit(const typename IntOf<IX>::T
       if (pl >= 0 && live) {
 #pragma unroll 1
         for (int j = 0; j < 2; ++j) { /* rows y-1, y */
-          const int r = pl * 5 + yi + j, rb = S.rb[ci & 1][2 * (yi + j) + (pl >= 3 ? 1 : 0)] - c0;
-          const int pA = S.pre[r][xi], pB = S.pre[r][xi + 1], pC = S.pre[r][xi + 2];
+          const int r = pl * 5 + yi + j, r0 = S.rb[ci & 1][2 * (yi + j) + (pl >= 3 ? 1 : 0)];
+          const int rb = (PACK ? 0 : r0) - c0, s0 = PACK ? r0 : 0; /* slots, counted from batch -rb's */
+          const int pA = s0 + S.pre[r][xi], pB = s0 + S.pre[r][xi + 1], pC = s0 + S.pre[r][xi + 2];
           for (int bb = max(pA >> 6, -rb); bb * 64 < pC && rb + bb < NB; ++bb) {
             const int q = rb + bb, o = 64 * bb;
             const uint64_t fB = bits_below(pB - o);
@@ -958,9 +998,13 @@ template <int IX, bool EX> static int fine_dep(cube_ctx *c, float mass, double *
   unsigned long long *hcount = (unsigned long long *)c->ured + CUBE_URED_FDHEAVY;
   const int st = cube_words_open(c, CUBE_OPEN_FDLIST, hcount, 2);
   if (st) return st;
-  hipLaunchKernelGGL((k_fine_deposit<IX, EX>), dim3((unsigned)std::min<int64_t>(nblk, FD_GRID)), dim3(64), 0, c->stream,
-                     xp, c->rhoc, c->cstart, geo_of(c), mass, c->rho_f, c->fdsum, (int)nblk, heavy_at, c->fdlist,
-                     c->fdmask, hcount);
+  /* by the mean density: a phase's 50 source cells in two batches, its rows of 5
+     in one each, or more than that (see k_fine_deposit) */
+  auto kern = 50 * c->nplocal <= 128 * c->ncells  ? k_fine_deposit<IX, EX, true, 4>
+              : 5 * c->nplocal <= 64 * c->ncells ? k_fine_deposit<IX, EX, false, 10>
+                                                 : k_fine_deposit<IX, EX, true, 24>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)std::min<int64_t>(nblk, FD_GRID)), dim3(64), 0, c->stream, xp, c->rhoc, c->cstart,
+                     geo_of(c), mass, c->rho_f, c->fdsum, (int)nblk, heavy_at, c->fdlist, c->fdmask, hcount);
   CUBE_LAUNCH_CHECK();
   /* a fixed grid, four waves a SIMD: the count stays on the device */
   hipLaunchKernelGGL((k_fine_deposit_heavy<IX, EX>), dim3((unsigned)std::min<int64_t>(nblk * FDH_W, 4096)), dim3(64), 0,

@@ -1124,11 +1124,12 @@ __global__ __launch_bounds__(CUBE_SLOTS) void k_pm_result(unsigned long long *__
    the 8 corners in the order of W/pm.f90:146-153 (fine: force_f with
    ((((F*a_mid)*dt)/6)/pi)*wx*wy*wz per term; coarse: the prescaled G with
    G*wx*wy*wz, W/pm.f90:341-348).  loc: 1-based cell in the tile, tt: tile. */
-template <int IX, bool FINE>
+template <int IX, bool FINE, bool PRE = false>
 __device__ __forceinline__ void kick_particle(const int32_t code[3], const int loc[3], const int tt[3],
                                               const Geo &g, const float *__restrict__ force, float a_mid,
                                               float dt, double vreal[3]) {
-  constexpr bool DIV = FINE;
+  /* PRE: the fine mesh already holds (((F*a_mid)*dt)/6)/pi per value */
+  constexpr bool DIV = FINE && !PRE;
   const int nt = g.nt, nfine = 4 * g.nc, nft = 4 * nt;
   int i1[3];
   float d1[3], d2[3];
@@ -1211,15 +1212,18 @@ template <int THREADS> __device__ __forceinline__ void vmax_reduce(double vm[3],
 /* kicks, one workgroup per cell row (tile, k, j): particles of the row are
    contiguous; each thread finds its cell by binary search in LDS.  The one
    kick of FINE (decode with vdec, encode with venc), for callers that take
-   the stages one by one; a step takes k_kicks. */
+   the stages one by one; or (BOTH) a step's two in one pass, as k_kicks below
+   but gathering from the meshes where they lie: for boxes of few particles, see
+   kicks_impl. */
 #define KICK_ROW 2048 /* particles of a row whose cells the kick tables in LDS (else a binary search) */
-template <int IX, int IV, bool FINE>
+template <int IX, int IV, bool FINE, bool BOTH>
 __global__ __launch_bounds__(KT) void k_kick(const typename IntOf<IX>::T *__restrict__ xp,
                                              typename IntOf<IV>::T *__restrict__ vp,
                                              const int64_t *__restrict__ cstart, const float *__restrict__ vfield,
                                              const float *__restrict__ force, const double *__restrict__ vdec,
                                              Geo g, int nvh, float a_mid, float dt, double venc,
-                                             unsigned long long *__restrict__ vmax_bits) {
+                                             unsigned long long *__restrict__ vmax_bits,
+                                             const float *__restrict__ force2, const double *__restrict__ vdec2) {
   const int nt = g.nt;
   const int64_t row = blockIdx.x;
   const int j = (int)(row % nt), k = (int)((row / nt) % nt), t = (int)(row / ((int64_t)nt * nt));
@@ -1235,7 +1239,7 @@ __global__ __launch_bounds__(KT) void k_kick(const typename IntOf<IX>::T *__rest
       for (int64_t q = cs[i]; q < cs[i + 1]; ++q) lcell[q - cs[0]] = (uint16_t)i;
     __syncthreads();
   }
-  constexpr bool VMAX = !FINE; /* the coarse kick reports vmax */
+  constexpr bool VMAX = !FINE || BOTH; /* the coarse kick reports vmax */
   double vm[3] = {0, 0, 0};
   for (int64_t p = cs[0] + threadIdx.x; p < cs[nt]; p += KT) {
     int lo = 0, hi = nt;
@@ -1256,7 +1260,14 @@ __global__ __launch_bounds__(KT) void k_kick(const typename IntOf<IX>::T *__rest
       code[a] = (int32_t)xp[3 * p + a];
       vreal[a] = vdec[(int32_t)vp[3 * p + a] + nvh];
     }
-    kick_particle<IX, FINE>(code, loc, tt, g, force, a_mid, dt, vreal);
+    kick_particle<IX, FINE, BOTH>(code, loc, tt, g, force, a_mid, dt, vreal);
+    if (BOTH) { /* the code the fine kick would store, decoded again for the coarse kick */
+      int32_t v1[3];
+      cube_encode_v3(IV, venc, vreal, v1);
+#pragma unroll
+      for (int a = 0; a < 3; ++a) vreal[a] = vdec2[v1[a] + nvh];
+      kick_particle<IX, false>(code, loc, tt, g, force2, a_mid, dt, vreal);
+    }
     F3 vc = {0.f, 0.f, 0.f};
     if (VMAX) vc = *reinterpret_cast<const F3 *>(vfield + 3 * (c0 + lo)); /* one 12-byte load */
     const float vcf[3] = {vc.x, vc.y, vc.z};
@@ -1448,6 +1459,17 @@ __global__ __launch_bounds__(KB) void k_kicks(const typename IntOf<IX>::T *__res
   vmax_reduce<KB>(vm, vmax_bits);
 }
 template <int IX, int IV> static int kicks_impl(cube_ctx *c, const float *G, double venc, unsigned long long *vmb) {
+  /* With few particles a block's staged mesh costs more than their gathers: with
+     1, 2, 3, 4, 8 particles a cell k_kicks takes 598, 625, 658, 706, 880 us on
+     128^3 cells and the rows 296, 482, 629, 753, 1149; on 48^3 56, 56, 57, 62, 70
+     and 41, 49, 54, 58, 78; on 32^3 and below the two differ by 3 % */
+  if (2 * c->nplocal <= 5 * c->ncells && c->nc >= 32) {
+    hipLaunchKernelGGL((k_kick<IX, IV, true, true>), dim3((unsigned)(c->ncells / c->nt)), dim3(KT), 0, c->stream,
+                       (const typename IntOf<IX>::T *)c->xp, (typename IntOf<IV>::T *)c->vp, c->cstart, c->vfield, c->force_f,
+                       c->vdec0, geo_of(c), c->nvbin / 2, 0.f, 0.f, venc, vmb, G, c->vdec1);
+    CUBE_LAUNCH_CHECK();
+    return CUBE_OK;
+  }
   const int64_t nt = c->nt, grid = ((nt + 3) / 4) * ((nt + 1) / 2) * ((nt + 1) / 2) * c->ntiles;
   auto kern = IX == 1 || nt <= 128 ? k_kicks<IX, IV, true> : k_kicks<IX, IV, IX == 1>; /* as in cube_fine_deposit */
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(KB), 0, c->stream, (const typename IntOf<IX>::T *)c->xp,
@@ -1460,9 +1482,9 @@ template <int IX, int IV> static int kicks_impl(cube_ctx *c, const float *G, dou
 template <int IX, int IV, bool FINE>
 static int kick_impl(cube_ctx *c, const float *force, float a_mid, float dt, double venc, unsigned long long *vmb) {
   const int64_t nrows = c->ncells / c->nt;
-  hipLaunchKernelGGL((k_kick<IX, IV, FINE>), dim3((unsigned)nrows), dim3(KT), 0, c->stream,
+  hipLaunchKernelGGL((k_kick<IX, IV, FINE, false>), dim3((unsigned)nrows), dim3(KT), 0, c->stream,
                      (const typename IntOf<IX>::T *)c->xp, (typename IntOf<IV>::T *)c->vp, c->cstart, c->vfield, force,
-                     c->vdec0, geo_of(c), c->nvbin / 2, a_mid, dt, venc, vmb);
+                     c->vdec0, geo_of(c), c->nvbin / 2, a_mid, dt, venc, vmb, (const float *)nullptr, (const double *)nullptr);
   CUBE_LAUNCH_CHECK();
   return CUBE_OK;
 }
